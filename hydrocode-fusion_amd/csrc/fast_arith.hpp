@@ -1,0 +1,162 @@
+// fast_arith.hpp -- IEEE division and square root in FP64 without the range
+// scaling, for operands known to be in range.
+//
+// What hipcc emits for a / b and sqrt(x) first scales the operands
+// (v_div_scale, v_ldexp with its compares) and fixes the result up at the end,
+// so that denormals, overflow and infinities come out right: 11 and 18
+// instructions besides the seed.  Where the caller knows that the operands are
+// far from the ends of the exponent range the same refinement without them
+// gives the same double: the scaling is by powers of two, and the last step
+// rounds the exact remainder's correction (Markstein).  A quotient is then 3
+// operations once the divisor's reciprocal is known, and several quotients by
+// one divisor share it (Rcp); a fresh reciprocal is the seed and 4 operations,
+// a square root the seed and 9, its reciprocal 3 more.
+//
+// In range means: divisors and radicands in [2^-700, 2^700], numerators zero
+// or in [2^-900, 2^900], quotients in [2^-900, 2^900].  The quotient of a zero
+// has the sign of IEEE division for a positive divisor.
+#pragma once
+#include <math.h>
+
+#include "fastpow.hpp"
+
+namespace hgrp {
+
+HGRP_HD double rcp_seed(double b)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_rcp(b);        // about 2^-24 relative
+#else
+    return 1.0 / b;
+#endif
+}
+HGRP_HD double rsq_seed(double x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_rsq(x);
+#else
+    return 1.0 / sqrt(x);
+#endif
+}
+
+// A divisor b with y = 1/b.  Two Newton steps leave y within 2^-95 of 1/b
+// before its rounding, so it is the rounded reciprocal but for one b in 2^40.
+struct Rcp {
+    double b, y;
+};
+HGRP_HD Rcp rcp_of(double b)
+{
+    double y = rcp_seed(b);
+    y = fma(y, fma(-b, y, 1.0), y);
+    y = fma(y, fma(-b, y, 1.0), y);
+    return {b, y};
+}
+
+// a / r.b
+HGRP_HD double div_q(double a, const Rcp &r)
+{
+    const double q = a * r.y;
+    return fma(-fma(q, r.b, -a), r.y, q);
+}
+HGRP_HD double div_1(double a, double b) { return div_q(a, rcp_of(b)); }
+
+// sqrt(x); *half_inv receives 1/(2 sqrt(x)) to about 2^-47
+HGRP_HD double sqrt_h(double x, double *half_inv)
+{
+    const double y = rsq_seed(x);
+    double s = x * y, h = 0.5 * y;
+    const double r = fma(-h, s, 0.5);
+    h = fma(h, r, h);
+    s = fma(s, r, s);
+    s = fma(fma(-s, s, x), h, s);
+    s = fma(fma(-s, s, x), h, s);
+    *half_inv = h;
+    return s;
+}
+HGRP_HD double sqrt_q(double x)
+{
+    double h;
+    return sqrt_h(x, &h);
+}
+// sqrt(x) as a divisor: its reciprocal comes from the root's own seed
+HGRP_HD Rcp sqrt_rcp(double x)
+{
+    double h;
+    const double s = sqrt_h(x, &h);
+    const double y = h + h;
+    return {s, fma(y, fma(-s, y, 1.0), y)};
+}
+
+// log_dd and exp_dd (fastpow.hpp) with every operation that changes nothing
+// left out: a sum whose larger term is known takes the 3-operation error term
+// (exact either way), products that are exact go into an FMA, and the result
+// is the same double-double.  The table index is masked, so that a base out of
+// range reads inside the table.  The logarithm of 1 is (0, ~1e-19), whose
+// exponential rounds to 1.
+HGRP_HD DD fast_sum(double a, double b)      // |a| >= |b| or a == 0
+{
+    const double s = a + b;
+    return {s, b - (s - a)};
+}
+
+HGRP_HD DD log_in_range(double x)            // x positive, normal
+{
+    int k;
+    double m = frexp(x, &k);
+    m *= 2.0;
+    k -= 1;
+    const int j = (int)fma(m, 128.0, -128.0) & 127;
+    const double *lt = powtab::TAB + powtab::LOG_ROW * j;
+    const double invc = lt[0];
+    const double r = fma(m, invc, -1.0);
+    const double q_hi = r * r;
+    const double q_lo = fma(r, r, -q_hi);
+    double t = -1.0 / 10.0;
+    t = fma(t, r, 1.0 / 9.0);
+    t = fma(t, r, -1.0 / 8.0);
+    t = fma(t, r, 1.0 / 7.0);
+    t = fma(t, r, -1.0 / 6.0);
+    t = fma(t, r, 1.0 / 5.0);
+    t = fma(t, r, -1.0 / 4.0);
+    t = fma(t, r, 1.0 / 3.0);
+    const double tail = t * (q_hi * r);
+    const double kd = (double)k;
+    const DD s1 = fast_sum(kd * powtab::LN2_HI, lt[1]);   // k = 0, or |k| ln2 >= log c
+    const DD s2 = two_sum(s1.hi, r);
+    const DD s3 = two_sum(s2.hi, -0.5 * q_hi);
+    const double lo = fma(-0.5, q_lo, s1.lo + s2.lo + s3.lo + kd * powtab::LN2_LO + lt[2]) + tail;
+    const double hi = s3.hi + lo;
+    return {hi, lo - (hi - s3.hi)};
+}
+
+HGRP_HD double exp_in_range(DD p)            // |p.hi| < 700
+{
+    const double kf = rint(p.hi * powtab::INV_LN2N);
+    const int k2 = (int)kf;
+    const DD z = two_sum(fma(-kf, powtab::LN2N_HI, p.hi), p.lo - kf * powtab::LN2N_LO);   // kf LN2N_HI is exact
+    const double z_hi = z.hi, z_lo = z.lo;
+    double t = 1.0 / 5040.0;
+    t = fma(t, z_hi, 1.0 / 720.0);
+    t = fma(t, z_hi, 1.0 / 120.0);
+    t = fma(t, z_hi, 1.0 / 24.0);
+    t = fma(t, z_hi, 1.0 / 6.0);
+    t = fma(t, z_hi, 0.5);
+    const double small = z_lo + z_hi * z_lo + (z_hi * z_hi) * t;
+    const double *et = powtab::TAB + powtab::EXP_BASE + powtab::EXP_ROW * (k2 & 127);
+    const double T_hi = et[0], T_lo = et[1];
+    const double prod_hi = T_hi * z_hi;
+    const double prod_lo = fma(T_hi, z_hi, -prod_hi);
+    const DD s = fast_sum(T_hi, prod_hi);                  // T_hi >= 1 > |prod_hi|
+    const double tail = s.lo + prod_lo + T_hi * small + T_lo + T_lo * (z_hi + small);
+    return ldexp(s.hi + tail, k2 >> 7);
+}
+
+// x^y from L = log(x): pow_with for x in range and |y log x| < 700
+HGRP_HD double pow_in_range(const DD &L, double y)
+{
+    const double p_hi = y * L.hi;
+    const double p_lo = fma(y, L.hi, -p_hi) + y * L.lo;
+    return exp_in_range(fast_sum(p_hi, p_lo));
+}
+
+}  // namespace hgrp

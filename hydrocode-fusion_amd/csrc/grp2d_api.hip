@@ -382,6 +382,7 @@ static void fill_args(hgrp2d *c, SweepArgs &a, int dir, double tau_flux, double 
     a.nu = nu;
     a.gas = make_gas(c->cfg[6]);
     a.eps = c->cfg[4];
+    a.near2 = near_threshold(a.eps);
     a.alpha = c->cfg[41];
     a.tol = c->newton_tol > 0.0 ? c->newton_tol : a.eps;
     a.conv = c->newton_rule == HGRP_NEWTON_CONVERGE;

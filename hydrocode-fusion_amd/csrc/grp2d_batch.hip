@@ -60,7 +60,7 @@ struct BatchSweep {
     int dir, in, sin, limiter3;    // direction; state and slope sets read; minmod3 (a direction's later sweeps)
     int step, slot, prev_slot;     // the step's index, status slot of this sweep, of the one before (-1: none)
     int bc, conv;                  // boundary condition along the sweep, Newton rule
-    double eps, alpha, tol;
+    double eps, alpha, tol, near2;
     const MlpPacked *mlp;
     Gas gas;
 };
@@ -96,7 +96,7 @@ __device__ __forceinline__ SweepArgs batch_args(const BatchSweep &b, int gi)
         a.nu = tau / g.h_y;
     }
     a.hh = 0.5 * a.h;
-    a.eps = b.eps; a.alpha = b.alpha; a.tol = b.tol;
+    a.eps = b.eps; a.alpha = b.alpha; a.tol = b.tol; a.near2 = b.near2;
     a.mlp = b.mlp;
     a.gas = b.gas;
     a.status = g.ring + b.slot;
@@ -151,7 +151,7 @@ __global__ void __launch_bounds__(256, MINW) batch_y_kernel(BatchSweep b)
     if (b.grids[t.x].halted) return;
     const SweepArgs a = batch_args(b, t.x);
     const int wv = (threadIdx.x >> 6) & 3;
-    y_sweep<NM, G>(a, BatchArgs{t.x}, (long)t.y + wv, t.z, stash[wv], mlp_lds[wv]);
+    y_sweep<MINW, NM, G>(a, BatchArgs{t.x}, (long)t.y + wv, t.z, stash[wv], mlp_lds[wv]);
 }
 
 // the one-grid launch variants (sweep2d.hip) X 0..4 and Y 0..4: X 0 = 8 rows
@@ -548,6 +548,7 @@ BatchSweep sweep_args(hgrp2db *c, int g, int slot, int prev_slot, int tiles_dir,
     b.bc = (int)c->cfg[b.dir == 0 ? 17 : 18];
     b.conv = c->newton_rule == HGRP_NEWTON_CONVERGE;
     b.eps = c->cfg[4];
+    b.near2 = near_threshold(b.eps);
     b.alpha = c->cfg[41];
     b.tol = c->newton_tol > 0.0 ? c->newton_tol : b.eps;
     b.mlp = c->use_mlp ? c->mlp : nullptr;

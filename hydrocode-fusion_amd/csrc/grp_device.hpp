@@ -34,7 +34,7 @@ struct Side {
 // expressions the reference writes inline, so every use sees the same double.
 // Passed by value in kernel arguments, they live in scalar registers; the ones
 // that are a single operation on g or zeta are formed where they are used
-// (the same operation, so the same double), which keeps the struct at ten
+// (the same operation, so the same double), which keeps the struct at twelve
 // doubles: the sweeps run short of scalar registers.
 struct Gas {
     double g;                      // gamma
@@ -43,6 +43,7 @@ struct Gas {
     double inv_g, e_cs;            // 1/g, 0.5 (g-1)/g            star density / sound speed
     double e_sonic, e_a, e_b;      // 2g/(g-1), 0.5/zeta, (1+zeta)/zeta
     double g_gm1;                  // g/(g-1)                      energy flux
+    double y_gm1, y_op2z;          // 1/(g-1), 1/(1+2 zeta)        divisions by reciprocal (fast_arith.hpp)
     __host__ __device__ double gm1() const { return g - 1.0; }
     __host__ __device__ double gp1() const { return g + 1.0; }
     __host__ __device__ double opz() const { return 1.0 + z; }          // 1 + zeta
@@ -67,6 +68,8 @@ __host__ __device__ inline Gas make_gas(double g)
     s.e_a = 0.5 / s.z;
     s.e_b = (1.0 + s.z) / s.z;
     s.g_gm1 = g / (g - 1.0);
+    s.y_gm1 = 1.0 / s.gm1();
+    s.y_op2z = 1.0 / s.op2z();
     return s;
 }
 
@@ -103,6 +106,40 @@ __device__ __forceinline__ double div_by(double a, const RecipDiv &d)
     if (__builtin_expect(d.ok && aq >= 0x1p-800 && aq <= 0x1p800, 1)) return q2;
     if (a == 0.0 && d.ok) return q;
     return div_slow(a, d.b);
+}
+
+// Four quotients by one divisor with a single check for the whole wave: div_by
+// for each where every lane's quotients are in range, else all of them by IEEE
+// division, out of line.  One branch instead of eight keeps the limiter short.
+struct Quot4 {
+    double q[4];
+};
+__device__ __attribute__((noinline)) static Quot4 quot4_slow(double a0, double a1, double a2, double a3, double b)
+{
+    return {{a0 / b, a1 / b, a2 / b, a3 / b}};
+}
+template <int N = 4>
+__device__ __forceinline__ void quot4(const double *a, const RecipDiv &d, double *out)
+{
+    bool in = d.ok;
+    double top = 0.0;
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const double q = a[k] * d.y;
+        out[k] = fma(-fma(q, d.b, -a[k]), d.y, q);
+        if (!(d.b > 0.0)) out[k] = a[k] == 0.0 ? q : out[k];     // the sign of a zero
+        in = in && (fabs(q) >= 0x1p-860 || a[k] == 0.0);
+        top = fmax(top, fabs(q));
+    }
+    if (__builtin_expect(!(in && top <= 0x1p800), 0)) {
+#pragma unroll
+        for (int k = 0; k < N; k += 4) {
+            const Quot4 r = quot4_slow(a[k], k + 1 < N ? a[k + 1] : 0.0, k + 2 < N ? a[k + 2] : 0.0,
+                                       k + 3 < N ? a[k + 3] : 0.0, d.b);
+#pragma unroll
+            for (int q = k; q < N && q < k + 4; ++q) out[q] = r.q[q - k];
+        }
+    }
 }
 
 __device__ __forceinline__ double minmod2(double s_L, double s_R)

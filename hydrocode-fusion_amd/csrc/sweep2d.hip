@@ -56,7 +56,7 @@ __global__ void __launch_bounds__(256, MINW) sweep_y_kernel(SweepArgs a, int chu
     __shared__ double stash[4][5][64];   // each wave's cell values and E, read back for the update
     const int wv = (threadIdx.x >> 6) & 3;
     const long wave = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    y_sweep<NM, G>(a, KernargArgs{}, wave, chunks, stash[wv], mlp_lds[wv]);
+    y_sweep<MINW, NM, G>(a, KernargArgs{}, wave, chunks, stash[wv], mlp_lds[wv]);
 }
 
 // min over cells of min(h_x, h_y) / (|c| + |u| + |v|)  (grp_solver_2D_split_EUL_source.c:185-191).

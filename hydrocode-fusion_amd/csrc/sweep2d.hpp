@@ -15,7 +15,7 @@
 #pragma once
 #include <stdint.h>
 
-#include "grp_device.hpp"
+#include "grp_fast.hpp"
 #include "mlp_guess.hpp"
 
 namespace hgrp {
@@ -45,6 +45,7 @@ struct SweepArgs {
                                               // (the launchers pick the kernel's Newton mode from it and mlp)
     double h, hh, tau, nu, eps, alpha;        // h, h/2, flux time, update factor, ...
     double tol;                               // Newton tolerance (the reference: eps)
+    double near2;                             // the acoustic switch dist < eps on dist^2 (near_threshold)
     RecipDiv div_h;                           // division by h
     const MlpPacked *mlp;                     // learned p* guess, or nullptr (the reference's guess)
     Gas gas;                                  // gamma and its derived constants

@@ -91,12 +91,14 @@ struct Line {
     __device__ void limited_sp(const double vm[4], const double v0[4], const double vp[4], const double sp[4],
                                double s[4]) const
     {
+        double d_L[4], d_R[4], s_L[4], s_R[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const double s_L = div_by(v0[q] - vm[q], a.div_h);
-            const double s_R = div_by(vp[q] - v0[q], a.div_h);
-            s[q] = a.limiter3 ? minmod3(a.alpha * s_L, a.alpha * s_R, sp[q]) : minmod2(s_L, s_R);
-        }
+        for (int q = 0; q < 4; ++q) { d_L[q] = v0[q] - vm[q]; d_R[q] = vp[q] - v0[q]; }
+        quot4(d_L, a.div_h, s_L);
+        quot4(d_R, a.div_h, s_R);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            s[q] = a.limiter3 ? minmod3(a.alpha * s_L[q], a.alpha * s_R[q], sp[q]) : minmod2(s_L[q], s_R[q]);
     }
     __device__ void limited(int k, const double vm[4], const double v0[4], const double vp[4], double s[4]) const
     {
@@ -130,6 +132,18 @@ struct Line {
             break;
         }
     }
+    // ghost slopes next to a boundary cell whose own slopes `near` the caller has: the rules of
+    // ghost_slope, which only the periodic one needs other cells for
+    __device__ void ghost_slope_near(bool lo, const double near[4], double s[4]) const
+    {
+        if (a.bc == BC_PERIODIC) {
+            limited_at(lo ? cnt - 1 : 0, s);
+            return;
+        }
+        const bool keep = a.bc == BC_REFLECT || (a.bc == BC_REFLECT_FREE && lo);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s[q] = keep && q == NV ? near[q] : 0.0;
+    }
     // conservative update of cell k and slope refresh (grp_solver_2D_split_EUL_source.c:236-254)
     __device__ void update(int k, const double w[4], const double Fl[4], const double Fr[4],
                            const double Il[4], const double Ir[4]) const
@@ -146,26 +160,65 @@ struct Line {
         const double mom_y = w[0] * w[2] - nu * (Fr[2] - Fl[2]);
         const double ene = w[0] * e - nu * (Fr[3] - Fl[3]);
         const double rho = w[0] + -nu * (Fr[0] - Fl[0]);
-        const double u = mom_x / rho;
-        const double v = mom_y / rho;
+        double u, v, e_new;
+        quot3(mom_x, mom_y, ene, rho, u, v, e_new);
         const double p = (ene - 0.5 * mom_x * u - 0.5 * mom_y * v) * a.gas.gm1();
         double *f = a.st_o + o;
         const size_t P = a.plane;
-        f[0] = rho; f[P] = u; f[2 * P] = v; f[4 * P] = ene / rho; f[3 * P] = p;
+        f[0] = rho; f[P] = u; f[2 * P] = v; f[4 * P] = e_new; f[3 * P] = p;
         if (p < a.eps || rho < a.eps) atomicOr(&a.status->flags, 1u);
+        double dI[4], sn[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) a.s_o[o + q * P] = div_by(Ir[q] - Il[q], a.div_h);
+        for (int q = 0; q < 4; ++q) dI[q] = Ir[q] - Il[q];
+        quot4(dI, a.div_h, sn);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) a.s_o[o + q * P] = sn[q];
     }
 };
 
-template <int DIR, int NM>
-__device__ __forceinline__ void solve_interface(const SweepArgs &a, const Side &SL, const Side &SR,
-                                                unsigned long long loop_index, double F[4], double I[4],
-                                                double p_guess = -1.0)
+// Face f of grid line `line` (between cells f - 1 and f) with the IEEE solver,
+// from the cells in memory: what the fast solver leaves (grp_fast.hpp).  F, I:
+// the flux and the values at t + tau; returns grp_2d_flux's code.  MINW: the
+// calling kernels' register budget (waves per SIMD); a copy of its own for each
+// keeps the compiler from giving the callee a larger one.
+template <int DIR, bool CONV, int MINW>
+__device__ __attribute__((noinline)) int redo_face(const SweepArgs *ap, int line, int f, double p_guess, double *FI)
 {
-    int code = ifvar_bad(SL, SR, a.eps) ? 1 : 0;
-    if (grp_2d_flux<DIR, NM != NM_REF>(SL, SR, a.gas, a.tau, a.eps, F, I, a.tol, p_guess)) code = 2;
-    if (code) atomicMax(&a.status->fail_key, ((loop_index << 2) | (unsigned long long)code) + 1ull);
+    const SweepArgs &a = *ap;
+    const Line<DIR> L(a, line);
+    double wl[4], wr[4], sl[4], sr[4];
+    L.value(f - 1, wl);
+    L.value(f, wr);
+    if (f > 0) L.limited_at(f - 1, sl); else L.ghost_slope(true, sl);
+    if (f < L.cnt) L.limited_at(f, sr); else L.ghost_slope(false, sr);
+    return grp_2d_flux<DIR, CONV>(recon(wl, sl, a.hh, true), recon(wr, sr, a.hh, false), a.gas, a.tau, a.eps, FI,
+                                  FI + 4, a.tol, p_guess);
+}
+
+// GRP flux of face f of grid line `line`, sides SL | SR.  src gives the
+// argument block again (see reload_args).
+template <int DIR, int NM, int MINW, class Src>
+__device__ __forceinline__ void solve_interface(const SweepArgs &a, const Src &src, const Side &SL, const Side &SR,
+                                                int line, int f, double F[4], double I[4], double p_guess = -1.0)
+{
+    int code = ifvar_bad(SL, SR, a.eps) ? 1 : 0, bad = 0;
+    const bool done = flux_split_q<DIR, NM != NM_REF>(SL, SR, a.gas, a.near2, a.tau, a.eps, F, I, a.tol, p_guess, &bad);
+    if (__builtin_expect(__any(!done), 0)) {
+        if (!done) {
+            const SweepArgs ar = src.get();
+            double o[8];
+            bad = redo_face<DIR, NM != NM_REF, MINW>(&ar, line, f, p_guess, o);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) { F[q] = o[q]; I[q] = o[4 + q]; }
+        }
+    }
+    if (bad) code = 2;
+    if (code) {
+        const SweepArgs ar = src.get();
+        const unsigned long long index = (unsigned long long)line * (unsigned long long)((DIR == 0 ? ar.m : ar.n) + 1)
+                                         + (unsigned long long)f;
+        atomicMax(&ar.status->fail_key, ((index << 2) | (unsigned long long)code) + 1ull);
+    }
 }
 
 // Learned starting pressure for the interface (SL | SR) normal to DIR, for
@@ -177,10 +230,9 @@ __device__ __forceinline__ double interface_guess(const SweepArgs &a, bool activ
                                                   uint32_t *lds)
 {
     const double uL = DIR == 0 ? SL.u : SL.v, uR = DIR == 0 ? SR.u : SR.v;
-    const double dist = sqrt((SL.rho - SR.rho) * (SL.rho - SR.rho) + (uL - uR) * (uL - uR)
-                             + (SL.p - SR.p) * (SL.p - SR.p));
+    const double dist2 = (SL.rho - SR.rho) * (SL.rho - SR.rho) + (uL - uR) * (uL - uR) + (SL.p - SR.p) * (SL.p - SR.p);
     // Newton runs only past the acoustic shortcut and the equal-state exit of the exact solver
-    const bool want = active && !(dist < a.eps) && !(fabs(uL - uR) < a.tol && fabs(SL.p - SR.p) < a.tol);
+    const bool want = active && !(dist2 < a.near2) && !(fabs(uL - uR) < a.tol && fabs(SL.p - SR.p) < a.tol);
     return learned_guess_wave(a.mlp, want, SL.rho, uL, SL.p, SR.rho, uR, SR.p, a.gas.g, a.gas.g, lds);
 }
 
@@ -278,24 +330,23 @@ __device__ __forceinline__ bool line_chunk(const SweepArgs &a, const Src &src, i
         for (int q = 0; q < 4; ++q) vr[q] = xa[w + 1][q][lane];
 
     double s[4] = {0.0, 0.0, 0.0, 0.0}, sr[4] = {0.0, 0.0, 0.0, 0.0};
-    if (col) {
-        if (own) L.limited_sp(vl, v, vr, sp, s);
-        else if (c == -1) L.ghost_slope(true, s);
-        else if (c == m) L.ghost_slope(false, s);
-        if (w == W - 1) {
-            if (next_own) {
-                L.limited_sp(v, vr, vrr, sp1, sr);
-            } else if (c + 1 == m) {
-                L.ghost_slope(false, sr);
-            }
-        }
-    }
+    if (own) L.limited_sp(vl, v, vr, sp, s);
+    if (next_own) L.limited_sp(v, vr, vrr, sp1, sr);
 #pragma unroll
     for (int q = 0; q < 4; ++q) xb[w][q][lane] = s[q];
     __syncthreads();
     if (w < W - 1)
 #pragma unroll
         for (int q = 0; q < 4; ++q) sr[q] = xb[w + 1][q][lane];
+    // the ghosts' slopes from the boundary cells' (the lane has them by now)
+    if (col && (c == -1 || c + 1 == m)) {
+        double g[4];
+        L.ghost_slope_near(c == -1, c == -1 ? sr : s, g);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (c == -1) s[q] = g[q]; else sr[q] = g[q];
+        }
+    }
 
     double F[4] = {0.0, 0.0, 0.0, 0.0}, I[4] = {0.0, 0.0, 0.0, 0.0};
     const int f = c + 1;
@@ -311,8 +362,7 @@ __device__ __forceinline__ bool line_chunk(const SweepArgs &a, const Src &src, i
         // none of it is held across the solve
         const Side SL = recon(v, s, hh, true);
         const Side SR = recon(vr, sr, hh, false);
-        solve_interface<DIR, NM>(src.get(), SL, SR,
-                                 (unsigned long long)line * (unsigned long long)(m + 1) + (unsigned long long)f, F, I, pg);
+        solve_interface<DIR, NM, 4>(src.get(), src, SL, SR, line, f, F, I, pg);
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q) { xf[w][q][lane] = F[q]; xi[w][q][lane] = I[q]; }
@@ -388,7 +438,7 @@ __device__ __forceinline__ void line_sweep_chunks(const Src &src, int bx, int by
 // wave: the wave's index in the grid's sweep (a group of 64/G rows, one run
 // of G - 1 cells); st, mlp: this wave's LDS slots; src gives the argument
 // block again after the solve.
-template <int NM, int G, class Src>
+template <int MINW, int NM, int G, class Src>
 __device__ __forceinline__ void y_sweep(const SweepArgs &a, const Src &src, long wave, int chunks,
                                         double (*st)[64], uint32_t *mlp)
 {
@@ -446,15 +496,19 @@ __device__ __forceinline__ void y_sweep(const SweepArgs &a, const Src &src, long
 
     double s[4] = {0.0, 0.0, 0.0, 0.0};
     if (own) L.limited_sp(wl, w, wr, sp, s);
-    else if (rowv && c == -1) L.ghost_slope(true, s);
-    else if (rowv && c == n) L.ghost_slope(false, s);
 
     double sr[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) sr[q] = __shfl_down(s[q], 1);
-    if (rowv && k == G - 1) {
-        if (last_own) L.limited_sp(w, wr, wrr, sp1, sr);
-        else if (c + 1 == n) L.ghost_slope(false, sr);
+    if (last_own) L.limited_sp(w, wr, wrr, sp1, sr);
+    // the ghosts' slopes from the boundary cells'
+    if (rowv && (c == -1 || c + 1 == n)) {
+        double g[4];
+        L.ghost_slope_near(c == -1, c == -1 ? sr : s, g);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (c == -1) s[q] = g[q]; else sr[q] = g[q];
+        }
     }
 
     double F[4] = {0.0, 0.0, 0.0, 0.0}, I[4] = {0.0, 0.0, 0.0, 0.0};
@@ -471,8 +525,7 @@ __device__ __forceinline__ void y_sweep(const SweepArgs &a, const Src &src, long
         // none of it is held across the solve
         const Side SL = recon(w, s, hh, true);
         const Side SR = recon(wr, sr, hh, false);
-        solve_interface<1, NM>(src.get(), SL, SR,
-                               (unsigned long long)j * (unsigned long long)(n + 1) + (unsigned long long)f, F, I, pg);
+        solve_interface<1, NM, MINW>(src.get(), src, SL, SR, j, f, F, I, pg);
     }
     double Fl[4], Il[4];
 #pragma unroll

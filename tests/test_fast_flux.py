@@ -1,0 +1,89 @@
+"""The steps' interface solver (csrc/grp_fast.hpp: shared reciprocals, no range
+scaling) against the IEEE solver of csrc/grp_device.hpp, both built for the
+host: every interface it takes has the same flux and interface values, bit for
+bit (a zero's sign aside), and it leaves those that are out of its range."""
+import ctypes as C
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+import cases
+from _libs import ROOT
+
+INC = [os.path.join(ROOT, "tests", "native", "shim"), os.path.join(ROOT, "hydrocode-fusion_amd", "csrc")]
+
+
+@pytest.fixture(scope="module")
+def fast(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fasthost") / "fast_host.so")
+    subprocess.run(["g++", "-std=c++17", "-O2", "-ffp-contract=off", "-fPIC", "-shared", *[f"-I{d}" for d in INC],
+                    os.path.join(ROOT, "tests", "native", "fast_host.cpp"), "-o", so], check=True)
+    lib = C.CDLL(so)
+    lib.fh_near_threshold.restype = C.c_double
+    lib.fh_near_threshold.argtypes = [C.c_double]
+    return lib
+
+
+def _dp(a):
+    return a.ctypes.data_as(C.POINTER(C.c_double))
+
+
+def _both(lib, L, R, direction, conv, guess):
+    L, R = np.ascontiguousarray(L), np.ascontiguousarray(R)
+    f, i = np.full((len(L), 9), np.nan), np.zeros((len(L), 9))
+    took = lib.fh_split_many(_dp(L), _dp(R), len(L), C.c_double(1e-3), C.c_double(1e-9), direction, conv,
+                             _dp(np.ascontiguousarray(guess)), _dp(f), _dp(i))
+    return took, f, i
+
+
+@pytest.mark.parametrize("gamma", [1.4, 1.67, 1.05, 3.0])
+@pytest.mark.parametrize("direction", [0, 1])
+@pytest.mark.parametrize("conv", [0, 1])
+def test_same_bits_as_the_ieee_solver(fast, gamma, direction, conv):
+    L, R = cases.interface_pairs(20000, 100 + direction, gamma)
+    guess = np.where(np.arange(len(L)) % 3 == 0, np.sqrt(L[:, 6] * R[:, 6]), -1.0) if conv else np.full(len(L), -1.0)
+    took, f, i = _both(fast, L, R, direction, conv, guess)
+    on = ~np.isnan(f[:, 0])
+    # it takes every interface that opens no vacuum (there p* goes to zero)
+    c = [np.sqrt(gamma * A[:, 6] / A[:, 3]) for A in (L, R)]
+    q = 4 + direction
+    vacuum = R[:, q] - L[:, q] > 0.99 * 2 * (c[0] + c[1]) / (gamma - 1)
+    assert took == on.sum() and np.all(on | vacuum)
+    assert np.array_equal(f[on], i[on])
+
+
+def test_velocities_of_every_magnitude(fast):
+    """Ahead of a front one velocity decays through every magnitude while the
+    pressure is uniform: equal states but for a tiny velocity and its slope."""
+    rng = np.random.default_rng(3)
+    n = 20000
+    L, R = np.zeros((n, 15)), np.zeros((n, 15))
+    for A in (L, R):
+        A[:, 0], A[:, 3], A[:, 6] = 1.4, 1.3, 0.7
+        for q in (4, 5, 8, 9):
+            A[:, q] = np.ldexp(rng.uniform(-1, 1, n), rng.integers(-1074, 0, n)) * (rng.random(n) < 0.7)
+    for direction in (0, 1):
+        took, f, i = _both(fast, L, R, direction, 0, np.full(n, -1.0))
+        on = ~np.isnan(f[:, 0])
+        assert took > 0.9 * n and np.array_equal(f[on], i[on])
+
+
+@pytest.mark.parametrize("at, value", [(3, 1e-40), (6, 1e40), (4, 1e40), (8, np.inf), (10, 1e200), (3, np.nan)])
+def test_out_of_range_is_left_to_the_ieee_solver(fast, at, value):
+    L, R = cases.interface_pairs(8, 5)
+    for A in (L, R):
+        B = [L.copy(), R.copy()]
+        B[0 if A is L else 1][:, at] = value
+        took, f, _ = _both(fast, B[0], B[1], 0, 0, np.full(8, -1.0))
+        assert took == 0 and np.isnan(f).all()
+
+
+@pytest.mark.parametrize("eps", [1e-9, 1e-12, 0.3, 1e-3, 7.3e-200, 1e-170, 1e160])
+def test_acoustic_switch_threshold(fast, eps):
+    """sqrt(x) < eps exactly where x < near_threshold(eps)."""
+    t = fast.fh_near_threshold(eps)
+    below, above = np.nextafter(t, 0.0), t
+    assert np.sqrt(above) >= eps and (t == 0.0 or np.sqrt(below) < eps)
+    assert fast.fh_near_threshold(0.0) == 0.0 and fast.fh_near_threshold(np.inf) == np.inf
