@@ -22,12 +22,18 @@
 
 namespace hgrp {
 
+// The seeds: within 2^-24.3 of 1/b (4e9 values on gfx950), and rounded where b
+// is one ulp below a power of two, the one b that the steps below could not put
+// right.  A host build's are as rough, but rounded over the few b just below a
+// power of two for which two steps from a rough one may end an ulp off (there
+// the device's IEEE division takes the same steps, the host's does not).
 HGRP_HD double rcp_seed(double b)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
-    return __builtin_amdgcn_rcp(b);        // about 2^-24 relative
+    return __builtin_amdgcn_rcp(b);
 #else
-    return 1.0 / b;
+    int e;
+    return fabs(frexp(b, &e)) > 1.0 - 0x1p-47 ? 1.0 / b : 1.0 / b * (1.0 + 0x1.3p-25);
 #endif
 }
 HGRP_HD double rsq_seed(double x)
@@ -35,12 +41,17 @@ HGRP_HD double rsq_seed(double x)
 #if defined(__HIP_DEVICE_COMPILE__)
     return __builtin_amdgcn_rsq(x);
 #else
-    return 1.0 / sqrt(x);
+    return 1.0 / sqrt(x) * (1.0 - 0x1.3p-25);
 #endif
 }
 
-// A divisor b with y = 1/b.  Two Newton steps leave y within 2^-95 of 1/b
-// before its rounding, so it is the rounded reciprocal but for one b in 2^40.
+// A divisor b with y = 1/b, as IEEE division forms it.  Two Newton steps leave y
+// within 2^-95 of 1/b before its rounding: that is the rounded reciprocal
+// except where 1/b lies that close to the middle of two doubles, as it does for
+// every other b just below 1 (1 in 100 there).  A quotient's last step makes up
+// for it (no quotient by 16 M such b was off on gfx950, nor was the IEEE
+// division's, which takes the same steps); a reciprocal that is a result takes
+// that step too (recip_q).
 struct Rcp {
     double b, y;
 };
@@ -58,6 +69,8 @@ HGRP_HD double div_q(double a, const Rcp &r)
     const double q = a * r.y;
     return fma(-fma(q, r.b, -a), r.y, q);
 }
+HGRP_HD double recip_q(const Rcp &r) { return fma(-fma(r.y, r.b, -1.0), r.y, r.y); }
+HGRP_HD double recip_1(double b) { return recip_q(rcp_of(b)); }
 HGRP_HD double div_1(double a, double b) { return div_q(a, rcp_of(b)); }
 
 // sqrt(x); *half_inv receives 1/(2 sqrt(x)) to about 2^-47
@@ -78,7 +91,9 @@ HGRP_HD double sqrt_q(double x)
     double h;
     return sqrt_h(x, &h);
 }
-// sqrt(x) as a divisor: its reciprocal comes from the root's own seed
+// sqrt(x) as a divisor, x >= 1: its reciprocal, rounded, comes from the root's
+// own seed (2^-94 before the rounding; no root from 1 up has a reciprocal so
+// close to the middle of two doubles)
 HGRP_HD Rcp sqrt_rcp(double x)
 {
     double h;

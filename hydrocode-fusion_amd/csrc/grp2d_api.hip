@@ -869,6 +869,7 @@ static void fill_unsplit_args(hgrp2d *c, UnsplitArgs &a, double tau, double nu, 
     a.div_hx = recip_div(c->cfg[10]); a.div_hy = recip_div(c->cfg[11]);
     a.tau = tau; a.nu = nu; a.mu = mu;
     a.eps = c->cfg[4];
+    a.near2 = near_threshold(a.eps);
     a.alpha = c->cfg[41];
     a.tol = c->newton_tol > 0.0 ? c->newton_tol : a.eps;
     a.conv = c->newton_rule == HGRP_NEWTON_CONVERGE;

@@ -30,16 +30,17 @@ HGRP_HD bool tiny(double x) { return fabs(x) < 0x1p-300 && x != 0.0; }
 // 2^100.  Ahead of a front velocities decay cell by cell through every
 // magnitude down to the denormals, over regions tens of cells wide, while
 // differences of pressure and density stop at their rounding: so what may be a
-// velocity (or a fraction) by itself is divided by IEEE division where such
-// interfaces come (the acoustic case, the passive members), and grp_q1d_q
-// leaves those that need the Riemann solve.
+// velocity (or a fraction) by itself is divided by IEEE division in the
+// acoustic case and in the passive members, and after the Riemann solve where
+// a wave holds such an interface (div_r).
+HGRP_HD double magnitude(const Side &S)           // of the velocities and derivatives; NaN for a NaN
+{
+    return ((fabs(S.u) + fabs(S.v)) + (fabs(S.d_rho) + fabs(S.d_u))) + (fabs(S.d_v) + fabs(S.d_p));
+}
 HGRP_HD bool sides_in_range(const Side &L, const Side &R)
 {
-    const double a = fmax(fmax(L.rho, L.p), fmax(R.rho, R.p)), b = fmax(fabs(L.u), fabs(R.u));
-    const double c = fmax(fmax(fabs(L.d_rho), fabs(R.d_rho)), fmax(fabs(L.d_u), fabs(R.d_u)));
-    const double d = fmax(fmax(fabs(L.d_v), fabs(R.d_v)), fmax(fabs(L.d_p), fabs(R.d_p)));
     return L.rho >= 0x1p-100 && L.p >= 0x1p-100 && R.rho >= 0x1p-100 && R.p >= 0x1p-100 &&
-           fmax(fmax(a, b), fmax(c, d)) <= 0x1p100;
+           fmax(fmax(L.rho, L.p), fmax(R.rho, R.p)) <= 0x1p100 && magnitude(L) + magnitude(R) <= 0x1p100;
 }
 // a / rho, b / rho, c / rho of a cell's update
 __device__ __forceinline__ void quot3(double a, double b, double c, double rho, double &qa, double &qb, double &qc)
@@ -61,6 +62,17 @@ __device__ __forceinline__ void quot3(double a, double b, double c, double rho, 
         qc = q.q[2];
     }
 }
+HGRP_HD bool any_lane(bool x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __any(x);
+#else
+    return x;
+#endif
+}
+// a / r.b; rough (the same for the whole wave): a may be tiny
+HGRP_HD double div_r(double a, const Rcp &r, bool rough) { return rough ? a / r.b : div_q(a, r); }
+
 HGRP_HD bool gas_in_range(const Gas &G) { return G.gm1() >= 0x1p-20 && G.g <= 0x1p20; }
 
 // ---- the exact Riemann solve ---------------------------------------------------------
@@ -93,7 +105,7 @@ HGRP_HD double slope_q(double p, const Rcp &p_s, double c_s, const Gas &G, const
         const double t3 = div_q(0.5 * t2 * G.nu, p_s);
         return t2 * t1 - t3 * (p - p_s.b) * cube(t1);
     }
-    return rcp_of(pow_in_range(keep, G.nu)).y * t2;
+    return recip_1(pow_in_range(keep, G.nu)) * t2;
 }
 
 struct StarQ {
@@ -101,12 +113,11 @@ struct StarQ {
     int crw0, crw1;
 };
 
-// riemann_exact with N = 500; false where the pressure leaves the range (or is not a number)
-template <bool CONV>
+// riemann_exact with at most N steps; false where the pressure leaves the range (or is not a number)
+template <bool CONV, int N = 500>
 HGRP_HD bool riemann_q(const Gas &GL, const Gas &GR, double u_L, double u_R, const Rcp &p_L, const Rcp &p_R,
                        double c_L, double c_R, double eps, double tol, double p_guess, StarQ &out)
 {
-    constexpr int N = 500;
     DD bL = {0.0, 0.0}, bR = {0.0, 0.0};
     const double u_LR = curve_q<-1>(p_R.b, u_L, p_L, c_L, GL, &bL);
     const double u_RL = curve_q<+1>(p_L.b, u_R, p_R, c_R, GR, &bR);
@@ -225,7 +236,8 @@ HGRP_HD void line_q(const Rcp &rho, double p, double c, double d_rho, double d_u
         double TdS, dI;
         invariants_q<SIGN>(rho, c, d_rho, d_u, d_p, G, TdS, dI);
         o.a = 1.0;
-        o.b = div_1(SIGN < 0 ? rrs.y : -rrs.y, cs);
+        const double inv = recip_q(rrs);
+        o.b = div_1(SIGN < 0 ? inv : -inv, cs);
         o.d = fan_line_q<SIGN>(div_1(cs, c), c, G, TdS, dI, &o.xb);
         o.Ss = o.S = 0.0;
     } else {
@@ -238,7 +250,7 @@ HGRP_HD void line_q(const Rcp &rho, double p, double c, double d_rho, double d_u
         const double H1 = div_q(0.5 * V * (p_star + G.op2z() * p), rq);
         const double H2 = div_q(-0.5 * V * (G.tpz() * p_star + G.z * p), rq);
         const double H3 = div_q(-0.5 * V * (p_star - p), rho);
-        const double inv = -rho.y;
+        const double inv = -recip_q(rho);
         const double h = rho.b * (c * c * H2 + H3);
         const double L_p = SIGN < 0 ? inv - S * H2 : inv + S * H2;
         const double L_u = SIGN < 0 ? S + h : S - h;
@@ -268,6 +280,7 @@ HGRP_HD bool grp_q1d_q(double D[4], double U[4], const Side &L, const Side &R, c
     const bool near = dist2 < near2;
 
     StarQ st;
+    bool rough = false;
     double rs_L, rs_R, cs_L, cs_R, speed_L, speed_R;
     if (near) {
         st.u = 0.5 * (R.u + L.u);
@@ -276,7 +289,7 @@ HGRP_HD bool grp_q1d_q(double D[4], double U[4], const Side &L, const Side &R, c
         rs_L = L.rho; cs_L = c_L; speed_L = st.u - c_L;
         rs_R = R.rho; cs_R = c_R; speed_R = st.u + c_R;
     } else {
-        if (tiny(L.u) || tiny(R.u) || tiny(L.d_u) || tiny(R.d_u)) return false;
+        rough = any_lane(tiny(L.u) || tiny(R.u) || tiny(L.d_u) || tiny(R.d_u));
         const Rcp pL = rcp_of(L.p), pR = rcp_of(R.p);
         if (!riemann_q<CONV>(GL, GR, L.u, R.u, pL, pR, c_L, c_R, eps, tol, p_guess, st)) return false;
         behind_q<-1>(L.rho, L.u, pL, c_L, st.p, st.crw0, GL, rs_L, cs_L, speed_L);
@@ -348,6 +361,7 @@ HGRP_HD bool grp_q1d_q(double D[4], double U[4], const Side &L, const Side &R, c
         const double tc = div_q(2.0 * c, {G.gm1(), G.y_gm1});
         U[1] = G.z * (in0 ? L.u + tc : R.u - tc);
         C = in0 ? U[1] : -U[1];
+        if (!(C >= 0x1p-200)) return false;                // no sonic point (a vacuum that the iteration left)
         const Rcp rC = rcp_of(C);
         const double x = div_1(C, c);
         U[3] = pow_in_range(log_in_range(x), G.e_sonic) * p;
@@ -371,23 +385,23 @@ HGRP_HD bool grp_q1d_q(double D[4], double U[4], const Side &L, const Side &R, c
         line_q<-1>(rL, L.p, c_L, L.d_rho, L.d_u, L.d_p, p_star, rs_L, cs_L, st.crw0, GL, l);
         line_q<+1>(rR, R.p, c_R, R.d_rho, R.d_u, R.d_p, p_star, rs_R, cs_R, st.crw1, GR, r);
         const Rcp det = rcp_of(l.a * r.b - l.b * r.a);
-        const double u_t = div_q(r.b * l.d - l.b * r.d, det);
-        const double p_t = div_q(l.a * r.d - r.a * l.d, det);
+        const double u_t = div_r(r.b * l.d - l.b * r.d, det, rough);
+        const double p_t = div_r(l.a * r.d - r.a * l.d, det, rough);
         // the side of the contact that the t-axis lies on
         const bool right = u_star < 0.0;
         const double rs = right ? rs_R : rs_L;
         C = right ? cs_R : cs_L;
         const Rcp rC = rcp_of(C), rrs = rcp_of(rs), rho = {right ? R.rho : L.rho, right ? rR.y : rL.y};
         U[0] = rs; U[1] = u_star; U[2] = right ? R.v : L.v; U[3] = p_star;
-        D[1] = u_t + div_q(div_q(div_q(u_star, rrs), rC), rC) * p_t;
+        D[1] = u_t + div_r(div_r(div_r(u_star, rrs, rough), rC, rough), rC, rough) * p_t;
         D[3] = p_t + u_star * rs * u_t;
         const double c = right ? c_R : c_L, p = right ? R.p : L.p, z = right ? GR.z : GL.z;
         const double d_rho = right ? R.d_rho : L.d_rho, d_u = right ? R.d_u : L.d_u, d_p = right ? R.d_p : L.d_p;
         const double d_v = right ? R.d_v : L.d_v;
         if (right ? st.crw1 : st.crw0) {
             const double xb = right ? r.xb : l.xb;
-            D[0] = div_q(rs * u_star * xb * (d_p - d_rho * c * c), rho);
-            D[0] = div_q(div_q(D[0] + D[3], rC), rC);
+            D[0] = div_r(rs * u_star * xb * (d_p - d_rho * c * c), rho, rough);
+            D[0] = div_r(div_r(D[0] + D[3], rC, rough), rC, rough);
             D[2] = -u_star * d_v * rs / rho.b;
             if constexpr (TF) { FO[0] = right ? FA[2] : FA[0]; FO[1] = -u_star * (right ? FA[3] : FA[1]) * rs / rho.b; }
         } else {
@@ -400,7 +414,7 @@ HGRP_HD bool grp_q1d_q(double D[4], double U[4], const Side &L, const Side &R, c
             const double L_u = -rho.b * (H2 * c * c + H3) * d_u;
             const double L_p = H2 * S * d_p;
             D[0] = (div_q(div_q(u_star + Ss, rC), rC) - u_star * H1) * p_t + rs * u_star * Ss * H1 * u_t;
-            D[0] = div_q(D[0] - u_star * (L_p + L_rho + L_u), rSs);
+            D[0] = div_r(D[0] - u_star * (L_p + L_rho + L_u), rSs, rough);
             // the reference adds lambda times a derivative over S + u here: nothing but NaN where that is zero
             if (S + (right ? R.u : L.u) == 0.0) D[0] = NAN;
             D[2] = -u_star * S * d_v / Ss;
@@ -454,6 +468,129 @@ __device__ __forceinline__ bool flux_split_q(const Side &L, const Side &R, const
     if (!grp_q1d_q<false, false, CONV>(D, U, l, r, nullptr, nullptr, G, G, near2, eps, tol, p_guess, nullptr, nullptr))
         return false;
     *code = flux_from_mid<DIR>(U, D, G, tau, eps, F, I);
+    return true;
+}
+
+// GRP_2D_flux in the unsplit step (grp_2d_flux_n: one gas, tangential
+// derivatives in grid axes), normal x (dir 0) or y (dir 1).
+template <bool CONV>
+__device__ __forceinline__ bool flux_transversal_q(const Side &L, const Side &R, const double TL[4], const double TR[4],
+                                                   const Gas &G, int dir, double near2, double tau, double eps, double F[4],
+                                                   double I[4], double tol, double p_guess, int *code)
+{
+    const double t = ((fabs(TL[0]) + fabs(TL[1])) + (fabs(TL[2]) + fabs(TL[3]))) +
+                     ((fabs(TR[0]) + fabs(TR[1])) + (fabs(TR[2]) + fabs(TR[3])));
+    if (!(gas_in_range(G) && sides_in_range(L, R) && t <= 0x1p100)) return false;
+    Side l = L, r = R;
+    double tl[4] = {TL[0], TL[1], TL[2], TL[3]}, tr[4] = {TR[0], TR[1], TR[2], TR[3]};
+    if (dir) {                                   // into the interface's frame
+        l.u = L.v; l.v = -L.u; l.d_u = L.d_v; l.d_v = -L.d_u;
+        r.u = R.v; r.v = -R.u; r.d_u = R.d_v; r.d_v = -R.d_u;
+        tl[1] = TL[2]; tl[2] = -TL[1];
+        tr[1] = TR[2]; tr[2] = -TR[1];
+    }
+    double D[4], U[4];
+    if (!grp_q1d_q<true, false, CONV>(D, U, l, r, tl, tr, G, G, near2, eps, tol, p_guess, nullptr, nullptr)) return false;
+    *code = flux_from_mid_n(U, D, G, dir ? 0.0 : 1.0, dir ? 1.0 : 0.0, tau, eps, F, I);
+    return true;
+}
+
+// ---- two fluids --------------------------------------------------------------------
+// mix_gamma, gas_of: a fraction is divided by constants, and what a tiny one's
+// quotient may be off by is lost in the sum
+__device__ __forceinline__ double mix_inv_gm1_q(double fa, const TwoGas &T)
+{
+    return div_q(fa, {T.a.gm1(), T.a.y_gm1}) + div_q(1.0 - fa, {T.b.gm1(), T.b.y_gm1});
+}
+__device__ __forceinline__ double mix_gamma_q(double fa, const TwoGas &T) { return recip_1(mix_inv_gm1_q(fa, T)) + 1.0; }
+
+__device__ __forceinline__ Gas make_gas_q(double g)      // make_gas for gas_in_range(g)
+{
+    const double gm1 = g - 1.0, gp1 = g + 1.0;
+    Rcp rg = rcp_of(g), rm = rcp_of(gm1);
+    rg.y = recip_q(rg);
+    rm.y = recip_q(rm);
+    const Rcp r2g = {2.0 * g, 0.5 * rg.y};
+    Gas s;
+    s.g = g;
+    s.mu = div_q(gm1, r2g);
+    s.nu = div_q(gp1, r2g);
+    s.z = div_1(gm1, gp1);
+    s.inv_g = rg.y;
+    s.e_cs = s.mu;                               // 0.5 (g-1) / g, the same quotient
+    s.e_sonic = div_q(2.0 * g, rm);
+    const Rcp rz = rcp_of(s.z);
+    s.e_a = div_q(0.5, rz);
+    s.e_b = div_q(1.0 + s.z, rz);
+    s.g_gm1 = div_q(g, rm);
+    s.y_gm1 = rm.y;
+    s.y_op2z = recip_1(s.op2z());
+    return s;
+}
+__device__ __forceinline__ bool two_in_range(const TwoGas &T)
+{
+    return T.a.gm1() >= 0x1p-20 && T.a.g <= 0x1p20 && T.b.gm1() >= 0x1p-20 && T.b.g <= 0x1p20;
+}
+
+// GRP_2D_flux with two fluids (grp_2d_flux_tf).
+template <int DIR, bool CONV>
+__device__ __forceinline__ bool flux_two_fluid_q(const Side &L, const Side &R, const TwoGas &T, const double FA[4],
+                                                 double near2, double tau, double eps, double F[4], double I[4],
+                                                 double FZ[3], double tol, double p_guess, int *code)
+{
+    constexpr double n_x = DIR == 0 ? 1.0 : 0.0, n_y = DIR == 0 ? 0.0 : 1.0;
+    // reconstructed fractions leave [0, 1] by rounding only
+    const bool fr = FA[0] >= -0.5 && FA[0] <= 1.5 && FA[2] >= -0.5 && FA[2] <= 1.5 &&
+                    fabs(FA[1]) + fabs(FA[3]) <= 0x1p100;
+    if (!(fr && two_in_range(T) && sides_in_range(L, R))) return false;
+    const bool pure_L = FA[0] == 1.0 || FA[0] == 0.0, pure_R = FA[2] == 1.0 || FA[2] == 0.0;
+    Gas GL = FA[0] == 1.0 ? T.a : T.b, GR = FA[2] == 1.0 ? T.a : T.b;
+    if (!pure_L) GL = make_gas_q(mix_gamma_q(FA[0], T));
+    if (!pure_R) GR = make_gas_q(mix_gamma_q(FA[2], T));
+    if (!(gas_in_range(GL) && gas_in_range(GR))) return false;
+    Side l = L, r = R;
+    if constexpr (DIR == 1) {
+        l.u = L.v; l.v = -L.u; l.d_u = L.d_v; l.d_v = -L.d_u;
+        r.u = R.v; r.v = -R.u; r.d_u = R.d_v; r.d_v = -R.d_u;
+    }
+    double dire[4], mid[4], fo[2];
+    if (!grp_q1d_q<false, true, CONV>(dire, mid, l, r, nullptr, nullptr, GL, GR, near2, eps, tol, p_guess, FA, fo))
+        return false;
+    *code = star_dire_bad(mid, dire, eps);
+    if (*code) {
+        F[0] = F[1] = F[2] = F[3] = 0.0;
+        I[0] = I[1] = I[2] = I[3] = 0.0;
+        FZ[0] = FZ[1] = FZ[2] = 0.0;
+        return true;
+    }
+    const double rho_mid = mid[0] + 0.5 * tau * dire[0];
+    const double u_mid = (mid[1] + 0.5 * tau * dire[1]) * n_x - (mid[2] + 0.5 * tau * dire[2]) * n_y;
+    const double v_mid = (mid[1] + 0.5 * tau * dire[1]) * n_y + (mid[2] + 0.5 * tau * dire[2]) * n_x;
+    const double p_mid = mid[3] + 0.5 * tau * dire[3];
+    const double a_mid = fo[0] + 0.5 * tau * fo[1];
+    double ge = a_mid == 1.0 ? T.a.g_gm1 : T.b.g_gm1;
+    if (!(a_mid == 1.0 || a_mid == 0.0)) {
+        if (a_mid >= -0.5 && a_mid <= 1.5) {
+            const double gamma_mid = mix_gamma_q(a_mid, T);
+            ge = div_1(gamma_mid, gamma_mid - 1.0);
+        } else {
+            const double gamma_mid = mix_gamma(a_mid, T);
+            ge = gamma_mid / (gamma_mid - 1.0);
+        }
+    }
+    F[0] = rho_mid * (u_mid * n_x + v_mid * n_y);
+    F[1] = F[0] * u_mid + p_mid * n_x;
+    F[2] = F[0] * v_mid + p_mid * n_y;
+    F[3] = ge * p_mid / rho_mid + 0.5 * (u_mid * u_mid + v_mid * v_mid);
+    F[3] = F[0] * F[3];
+    I[1] = (mid[1] + tau * dire[1]) * n_x - (mid[2] + tau * dire[2]) * n_y;
+    I[2] = (mid[1] + tau * dire[1]) * n_y + (mid[2] + tau * dire[2]) * n_x;
+    I[0] = mid[0] + tau * dire[0];
+    I[3] = mid[3] + tau * dire[3];
+    const double un_mid = u_mid * n_x + v_mid * n_y;
+    FZ[0] = un_mid * a_mid;
+    FZ[1] = un_mid;
+    FZ[2] = fo[0] + tau * fo[1];
     return true;
 }
 

@@ -205,7 +205,7 @@ __device__ inline float mlp_eval_wave(const MlpPacked *__restrict__ W, const flo
 // start from p_TR itself, which is already within O(jump^3) of p* and where
 // the network's correction is nil, and so do two rarefactions of one gas; the
 // network runs only in waves that hold another (strong) interface.
-__device__ inline double learned_guess_wave(const MlpPacked *__restrict__ W, bool want, double rho_L, double u_L,
+__device__ __attribute__((noinline)) inline double learned_guess_wave(const MlpPacked *__restrict__ W, bool want, double rho_L, double u_L,
                                             double p_L, double rho_R, double u_R, double p_R, double g_L,
                                             double g_R, uint32_t *lds)
 {

@@ -83,38 +83,14 @@ struct Grid {
     __device__ __forceinline__ void limit(const double vm[4], const double v0[4], const double vp[4], const double *prev,
                           size_t o, int lim3, const RecipDiv &d, double s[4]) const
     {
+        double d_L[4], d_R[4], s_L[4], s_R[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const double s_L = div_by(v0[q] - vm[q], d);
-            const double s_R = div_by(vp[q] - v0[q], d);
-            s[q] = lim3 ? minmod3(a.alpha * s_L, a.alpha * s_R, prev[o + q * a.plane]) : minmod2(s_L, s_R);
-        }
-    }
-    __device__ __forceinline__ void lim_x(int c, int ci, const double v0[4], double s[4]) const
-    {
-        double vm[4], vp[4];
-        xval(c - 1, ci, vm);
-        xval(c + 1, ci, vp);
-        limit(vm, v0, vp, a.s, at(c, ci), a.lim3_x, a.div_hx, s);
-    }
-    __device__ __forceinline__ void lim_y(int c, int ci, const double v0[4], double t[4]) const
-    {
-        double vm[4], vp[4];
-        yval(c, ci - 1, vm);
-        yval(c, ci + 1, vp);
-        limit(vm, v0, vp, a.t, at(c, ci), a.lim3_y, a.div_hy, t);
-    }
-    __device__ __forceinline__ void lim_x_at(int c, int ci, double s[4]) const
-    {
-        double v0[4];
-        cell(c, ci, v0);
-        lim_x(c, ci, v0, s);
-    }
-    __device__ __forceinline__ void lim_y_at(int c, int ci, double t[4]) const
-    {
-        double v0[4];
-        cell(c, ci, v0);
-        lim_y(c, ci, v0, t);
+        for (int q = 0; q < 4; ++q) { d_L[q] = v0[q] - vm[q]; d_R[q] = vp[q] - v0[q]; }
+        quot4(d_L, d, s_L);
+        quot4(d_R, d, s_R);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            s[q] = lim3 ? minmod3(a.alpha * s_L[q], a.alpha * s_R[q], prev[o + q * a.plane]) : minmod2(s_L[q], s_R[q]);
     }
 
     // Side data of (c, ci): value v, x-slope s, y-slope t.  A cell: its limited
@@ -123,46 +99,37 @@ struct Grid {
     // the boundary cell (bound_cond_slope_limiter_y.c:111-126).  A y-ghost
     // (ci = -1 or n): bfv_D/U with the mirrored rules.  Slopes the reference
     // never sets stay zero (its ghost arrays are calloc'ed).  Not for corners.
+    // Every ghost takes what it takes from one cell: the one next to it, or the
+    // last one of the line with periodic ends; so one limiter serves all.
     __device__ __forceinline__ void side(int c, int ci, double v[4], double s[4], double t[4]) const
     {
         const bool xin = c >= 0 && c < a.m, yin = ci >= 0 && ci < a.n;
+        const bool lo = c < 0 || ci < 0;
+        const int bc = xin ? a.bc_y : a.bc_x;                 // of a ghost
+        const bool far = bc == BC_PERIODIC;
+        const int cs = xin ? c : (lo != far ? 0 : a.m - 1), is = yin ? ci : (lo != far ? 0 : a.n - 1);
+        double v0[4], vm[4], vp[4];
+        cell(cs, is, v0);
+        xval(cs - 1, is, vm);
+        xval(cs + 1, is, vp);
+        limit(vm, v0, vp, a.s, at(cs, is), a.lim3_x, a.div_hx, s);
+        yval(cs, is - 1, vm);
+        yval(cs, is + 1, vp);
+        limit(vm, v0, vp, a.t, at(cs, is), a.lim3_y, a.div_hy, t);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) { s[q] = 0.0; t[q] = 0.0; }
-        if (xin && yin) {
-            cell(c, ci, v);
-            lim_x(c, ci, v, s);
-            lim_y(c, ci, v, t);
-        } else if (yin) {
-            const bool lo = c < 0;
-            const int near = lo ? 0 : a.m - 1, far = lo ? a.m - 1 : 0;
-            xval(c, ci, v);
-            double q4[4];
-            switch (a.bc_x) {
-            case BC_REFLECT: lim_x_at(near, ci, q4); s[1] = q4[1]; break;
-            case BC_PERIODIC: lim_x_at(far, ci, s); break;
-            case BC_REFLECT_FREE: if (lo) { lim_x_at(0, ci, q4); s[1] = q4[1]; } break;
-            default: break;
+        for (int q = 0; q < 4; ++q) v[q] = v0[q];
+        if (!(xin && yin)) {
+            // the normal velocity and its slope across the boundary that the ghost lies behind
+            const bool mirror = bc == BC_REFLECT || (bc == BC_REFLECT_FREE && lo);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const bool normal = q == (xin ? 2 : 1);
+                if (mirror && normal) v[q] = -v[q];
+                if (!(far || (mirror && normal))) { if (xin) t[q] = 0.0; else s[q] = 0.0; }
+                if (bc == BC_INITIAL) { if (xin) s[q] = 0.0; else t[q] = 0.0; }
             }
-            switch (a.bc_x) {
-            case BC_REFLECT: case BC_FREE: case BC_REFLECT_FREE: lim_y_at(near, ci, t); break;
-            case BC_PERIODIC: lim_y_at(far, ci, t); break;
-            default: break;
-            }
-        } else {
-            const bool lo = ci < 0;
-            const int near = lo ? 0 : a.n - 1, far = lo ? a.n - 1 : 0;
-            yval(c, ci, v);
-            double q4[4];
-            switch (a.bc_y) {
-            case BC_REFLECT: lim_y_at(c, near, q4); t[2] = q4[2]; break;
-            case BC_PERIODIC: lim_y_at(c, far, t); break;
-            case BC_REFLECT_FREE: if (lo) { lim_y_at(c, 0, q4); t[2] = q4[2]; } break;
-            default: break;
-            }
-            switch (a.bc_y) {
-            case BC_REFLECT: case BC_FREE: case BC_REFLECT_FREE: lim_x_at(c, near, s); break;
-            case BC_PERIODIC: lim_x_at(c, far, s); break;
-            default: break;
+            if (bc == BC_INITIAL) {
+                if (xin) yval(c, ci, v); else xval(c, ci, v);
             }
         }
     }
@@ -172,19 +139,63 @@ struct Grid {
 // or y (dir 1); failures are recorded in status[dir] as
 // ((loop index << 2) | code) + 1, the reference's loop order
 // G2: GRP_2D_flux with its alternative solver, G2D (grp_2d_flux_g2d).
+// (c, ci): the cell on its left (lower) side.
+
+// The face with the IEEE solver, from the cells in memory: what the fast solver
+// leaves (grp_fast.hpp).
+template <int NM>
+__device__ __attribute__((noinline)) int redo_face_t(const UnsplitArgs *ap, int dir, int c, int ci, double p_guess,
+                                                     double *FI)
+{
+    const UnsplitArgs &a = *ap;
+    const Grid G(a);
+    double vl[4], sl[4], tl[4], vr[4], sr[4], tr[4];
+    G.side(c, ci, vl, sl, tl);
+    G.side(dir ? c : c + 1, dir ? ci + 1 : ci, vr, sr, tr);
+    if (dir) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            double x = sl[q];
+            sl[q] = tl[q]; tl[q] = -x;
+            x = sr[q];
+            sr[q] = tr[q]; tr[q] = -x;
+        }
+    }
+    const double hh = dir ? a.hh_y : a.hh_x;
+    return grp_2d_flux_n<NM != NM_REF>(recon(vl, sl, hh, true), recon(vr, sr, hh, false), tl, tr, a.gas, dir ? 0.0 : 1.0,
+                                       dir ? 1.0 : 0.0, a.tau, a.eps, FI, FI + 4, a.tol, p_guess);
+}
+
 template <int NM, bool G2>
 __device__ __forceinline__ void solve_t(const UnsplitArgs &a, int dir, const Side &SL, const Side &SR,
-                                        const double TL[4], const double TR[4], unsigned long long loop_index,
-                                        double F[4], double I[4], double p_guess)
+                                        const double TL[4], const double TR[4], int c, int ci, double F[4], double I[4],
+                                        double p_guess)
 {
-    int code = ifvar_bad_t(SL, SR, TL, TR, a.eps) ? 1 : 0;
+    int code = ifvar_bad_t(SL, SR, TL, TR, a.eps) ? 1 : 0, bad = 0;
     const double n_x = dir ? 0.0 : 1.0, n_y = dir ? 1.0 : 0.0;
-    const int bad = G2 ? grp_2d_flux_g2d<NM != NM_REF>(SL, SR, TL, TR, a.gas, n_x, n_y, a.tau, a.eps, F, I, a.tol,
-                                                       p_guess)
-                       : grp_2d_flux_n<NM != NM_REF>(SL, SR, TL, TR, a.gas, n_x, n_y, a.tau, a.eps, F, I, a.tol,
-                                                     p_guess);
+    if constexpr (G2) {
+        bad = grp_2d_flux_g2d<NM != NM_REF>(SL, SR, TL, TR, a.gas, n_x, n_y, a.tau, a.eps, F, I, a.tol, p_guess);
+    } else {
+        const bool done = flux_transversal_q<NM != NM_REF>(SL, SR, TL, TR, a.gas, dir, a.near2, a.tau, a.eps, F, I, a.tol,
+                                                           p_guess, &bad);
+        if (__builtin_expect(__any(!done), 0)) {
+            if (!done) {
+                const UnsplitArgs ar = reload_args<UnsplitArgs>();
+                double o[8];
+                bad = redo_face_t<NM>(&ar, dir, c, ci, p_guess, o);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) { F[q] = o[q]; I[q] = o[4 + q]; }
+            }
+        }
+    }
     if (bad) code = 2;
-    if (code) atomicMax(&a.status[dir].fail_key, ((loop_index << 2) | (unsigned long long)code) + 1ull);
+    if (code) {
+        const UnsplitArgs ar = reload_args<UnsplitArgs>();
+        const unsigned long long index =
+            dir ? (unsigned long long)c * (unsigned long long)(ar.n + 1) + (unsigned long long)(ci + 1)
+                : (unsigned long long)ci * (unsigned long long)(ar.m + 1) + (unsigned long long)(c + 1);
+        atomicMax(&ar.status[dir].fail_key, ((index << 2) | (unsigned long long)code) + 1ull);
+    }
 }
 
 // Learned starting pressure for the interface (SL | SR) with normal x (dir 0)
@@ -200,25 +211,21 @@ __device__ __forceinline__ double unsplit_guess(const UnsplitArgs &a, bool activ
         return -1.0;
     } else {
         const double uL = dir ? SL.v : SL.u, uR = dir ? SR.v : SR.u;
-        const double dist = sqrt((SL.rho - SR.rho) * (SL.rho - SR.rho) + (uL - uR) * (uL - uR)
-                                 + (SL.p - SR.p) * (SL.p - SR.p));
-        const bool want = active && !(dist < a.eps) && !(fabs(uL - uR) < a.tol && fabs(SL.p - SR.p) < a.tol);
+        const double dist2 = (SL.rho - SR.rho) * (SL.rho - SR.rho) + (uL - uR) * (uL - uR)
+                             + (SL.p - SR.p) * (SL.p - SR.p);
+        const bool want = active && !(dist2 < a.near2) && !(fabs(uL - uR) < a.tol && fabs(SL.p - SR.p) < a.tol);
         return learned_guess_wave(a.mlp, want, SL.rho, uL, SL.p, SR.rho, uR, SR.p, a.gas.g, a.gas.g, lds);
     }
 }
 
 }  // namespace
 
-// TRIM: the y-interface results go to the slope slots of the side data (dead
-// after both solve passes; one more barrier) instead of an array of their own,
-// where the block's LDS would not fit otherwise.
-template <int W, int NM, bool G2, bool TRIM>
+template <int W, int NM, bool G2>
 __device__ __forceinline__ void unsplit_step_body(const UnsplitArgs &a)
 {
     __shared__ double sd[W][12][64];     // side data of row c: value, x-slope, y-slope
     __shared__ double fx[W - 1][8][64];  // x-interface c+1: flux, values at t + tau
-    __shared__ double gy[TRIM ? 1 : W - 2][8][64];  // y-interfaces of the updated rows: flux, values at t + tau
-    __shared__ uint32_t mlp_lds[NM == NM_LEARNED ? W : 1][NM == NM_LEARNED ? 64 * 8 : 1];   // network inputs
+    __shared__ double gy[W - 2][8][64];  // y-interfaces of the updated rows: flux, values at t + tau
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int m = a.m, n = a.n;
     const int i0 = blockIdx.x * 62, ci = i0 - 1 + lane;
@@ -243,79 +250,63 @@ __device__ __forceinline__ void unsplit_step_body(const UnsplitArgs &a)
     }
     __syncthreads();
 
-    // pass 0: x-interface f = c + 1 between rows c and c + 1 (flux_generator_x.c:42-121),
-    //         the right side from the next wave;
-    // pass 1: y-interfaces of the updated rows (flux_generator_y.c:42-121), normal derivative =
-    //         y-slope, transversal = -(x-slope); wave w takes half a row pair (2 rows x 32
-    //         interfaces), so a front lying along y meets half as many waves as with one
-    //         64-lane row per wave.
-    // One solve site for both, so the GRP code and its registers are laid out once.
+    // dir 1: y-interfaces of the updated rows (flux_generator_y.c:42-121), normal derivative =
+    //        y-slope, transversal = -(x-slope); wave w takes half a row pair (2 rows x 32
+    //        interfaces), so a front lying along y meets half as many waves as with one
+    //        64-lane row per wave;
+    // dir 0: x-interface f = c + 1 between rows c and c + 1 (flux_generator_x.c:42-121),
+    //        the right side from the next wave.
+    // One solve site for both, so the GRP code and its registers are laid out once.  The x-pass
+    // comes last: until a wave has solved its x-interfaces its slots of fx are free, and both
+    // passes' network inputs (the learned guess) lie there.
     const int f = c + 1;
     const int task = w - 1;                                  // waves 1 .. W-2
     const int yr = 1 + 2 * (task >> 1) + (lane >> 5);        // tile row of this lane's y-interface
     const int yt = ((task & 1) << 5) + (lane & 31);          // between tile lanes yt and yt + 1
     const int yc = j0 - 1 + yr, ycell = i0 - 1 + yt;
-    double Fy[4] = {0.0, 0.0, 0.0, 0.0}, Iyv[4] = {0.0, 0.0, 0.0, 0.0};   // TRIM: pass 1's results
 #pragma unroll 1
-    for (int pass = 0; pass < 2; ++pass) {
+    for (int dir = 1; dir >= 0; --dir) {
+        const bool active = dir ? w >= 1 && w <= W - 2 && yc >= 0 && yc < m && yt <= 62 && ycell <= n - 1
+                                : w <= W - 2 && lane >= 1 && lane <= 62 && yin && f <= m;
+        const int r0 = dir ? yr : w, k0 = dir ? yt : lane, r1 = dir ? yr : w + 1, k1 = dir ? yt + 1 : lane;
         Side SL, SR;
         double TL[4], TR[4];
-        unsigned long long idx = 0;
-        bool active;
-        if (pass == 0) {
-            active = w <= W - 2 && lane >= 1 && lane <= 62 && yin && f <= m;
-            if (active) {
-                double vl[4], sl[4], vr[4], sr[4];
+        // the two cells' side data: value, normal and transversal slope
+        auto sides = [&]() {
+            const int sn = dir ? 8 : 4, st = dir ? 4 : 8;
+            const double hh = dir ? a.hh_y : a.hh_x;
+            double vl[4], sl[4], vr[4], sr[4];
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    vl[q] = sd[w][q][lane];     sl[q] = sd[w][4 + q][lane];     TL[q] = sd[w][8 + q][lane];
-                    vr[q] = sd[w + 1][q][lane]; sr[q] = sd[w + 1][4 + q][lane]; TR[q] = sd[w + 1][8 + q][lane];
-                }
-                SL = recon(vl, sl, a.hh_x, true);
-                SR = recon(vr, sr, a.hh_x, false);
-                idx = (unsigned long long)ci * (unsigned long long)(m + 1) + (unsigned long long)f;
+            for (int q = 0; q < 4; ++q) {
+                vl[q] = sd[r0][q][k0]; sl[q] = sd[r0][sn + q][k0]; TL[q] = sd[r0][st + q][k0];
+                vr[q] = sd[r1][q][k1]; sr[q] = sd[r1][sn + q][k1]; TR[q] = sd[r1][st + q][k1];
             }
-        } else {
-            active = w >= 1 && w <= W - 2 && yc >= 0 && yc < m && yt <= 62 && ycell <= n - 1;
-            if (active) {
-                double vd[4], td[4], vu[4], tu[4];
+            if (dir)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    vd[q] = sd[yr][q][yt];     td[q] = sd[yr][8 + q][yt];     TL[q] = -sd[yr][4 + q][yt];
-                    vu[q] = sd[yr][q][yt + 1]; tu[q] = sd[yr][8 + q][yt + 1]; TR[q] = -sd[yr][4 + q][yt + 1];
-                }
-                SL = recon(vd, td, a.hh_y, true);
-                SR = recon(vu, tu, a.hh_y, false);
-                idx = (unsigned long long)yc * (unsigned long long)(n + 1) + (unsigned long long)(ycell + 1);
-            }
+                for (int q = 0; q < 4; ++q) { TL[q] = -TL[q]; TR[q] = -TR[q]; }
+            SL = recon(vl, sl, hh, true);
+            SR = recon(vr, sr, hh, false);
+        };
+        double F[4] = {0.0, 0.0, 0.0, 0.0}, I[4] = {0.0, 0.0, 0.0, 0.0}, pg = -1.0;
+        if constexpr (NM == NM_LEARNED) {   // a call: the sides are read again after it, not held across
+            if (active) sides();
+            pg = unsplit_guess<NM>(a, active, dir, SL, SR, (uint32_t *)&fx[w < W - 1 ? w : 0][0][0]);
         }
-        double F[4] = {0.0, 0.0, 0.0, 0.0}, I[4] = {0.0, 0.0, 0.0, 0.0};
-        const double pg = unsplit_guess<NM>(a, active, pass, SL, SR, mlp_lds[NM == NM_LEARNED ? w : 0]);
         // the argument block is read again for the solve, so no scalar register holds it across
-        if (active) solve_t<NM, G2>(reload_args<UnsplitArgs>(), pass, SL, SR, TL, TR, idx, F, I, pg);
-        if (pass == 0 && w <= W - 2) {
+        if (active) {
+            sides();
+            solve_t<NM, G2>(reload_args<UnsplitArgs>(), dir, SL, SR, TL, TR, dir ? yc : c, dir ? ycell : ci, F, I, pg);
+        }
+        if (dir == 0 && w <= W - 2) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) { fx[w][q][lane] = F[q]; fx[w][4 + q][lane] = I[q]; }
         }
-        if (pass == 1 && w >= 1 && w <= W - 2) {
-            if constexpr (TRIM) {
+        if (dir == 1 && w >= 1 && w <= W - 2) {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) { Fy[q] = F[q]; Iyv[q] = I[q]; }
-            } else {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) { gy[yr - 1][q][yt] = F[q]; gy[yr - 1][4 + q][yt] = I[q]; }
-            }
+            for (int q = 0; q < 4; ++q) { gy[yr - 1][q][yt] = F[q]; gy[yr - 1][4 + q][yt] = I[q]; }
         }
     }
     __syncthreads();
-    if constexpr (TRIM) {
-        // every wave is past both passes: the slopes of the side data are dead
-        if (w >= 1 && w <= W - 2) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) { sd[yr][4 + q][yt] = Fy[q]; sd[yr][8 + q][yt] = Iyv[q]; }
-        }
-        __syncthreads();
-    }
 
     // combined update and slope refresh (grp_solver_2D_EUL_source.c:231-262)
     if (w >= 1 && w <= W - 2 && xin && yin && lane >= 1 && lane <= 62) {
@@ -328,55 +319,41 @@ __device__ __forceinline__ void unsplit_step_body(const UnsplitArgs &a)
             vc[q] = sd[w][q][lane];
             Fl[q] = fx[w - 1][q][lane]; Ixl[q] = fx[w - 1][4 + q][lane];
             Fr[q] = fx[w][q][lane];     Ixr[q] = fx[w][4 + q][lane];
-            if constexpr (TRIM) {
-                Gl[q] = sd[w][4 + q][lane - 1]; Iyl[q] = sd[w][8 + q][lane - 1];
-                Gy[q] = sd[w][4 + q][lane];     Iy[q] = sd[w][8 + q][lane];
-            } else {
-                Gl[q] = gy[w - 1][q][lane - 1]; Iyl[q] = gy[w - 1][4 + q][lane - 1];
-                Gy[q] = gy[w - 1][q][lane];     Iy[q] = gy[w - 1][4 + q][lane];
-            }
+            Gl[q] = gy[w - 1][q][lane - 1]; Iyl[q] = gy[w - 1][4 + q][lane - 1];
+            Gy[q] = gy[w - 1][q][lane];     Iy[q] = gy[w - 1][4 + q][lane];
         }
         const double nu = a.nu, mu = a.mu;
         const double mom_x = vc[0] * vc[1] - nu * (Fr[1] - Fl[1]) - mu * (Gy[1] - Gl[1]);
         const double mom_y = vc[0] * vc[2] - nu * (Fr[2] - Fl[2]) - mu * (Gy[2] - Gl[2]);
         const double ene = vc[0] * e_c - nu * (Fr[3] - Fl[3]) - mu * (Gy[3] - Gl[3]);
         const double rho = vc[0] + (-nu * (Fr[0] - Fl[0]) - mu * (Gy[0] - Gl[0]));
-        const double uu = mom_x / rho;
-        const double vv = mom_y / rho;
+        double uu, vv, e_new, dx[4], dy[4], sn[4], tn[4];
+        quot3(mom_x, mom_y, ene, rho, uu, vv, e_new);
         const double p = (ene - 0.5 * mom_x * uu - 0.5 * mom_y * vv) * a.gas.gm1();
         double *fo = a.st_o + o;
         const size_t P = a.plane;
-        fo[0] = rho; fo[P] = uu; fo[2 * P] = vv; fo[4 * P] = ene / rho; fo[3 * P] = p;
+        fo[0] = rho; fo[P] = uu; fo[2 * P] = vv; fo[4 * P] = e_new; fo[3 * P] = p;
         if (p < a.eps || rho < a.eps) atomicOr(&a.status[0].flags, 1u);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            a.s_o[o + q * P] = div_by(Ixr[q] - Ixl[q], a.div_hx);
-            a.t_o[o + q * P] = div_by(Iy[q] - Iyl[q], a.div_hy);
-        }
+        for (int q = 0; q < 4; ++q) { dx[q] = Ixr[q] - Ixl[q]; dy[q] = Iy[q] - Iyl[q]; }
+        quot4(dx, a.div_hx, sn);
+        quot4(dy, a.div_hy, tn);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) { a.s_o[o + q * P] = sn[q]; a.t_o[o + q * P] = tn[q]; }
     }
-}
-
-// LDS of a tile of W rows: side data, x- and y-interface results, the
-// learned guess's network inputs; over 160 KiB the y results move into the
-// side data (TRIM)
-template <int W, int NM>
-constexpr bool tile_trim()
-{
-    return (size_t)W * 12 * 512 + (size_t)(W - 1) * 8 * 512 + (size_t)(W - 2) * 8 * 512 +
-               (NM == NM_LEARNED ? (size_t)W * 2048 : 0) > 160 * 1024;
 }
 
 template <int W, int MINW, int NM>
 __global__ void __launch_bounds__(64 * W, MINW) unsplit_step_kernel(UnsplitArgs a)
 {
-    unsplit_step_body<W, NM, false, tile_trim<W, NM>()>(a);
+    unsplit_step_body<W, NM, false>(a);
 }
 
 // the same step with GRP_2D_flux's alternative interface solver, G2D
 template <int W, int MINW, int NM>
 __global__ void __launch_bounds__(64 * W, MINW) unsplit_step_g2d_kernel(UnsplitArgs a)
 {
-    unsplit_step_body<W, NM, true, tile_trim<W, NM>()>(a);
+    unsplit_step_body<W, NM, true>(a);
 }
 
 // Strip form: one wave per block walks down R cell rows of a 62-cell strip
@@ -428,7 +405,6 @@ __device__ __forceinline__ void unsplit_strip_body(const UnsplitArgs &a, int R)
         for (int pass = 0; pass < 2; ++pass) {
             Side SL, SR;
             double TL[4], TR[4];
-            unsigned long long idx = 0;
             bool active;
             if (pass == 0) {   // y-interface ci + 1 of row r: normal = y-slope, transversal = -(x-slope)
                 active = xin && lane <= 62 && ci <= n - 1;
@@ -441,7 +417,6 @@ __device__ __forceinline__ void unsplit_strip_body(const UnsplitArgs &a, int R)
                     }
                     SL = recon(vd, td, a.hh_y, true);
                     SR = recon(vu, tu, a.hh_y, false);
-                    idx = (unsigned long long)r * (unsigned long long)(n + 1) + (unsigned long long)(ci + 1);
                 }
             } else {           // x-interface r + 1 between rows r and r + 1
                 active = lane >= 1 && lane <= 62 && yin && r + 1 <= m;
@@ -454,12 +429,11 @@ __device__ __forceinline__ void unsplit_strip_body(const UnsplitArgs &a, int R)
                     }
                     SL = recon(vl, sl, a.hh_x, true);
                     SR = recon(vr, sr, a.hh_x, false);
-                    idx = (unsigned long long)ci * (unsigned long long)(m + 1) + (unsigned long long)(r + 1);
                 }
             }
             double Fo[4] = {0.0, 0.0, 0.0, 0.0}, Io[4] = {0.0, 0.0, 0.0, 0.0};
             const double pg = unsplit_guess<NM>(a, active, 1 - pass, SL, SR, mlp_lds);
-            if (active) solve_t<NM, G2>(reload_args<UnsplitArgs>(), 1 - pass, SL, SR, TL, TR, idx, Fo, Io, pg);
+            if (active) solve_t<NM, G2>(reload_args<UnsplitArgs>(), 1 - pass, SL, SR, TL, TR, r, ci, Fo, Io, pg);
             if (pass == 0) {
 #pragma unroll
                 for (int q = 0; q < 4; ++q) { gb[q][lane] = Fo[q]; gb[4 + q][lane] = Io[q]; }
@@ -485,18 +459,19 @@ __device__ __forceinline__ void unsplit_strip_body(const UnsplitArgs &a, int R)
             const double mom_y = vc[0] * vc[2] - nu * (F[2] - Fl[2]) - mu * (Gy[2] - Gl[2]);
             const double ene = vc[0] * e_c - nu * (F[3] - Fl[3]) - mu * (Gy[3] - Gl[3]);
             const double rho = vc[0] + (-nu * (F[0] - Fl[0]) - mu * (Gy[0] - Gl[0]));
-            const double uu = mom_x / rho;
-            const double vv = mom_y / rho;
+            double uu, vv, e_new, dx[4], dy[4], sn[4], tn[4];
+            quot3(mom_x, mom_y, ene, rho, uu, vv, e_new);
             const double p = (ene - 0.5 * mom_x * uu - 0.5 * mom_y * vv) * a.gas.gm1();
             double *fo = a.st_o + o;
             const size_t P = a.plane;
-            fo[0] = rho; fo[P] = uu; fo[2 * P] = vv; fo[4 * P] = ene / rho; fo[3 * P] = p;
+            fo[0] = rho; fo[P] = uu; fo[2 * P] = vv; fo[4 * P] = e_new; fo[3 * P] = p;
             if (p < a.eps || rho < a.eps) atomicOr(&a.status[0].flags, 1u);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                a.s_o[o + q * P] = div_by(I[q] - Ixl[q], a.div_hx);
-                a.t_o[o + q * P] = div_by(Iy[q] - Iyl[q], a.div_hy);
-            }
+            for (int q = 0; q < 4; ++q) { dx[q] = I[q] - Ixl[q]; dy[q] = Iy[q] - Iyl[q]; }
+            quot4(dx, a.div_hx, sn);
+            quot4(dy, a.div_hy, tn);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) { a.s_o[o + q * P] = sn[q]; a.t_o[o + q * P] = tn[q]; }
         }
         // x-interface r + 1 is the next row's lower interface (each lane keeps its own slot)
 #pragma unroll

@@ -34,6 +34,7 @@ struct UnsplitArgs {
     int form;                                 // launch form: 0 by grid size, 1 tile, 2 strip
     double hh_x, hh_y;                        // h/2
     double tau, nu, mu, eps, alpha, tol;      // tau, tau/h_x, tau/h_y, ...
+    double near2;                             // the acoustic switch dist < eps on dist^2 (near_threshold)
     RecipDiv div_hx, div_hy;                  // division by h_x, h_y
     Gas gas;
     const MlpPacked *mlp;                     // learned p* guess, or nullptr (the reference's guess)

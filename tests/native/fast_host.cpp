@@ -2,6 +2,7 @@
 // IEEE solver it stands in for (grp_device.hpp), on the same interfaces.
 #include <hip/hip_runtime.h>
 #include "grp_fast.hpp"
+#include "grp1d_fast.hpp"
 
 using namespace hgrp;
 
@@ -36,6 +37,77 @@ extern "C" int fh_split_many(const double *L, const double *R, int n, double tau
             took += conv ? both<0, true>(l, r, tau, eps, tol, guess[k], f, i) : both<0, false>(l, r, tau, eps, tol, guess[k], f, i);
         else
             took += conv ? both<1, true>(l, r, tau, eps, tol, guess[k], f, i) : both<1, false>(l, r, tau, eps, tol, guess[k], f, i);
+    }
+    return took;
+}
+
+// the unsplit step's flux: tangential derivatives of both sides (members 11..14)
+extern "C" int fh_transversal_many(const double *L, const double *R, int n, double tau, double eps, int dir, double *fast,
+                                   double *ieee)
+{
+    int took = 0;
+    for (int k = 0; k < n; ++k) {
+        const double *l = L + 15 * k, *r = R + 15 * k;
+        const Side a{l[3], l[4], l[5], l[6], l[7], l[8], l[9], l[10]}, b{r[3], r[4], r[5], r[6], r[7], r[8], r[9], r[10]};
+        const Gas G = make_gas(l[0]);
+        double *f = fast + 9 * k, *o = ieee + 9 * k;
+        o[0] = grp_2d_flux_n(a, b, l + 11, r + 11, G, dir ? 0.0 : 1.0, dir ? 1.0 : 0.0, tau, eps, o + 1, o + 5, eps);
+        int code = 0;
+        if (!flux_transversal_q<false>(a, b, l + 11, r + 11, G, dir, near_threshold(eps), tau, eps, f + 1, f + 5, eps, -1.0,
+                                       &code)) {
+            f[0] = NAN;
+            continue;
+        }
+        f[0] = code;
+        ++took;
+    }
+    return took;
+}
+
+// the two-fluid flux: FA = {a_L, d_a_L, a_R, d_a_R} per interface
+extern "C" int fh_two_fluid_many(const double *L, const double *R, const double *FA, int n, double tau, double eps, int dir,
+                                 double ga, double gb, double *fast, double *ieee)
+{
+    int took = 0;
+    TwoGas T;
+    T.a = make_gas(ga);
+    T.b = make_gas(gb);
+    for (int k = 0; k < n; ++k) {
+        const double *l = L + 15 * k, *r = R + 15 * k, *fa = FA + 4 * k;
+        const Side a{l[3], l[4], l[5], l[6], l[7], l[8], l[9], l[10]}, b{r[3], r[4], r[5], r[6], r[7], r[8], r[9], r[10]};
+        double *f = fast + 12 * k, *o = ieee + 12 * k;
+        int code = 0;
+        bool ok;
+        if (dir == 0) {
+            o[0] = grp_2d_flux_tf<0, true>(a, b, T, fa, tau, eps, o + 1, o + 5, o + 9, 1e-12);
+            ok = flux_two_fluid_q<0, true>(a, b, T, fa, near_threshold(eps), tau, eps, f + 1, f + 5, f + 9, 1e-12, -1.0, &code);
+        } else {
+            o[0] = grp_2d_flux_tf<1, true>(a, b, T, fa, tau, eps, o + 1, o + 5, o + 9, 1e-12);
+            ok = flux_two_fluid_q<1, true>(a, b, T, fa, near_threshold(eps), tau, eps, f + 1, f + 5, f + 9, 1e-12, -1.0, &code);
+        }
+        f[0] = ok ? code : NAN;
+        took += ok;
+    }
+    return took;
+}
+
+// the 1D solver: rows of D U
+extern "C" int fh_edir_many(const double *L, const double *R, int n, double eps, double *fast, double *ieee)
+{
+    int took = 0;
+    for (int k = 0; k < n; ++k) {
+        const double *l = L + 15 * k, *r = R + 15 * k;
+        const Side1 a{l[3], l[4], l[6], l[7], l[8], l[10]}, b{r[3], r[4], r[6], r[7], r[8], r[10]};
+        const Gas G = make_gas(l[0]);
+        double *f = fast + 6 * k, *o = ieee + 6 * k;
+        grp_edir(o, o + 3, a, b, G, eps);
+        const Rcp rL = rcp_of(a.rho), rR = rcp_of(b.rho);
+        if (sides1_in_range(a, b) &&
+            grp_edir_q(f, f + 3, a, b, rL, rR, sqrt_q(div_q(G.g * a.p, rL)), sqrt_q(div_q(G.g * b.p, rR)), G,
+                       near_threshold(eps), eps))
+            ++took;
+        else
+            for (int q = 0; q < 6; ++q) f[q] = o[q];
     }
     return took;
 }

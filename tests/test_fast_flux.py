@@ -54,30 +54,82 @@ def test_same_bits_as_the_ieee_solver(fast, gamma, direction, conv):
     assert np.array_equal(f[on], i[on])
 
 
-def test_velocities_of_every_magnitude(fast):
-    """Ahead of a front one velocity decays through every magnitude while the
-    pressure is uniform: equal states but for a tiny velocity and its slope."""
-    rng = np.random.default_rng(3)
-    n = 20000
+def _tails(n, seed, jump):
+    """Interfaces ahead of a front: uniform pressure to within its rounding and
+    velocities of every magnitude down to the denormals; `jump`: a contact too."""
+    rng = np.random.default_rng(seed)
     L, R = np.zeros((n, 15)), np.zeros((n, 15))
+    some = lambda f: (rng.random(n) < f)
     for A in (L, R):
         A[:, 0], A[:, 3], A[:, 6] = 1.4, 1.3, 0.7
-        for q in (4, 5, 8, 9):
-            A[:, q] = np.ldexp(rng.uniform(-1, 1, n), rng.integers(-1074, 0, n)) * (rng.random(n) < 0.7)
-    for direction in (0, 1):
-        took, f, i = _both(fast, L, R, direction, 0, np.full(n, -1.0))
+        if jump:
+            A[:, 3] = np.where(some(0.5), rng.uniform(0.1, 1.3, n), 1.0 - np.arange(n) % 16 * 2.0 ** -53)
+            A[:, 6] = 1.0 - 2.0 ** -53 * rng.integers(0, 16, n)
+            A[:, 7] = np.where(some(0.5), rng.uniform(-1, 1, n), 0.0)
+            A[:, 10] = np.where(some(0.5), 2.0 ** -42 * rng.integers(-9, 9, n), 0.0)
+        low = np.where(some(0.5), -200, -1074)
+        for q in (4, 5, 8, 9, 12, 13):
+            A[:, q] = np.ldexp(rng.uniform(-1, 1, n), (low * rng.random(n)).astype(int)) * some(0.7)
+    return L, R, rng
+
+
+@pytest.mark.parametrize("jump", [False, True])
+@pytest.mark.parametrize("direction", [0, 1])
+def test_velocities_of_every_magnitude(fast, direction, jump):
+    L, R, _ = _tails(40000, 3, jump)
+    took, f, i = _both(fast, L, R, direction, 0, np.full(len(L), -1.0))
+    assert took == len(L) and np.array_equal(f, i)
+
+
+@pytest.mark.parametrize("direction", [0, 1])
+def test_transversal_flux(fast, direction):
+    for L, R in (cases.interface_pairs(20000, 7 + direction), _tails(20000, 8, True)[:2]):
+        L, R = np.ascontiguousarray(L), np.ascontiguousarray(R)
+        f, i = np.zeros((len(L), 9)), np.zeros((len(L), 9))
+        took = fast.fh_transversal_many(_dp(L), _dp(R), len(L), C.c_double(1e-3), C.c_double(1e-9), direction, _dp(f), _dp(i))
         on = ~np.isnan(f[:, 0])
-        assert took > 0.9 * n and np.array_equal(f[on], i[on])
+        assert took == on.sum() > 0.95 * len(L) and np.array_equal(f[on], i[on])
 
 
-@pytest.mark.parametrize("at, value", [(3, 1e-40), (6, 1e40), (4, 1e40), (8, np.inf), (10, 1e200), (3, np.nan)])
+@pytest.mark.parametrize("direction", [0, 1])
+def test_two_fluid_flux(fast, direction):
+    """Pure, mixed and nearly pure sides, fractions' tails among them."""
+    for k, (L, R) in enumerate((cases.interface_pairs(20000, 17), _tails(20000, 18, True)[:2])):
+        L, R = np.ascontiguousarray(L), np.ascontiguousarray(R)
+        n, rng = len(L), np.random.default_rng(k)
+        FA = np.zeros((n, 4))
+        for q in (0, 2):
+            kind = rng.integers(0, 5, n)
+            FA[:, q] = np.choose(kind, [np.zeros(n), np.ones(n), rng.random(n), 10.0 ** rng.uniform(-320, 0, n),
+                                        1.0 - 10.0 ** rng.uniform(-17, 0, n)])
+            FA[:, q + 1] = rng.choice([0.0, 1.0, 1e-200, 1e-305], n) * rng.uniform(-1, 1, n)
+        f, i = np.zeros((n, 12)), np.zeros((n, 12))
+        took = fast.fh_two_fluid_many(_dp(L), _dp(R), _dp(FA), n, C.c_double(1e-3), C.c_double(1e-9), direction,
+                                      C.c_double(1.4), C.c_double(1.67), _dp(f), _dp(i))
+        on = ~np.isnan(f[:, 0])
+        # (interface_pairs are drawn for one gas: with two, a few more open a vacuum)
+        assert took == on.sum() > 0.9 * n and np.array_equal(f[on], i[on])
+
+
+@pytest.mark.parametrize("gamma", [1.4, 1.67, 3.0])
+def test_1d_solver(fast, gamma):
+    for L, R in (cases.interface_pairs(20000, 27, gamma), _tails(20000, 28, True)[:2]):
+        L, R = np.ascontiguousarray(L), np.ascontiguousarray(R)
+        f, i = np.zeros((len(L), 6)), np.zeros((len(L), 6))
+        took = fast.fh_edir_many(_dp(L), _dp(R), len(L), C.c_double(1e-9), _dp(f), _dp(i))
+        assert took > 0.9 * len(L) and np.array_equal(f, i, equal_nan=True)
+
+
+@pytest.mark.parametrize("at, value", [(3, 1e-40), (6, 1e40), (4, 1e40), (8, np.inf), (10, 1e200)]
+                         + [(k, np.nan) for k in range(3, 11)])
 def test_out_of_range_is_left_to_the_ieee_solver(fast, at, value):
     L, R = cases.interface_pairs(8, 5)
     for A in (L, R):
         B = [L.copy(), R.copy()]
         B[0 if A is L else 1][:, at] = value
-        took, f, _ = _both(fast, B[0], B[1], 0, 0, np.full(8, -1.0))
-        assert took == 0 and np.isnan(f).all()
+        for direction in (0, 1):
+            took, f, _ = _both(fast, B[0], B[1], direction, 0, np.full(8, -1.0))
+            assert took == 0 and np.isnan(f).all()
 
 
 @pytest.mark.parametrize("eps", [1e-9, 1e-12, 0.3, 1e-3, 7.3e-200, 1e-170, 1e160])
