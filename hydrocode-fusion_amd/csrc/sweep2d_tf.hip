@@ -68,12 +68,14 @@ struct LineTF {
     __device__ void limited_sp(const double vm[NQ], const double v0[NQ], const double vp[NQ], const double sp[NQ],
                                double s[NQ]) const
     {
+        double d_L[NQ], d_R[NQ], s_L[NQ], s_R[NQ];
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            const double s_L = div_by(v0[q] - vm[q], a.div_h);
-            const double s_R = div_by(vp[q] - v0[q], a.div_h);
-            s[q] = a.limiter3 ? minmod3(a.alpha * s_L, a.alpha * s_R, sp[q]) : minmod2(s_L, s_R);
-        }
+        for (int q = 0; q < NQ; ++q) { d_L[q] = v0[q] - vm[q]; d_R[q] = vp[q] - v0[q]; }
+        quot4<NQ>(d_L, a.div_h, s_L);
+        quot4<NQ>(d_R, a.div_h, s_R);
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+            s[q] = a.limiter3 ? minmod3(a.alpha * s_L[q], a.alpha * s_R[q], sp[q]) : minmod2(s_L[q], s_R[q]);
     }
     __device__ void limited_at(int k, double s[NQ]) const
     {
@@ -102,6 +104,18 @@ struct LineTF {
             break;
         }
     }
+    // ghost slopes next to a boundary cell whose own slopes `near` the caller has: the rules of
+    // ghost_slope, which only the periodic one needs other cells for
+    __device__ void ghost_slope_near(bool lo, const double near[NQ], double s[NQ]) const
+    {
+        if (a.bc == BC_PERIODIC) {
+            limited_at(lo ? cnt - 1 : 0, s);
+            return;
+        }
+        const bool keep = a.bc == BC_REFLECT || (a.bc == BC_REFLECT_FREE && lo);
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) s[q] = keep && q == NV ? near[q] : 0.0;
+    }
     // update of cell k: the single-fluid update with the mixture's gamma, and
     // the volume fraction in quasi-conservative form
     __device__ void update(int k, const double w[NQ], double e, const double Fl[4], const double Fr[4],
@@ -113,22 +127,26 @@ struct LineTF {
         const double mom_y = w[0] * w[2] - nu * (Fr[2] - Fl[2]);
         const double ene = w[0] * e - nu * (Fr[3] - Fl[3]);
         const double rho = w[0] + -nu * (Fr[0] - Fl[0]);
-        const double u = mom_x / rho;
-        const double v = mom_y / rho;
+        double u, v, e_new;
+        quot3(mom_x, mom_y, ene, rho, u, v, e_new);
         double fa = w[4] - nu * ((Zr[0] - Zl[0]) - w[4] * (Zr[1] - Zl[1]));
         fa = fmin(fmax(fa, 0.0), 1.0);
         const double X = ene - 0.5 * mom_x * u - 0.5 * mom_y * v;
         double p;
         if (fa == 1.0) p = X * a.two.a.gm1();
         else if (fa == 0.0) p = X * a.two.b.gm1();
+        else if (two_in_range(a.two) && fabs(X) >= 0x1p-300 && fabs(X) <= 0x1p300) p = div_1(X, mix_inv_gm1_q(fa, a.two));
         else p = X / (fa / (a.two.a.g - 1.0) + (1.0 - fa) / (a.two.b.g - 1.0));
         double *f = a.st_o + o;
         const size_t P = a.plane;
-        f[0] = rho; f[P] = u; f[2 * P] = v; f[4 * P] = ene / rho; f[3 * P] = p; a.fa_o[o] = fa;
+        f[0] = rho; f[P] = u; f[2 * P] = v; f[4 * P] = e_new; f[3 * P] = p; a.fa_o[o] = fa;
         if (p < a.eps || rho < a.eps) atomicOr(&a.status->flags, 1u);
+        const double dI[NQ] = {Ir[0] - Il[0], Ir[1] - Il[1], Ir[2] - Il[2], Ir[3] - Il[3], Zr[2] - Zl[2]};
+        double sn[NQ];
+        quot4<NQ>(dI, a.div_h, sn);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) a.s_o[o + q * P] = div_by(Ir[q] - Il[q], a.div_h);
-        a.sa_o[o] = div_by(Zr[2] - Zl[2], a.div_h);
+        for (int q = 0; q < 4; ++q) a.s_o[o + q * P] = sn[q];
+        a.sa_o[o] = sn[4];
     }
 };
 
@@ -146,19 +164,55 @@ __device__ __forceinline__ void recon_tf(const double w[NQ], const double s[NQ],
     d_fa = s[4];
 }
 
+// Face f of grid line `line` (between cells f - 1 and f) with the IEEE solver,
+// from the cells in memory: what the fast solver leaves (grp_fast.hpp).
+// FIZ: flux, values at t + tau, the fraction's three.
+template <int DIR, bool CONV>
+__device__ __attribute__((noinline)) int redo_face_tf(const SweepArgs *ap, int line, int f, double p_guess, double *FIZ)
+{
+    const SweepArgs &a = *ap;
+    const LineTF<DIR> L(a, line);
+    double wl[NQ], wr[NQ], sl[NQ], sr[NQ], FA[4];
+    L.value(f - 1, wl);
+    L.value(f, wr);
+    if (f > 0) L.limited_at(f - 1, sl); else L.ghost_slope(true, sl);
+    if (f < L.cnt) L.limited_at(f, sr); else L.ghost_slope(false, sr);
+    Side SL, SR;
+    recon_tf(wl, sl, a.hh, true, SL, FA[0], FA[1]);
+    recon_tf(wr, sr, a.hh, false, SR, FA[2], FA[3]);
+    return grp_2d_flux_tf<DIR, CONV>(SL, SR, a.two, FA, a.tau, a.eps, FIZ, FIZ + 4, FIZ + 8, a.tol, p_guess);
+}
+
 template <int DIR, int NM>
 __device__ __forceinline__ void solve_interface_tf(const SweepArgs &a, const double wl[NQ], const double sl[NQ],
-                                                   const double wr[NQ], const double sr[NQ],
-                                                   unsigned long long loop_index, double F[4], double I[4],
-                                                   double Z[3], double p_guess = -1.0)
+                                                   const double wr[NQ], const double sr[NQ], int line, int f, double F[4],
+                                                   double I[4], double Z[3], double p_guess = -1.0)
 {
     Side SL, SR;
     double FA[4];
     recon_tf(wl, sl, a.hh, true, SL, FA[0], FA[1]);
     recon_tf(wr, sr, a.hh, false, SR, FA[2], FA[3]);
-    int code = ifvar_bad(SL, SR, a.eps) ? 1 : 0;
-    if (grp_2d_flux_tf<DIR, NM != NM_REF>(SL, SR, a.two, FA, a.tau, a.eps, F, I, Z, a.tol, p_guess)) code = 2;
-    if (code) atomicMax(&a.status->fail_key, ((loop_index << 2) | (unsigned long long)code) + 1ull);
+    int code = ifvar_bad(SL, SR, a.eps) ? 1 : 0, bad = 0;
+    const bool done = flux_two_fluid_q<DIR, NM != NM_REF>(SL, SR, a.two, FA, a.near2, a.tau, a.eps, F, I, Z, a.tol,
+                                                          p_guess, &bad);
+    if (__builtin_expect(__any(!done), 0)) {
+        if (!done) {
+            const SweepArgs ar = reload_args<SweepArgs>();
+            double o[11];
+            bad = redo_face_tf<DIR, NM != NM_REF>(&ar, line, f, p_guess, o);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) { F[q] = o[q]; I[q] = o[4 + q]; }
+#pragma unroll
+            for (int q = 0; q < 3; ++q) Z[q] = o[8 + q];
+        }
+    }
+    if (bad) code = 2;
+    if (code) {
+        const SweepArgs ar = reload_args<SweepArgs>();
+        const unsigned long long index = (unsigned long long)line * (unsigned long long)((DIR == 0 ? ar.m : ar.n) + 1)
+                                         + (unsigned long long)f;
+        atomicMax(&ar.status->fail_key, ((index << 2) | (unsigned long long)code) + 1ull);
+    }
 }
 
 // learned starting pressure for the interface (wl, sl | wr, sr), every lane of
@@ -173,12 +227,11 @@ __device__ __forceinline__ double interface_guess_tf(const SweepArgs &a, bool ac
     recon_tf(wl, sl, a.hh, true, SL, aL, daL);
     recon_tf(wr, sr, a.hh, false, SR, aR, daR);
     const double uL = DIR == 0 ? SL.u : SL.v, uR = DIR == 0 ? SR.u : SR.v;
-    const double dist = sqrt((SL.rho - SR.rho) * (SL.rho - SR.rho) + (uL - uR) * (uL - uR)
-                             + (SL.p - SR.p) * (SL.p - SR.p));
+    const double dist2 = (SL.rho - SR.rho) * (SL.rho - SR.rho) + (uL - uR) * (uL - uR) + (SL.p - SR.p) * (SL.p - SR.p);
     // Newton runs only past the acoustic shortcut and the equal-state exit of the exact solver
-    const bool want = active && !(dist < a.eps) && !(fabs(uL - uR) < a.tol && fabs(SL.p - SR.p) < a.tol);
-    const double gL = aL == 1.0 ? a.two.a.g : (aL == 0.0 ? a.two.b.g : mix_gamma(aL, a.two));
-    const double gR = aR == 1.0 ? a.two.a.g : (aR == 0.0 ? a.two.b.g : mix_gamma(aR, a.two));
+    const bool want = active && !(dist2 < a.near2) && !(fabs(uL - uR) < a.tol && fabs(SL.p - SR.p) < a.tol);
+    const double gL = aL == 1.0 ? a.two.a.g : (aL == 0.0 ? a.two.b.g : mix_gamma_q(aL, a.two));
+    const double gR = aR == 1.0 ? a.two.a.g : (aR == 0.0 ? a.two.b.g : mix_gamma_q(aR, a.two));
     return learned_guess_wave(a.mlp, want, SL.rho, uL, SL.p, SR.rho, uR, SR.p, gL, gR, lds);
 }
 
@@ -246,21 +299,23 @@ __global__ void __launch_bounds__(64 * W, (W + 3) / 4) sweep_x_tf_kernel(SweepAr
         for (int q = 0; q < NQ; ++q) vr[q] = xa[w + 1][q][lane];
 
     double s[NQ] = {0.0, 0.0, 0.0, 0.0, 0.0}, sr[NQ] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    if (col) {
-        if (own) L.limited_sp(vl, v, vr, sp, s);
-        else if (c == -1) L.ghost_slope(true, s);
-        else if (c == m) L.ghost_slope(false, s);
-        if (w == W - 1) {
-            if (next_own) L.limited_sp(v, vr, vrr, sp1, sr);
-            else if (c + 1 == m) L.ghost_slope(false, sr);
-        }
-    }
+    if (own) L.limited_sp(vl, v, vr, sp, s);
+    if (next_own) L.limited_sp(v, vr, vrr, sp1, sr);
 #pragma unroll
     for (int q = 0; q < NQ; ++q) xb[w][q][lane] = s[q];
     __syncthreads();
     if (w < W - 1)
 #pragma unroll
         for (int q = 0; q < NQ; ++q) sr[q] = xb[w + 1][q][lane];
+    // the ghosts' slopes from the boundary cells'
+    if (col && (c == -1 || c + 1 == m)) {
+        double g[NQ];
+        L.ghost_slope_near(c == -1, c == -1 ? sr : s, g);
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            if (c == -1) s[q] = g[q]; else sr[q] = g[q];
+        }
+    }
 
     double F[4] = {0.0, 0.0, 0.0, 0.0}, I[4] = {0.0, 0.0, 0.0, 0.0}, Z[3] = {0.0, 0.0, 0.0};
     const int f = c + 1;
@@ -268,8 +323,7 @@ __global__ void __launch_bounds__(64 * W, (W + 3) / 4) sweep_x_tf_kernel(SweepAr
     if constexpr (LEARNED)   // xf[w] is not written before the solve: it holds the network inputs
         pg = interface_guess_tf<0>(a, col && f <= m, v, s, vr, sr, (uint32_t *)&xf[w][0][0]);
     if (col && f <= m)
-        solve_interface_tf<0, NM>(a, v, s, vr, sr, (unsigned long long)i * (unsigned long long)(m + 1) + (unsigned long long)f,
-                              F, I, Z, pg);
+        solve_interface_tf<0, NM>(a, v, s, vr, sr, i, f, F, I, Z, pg);
 #pragma unroll
     for (int q = 0; q < 4; ++q) { xf[w][q][lane] = F[q]; xi[w][q][lane] = I[q]; }
 #pragma unroll
@@ -343,14 +397,18 @@ __global__ void __launch_bounds__(256, 3) sweep_y_tf_kernel(SweepArgs a, int chu
 
     double s[NQ] = {0.0, 0.0, 0.0, 0.0, 0.0};
     if (own) L.limited_sp(wl, w, wr, sp, s);
-    else if (rowv && c == -1) L.ghost_slope(true, s);
-    else if (rowv && c == n) L.ghost_slope(false, s);
     double sr[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) sr[q] = __shfl_down(s[q], 1);
-    if (rowv && k == G - 1) {
-        if (last_own) L.limited_sp(w, wr, wrr, sp1, sr);
-        else if (c + 1 == n) L.ghost_slope(false, sr);
+    if (last_own) L.limited_sp(w, wr, wrr, sp1, sr);
+    // the ghosts' slopes from the boundary cells'
+    if (rowv && (c == -1 || c + 1 == n)) {
+        double g[NQ];
+        L.ghost_slope_near(c == -1, c == -1 ? sr : s, g);
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            if (c == -1) s[q] = g[q]; else sr[q] = g[q];
+        }
     }
 
     double F[4] = {0.0, 0.0, 0.0, 0.0}, I[4] = {0.0, 0.0, 0.0, 0.0}, Z[3] = {0.0, 0.0, 0.0};
@@ -359,8 +417,7 @@ __global__ void __launch_bounds__(256, 3) sweep_y_tf_kernel(SweepArgs a, int chu
     double pg = -1.0;
     if constexpr (LEARNED) pg = interface_guess_tf<1>(a, face, w, s, wr, sr, mlp_lds[(threadIdx.x >> 6) & 3]);
     if (face)
-        solve_interface_tf<1, NM>(a, w, s, wr, sr, (unsigned long long)j * (unsigned long long)(n + 1) + (unsigned long long)f,
-                              F, I, Z, pg);
+        solve_interface_tf<1, NM>(a, w, s, wr, sr, j, f, F, I, Z, pg);
     double Fl[4], Il[4], Zl[3];
 #pragma unroll
     for (int q = 0; q < 4; ++q) { Fl[q] = __shfl_up(F[q], 1); Il[q] = __shfl_up(I[q], 1); }
