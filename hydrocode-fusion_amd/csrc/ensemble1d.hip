@@ -35,7 +35,7 @@
 #include <vector>
 
 #include "../../include/hydrocode_grp.h"
-#include "grp1d_device.hpp"
+#include "grp1d_fast.hpp"
 
 using namespace hgrp;
 
@@ -62,6 +62,7 @@ struct Inst {
     unsigned uflags;              // FLAG_STOP raised by the update of the current step
     int paused;                   // time_c reached t_pause at the start of a step: waits for the host
     double h, time_c, tau;
+    RecipDiv div_h;               // division by h
     double t_pause;               // plot time the host waits for (INFINITY: none)
     unsigned long long hsm_bits;  // min over interfaces of h/S, as bits (positive doubles order like them)
     double b0[6];                 // BC -1 ghosts from the initial data: rho u p left, rho u p right
@@ -69,6 +70,7 @@ struct Inst {
 
 struct Params {
     double t_all, eps, gamma, cfl, tau_fixed, alpha;
+    double near2;                 // the acoustic switch dist < eps on dist^2 (near_threshold)
     int n_max;
     Gas gas;
 };
@@ -104,12 +106,14 @@ __device__ __forceinline__ void cell_value(const Inst &I, const double *rho, con
 __device__ __forceinline__ void limit3(const Inst &I, const Params &P, const double *const s_prev[3], int c,
                                        const double vm[3], const double v0[3], const double vp[3], double s[3])
 {
-    const double h = I.h;
-    for (int q = 0; q < 3; ++q) {
-        const double s_L = (v0[q] - vm[q]) / h;
-        const double s_R = (vp[q] - v0[q]) / h;
-        s[q] = I.found ? minmod3(P.alpha * s_L, P.alpha * s_R, s_prev[q][(size_t)I.coff + c]) : minmod2(s_L, s_R);
-    }
+    const double d_L[3] = {v0[0] - vm[0], v0[1] - vm[1], v0[2] - vm[2]};
+    const double d_R[3] = {vp[0] - v0[0], vp[1] - v0[1], vp[2] - v0[2]};
+    double s_L[3], s_R[3];
+    quot4<3>(d_L, I.div_h, s_L);
+    quot4<3>(d_R, I.div_h, s_R);
+    for (int q = 0; q < 3; ++q)
+        s[q] = I.found ? minmod3(P.alpha * s_L[q], P.alpha * s_R[q], s_prev[q][(size_t)I.coff + c])
+                       : minmod2(s_L[q], s_R[q]);
 }
 
 // the same, loading the three values
@@ -138,6 +142,54 @@ __device__ __forceinline__ void ghost_slope(const Inst &I, const Params &P, cons
         limited(I, P, rho, u, p, s_prev, 0, t);
         s[1] = t[1];
     }
+}
+
+// the same for the ghost next to a boundary cell whose own slopes `near` the caller has
+__device__ __forceinline__ void ghost_slope_near(const Inst &I, const Params &P, const double *rho, const double *u,
+                                                 const double *p, const double *const s_prev[3], bool lo,
+                                                 const double near[3], double s[3])
+{
+    if (I.bc == -7) {
+        limited(I, P, rho, u, p, s_prev, lo ? I.m - 1 : 0, s);
+        return;
+    }
+    s[0] = s[2] = 0.0;
+    s[1] = I.bc == -2 || (I.bc == -24 && lo) ? near[1] : 0.0;
+}
+
+// sides of an interface between cells with values wl, wr and slopes sl, sr
+__device__ __forceinline__ void sides(double h, bool last, const double wl[3], const double sl[3], const double wr[3],
+                                      const double sr[3], Side1 &L, Side1 &R)
+{
+    L.rho = wl[0] + 0.5 * h * sl[0]; L.u = wl[1] + 0.5 * h * sl[1]; L.p = wl[2] + 0.5 * h * sl[2];
+    if (!last) {
+        R.rho = wr[0] - 0.5 * h * sr[0]; R.u = wr[1] - 0.5 * h * sr[1]; R.p = wr[2] - 0.5 * h * sr[2];
+    } else {   // the reference reconstructs the right ghost with +h/2 (grp_solver_EUL_source.c:154-158)
+        R.rho = wr[0] + 0.5 * h * sr[0]; R.u = wr[1] + 0.5 * h * sr[1]; R.p = wr[2] + 0.5 * h * sr[2];
+    }
+    L.s_rho = sl[0]; L.s_u = sl[1]; L.s_p = sl[2];
+    R.s_rho = sr[0]; R.s_u = sr[1]; R.s_p = sr[2];
+}
+
+// Interface j of instance I with the IEEE solver, from the cells in memory: what
+// the fast solver leaves (grp1d_fast.hpp).  DU: D[3], U[3].
+__device__ __attribute__((noinline)) void redo_iface(const Inst *Ip, double eps, double alpha, double gamma,
+                                                     const double *rho, const double *u, const double *p,
+                                                     const double *s_rho, const double *s_u, const double *s_p, int j,
+                                                     double *DU)
+{
+    const Inst &I = *Ip;
+    const double *const sp[3] = {s_rho, s_u, s_p};
+    Params P = {};
+    P.alpha = alpha;
+    double wl[3], wr[3], sl[3], sr[3];
+    cell_value(I, rho, u, p, j - 1, wl);
+    cell_value(I, rho, u, p, j, wr);
+    if (j > 0) limited(I, P, rho, u, p, sp, j - 1, sl); else ghost_slope(I, P, rho, u, p, sp, true, sl);
+    if (j < I.m) limited(I, P, rho, u, p, sp, j, sr); else ghost_slope(I, P, rho, u, p, sp, false, sr);
+    Side1 L, R;
+    sides(I.h, j == I.m, wl, sl, wr, sr, L, R);
+    grp_edir(DU, DU + 3, L, R, make_gas(gamma), eps);
 }
 
 struct Tables {
@@ -183,34 +235,43 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) if
     if (t == 0 && interior) cell_value(I, rho, u, p, c - 1, vm);
     if (t == 63 && interior) cell_value(I, rho, u, p, c + 1, wr);
     if (interior) limit3(I, P, sp, c, vm, wl, wr, sl);
-    else if (c == -1) ghost_slope(I, P, rho, u, p, sp, true, sl);
-    else if (c == m) ghost_slope(I, P, rho, u, p, sp, false, sl);
     for (int q = 0; q < 3; ++q) sr[q] = __shfl_down(sl[q], 1);
     if (t == 63 && j < m) limited(I, P, rho, u, p, sp, j, sr);
-    else if (t == 63 && j == m) ghost_slope(I, P, rho, u, p, sp, false, sr);
+    // the ghosts' slopes from the boundary cells'
+    if (j == 0 || j == m) {
+        double g[3];
+        ghost_slope_near(I, P, rho, u, p, sp, j == 0, j == 0 ? sr : sl, g);
+        for (int q = 0; q < 3; ++q) {
+            if (j == 0) sl[q] = g[q]; else sr[q] = g[q];
+        }
+    }
     double hs = INFINITY;
     if (j <= m) {
         const double h = I.h, gamma = P.gamma;
         Side1 L, R;
-        L.rho = wl[0] + 0.5 * h * sl[0]; L.u = wl[1] + 0.5 * h * sl[1]; L.p = wl[2] + 0.5 * h * sl[2];
-        if (j < m) {
-            R.rho = wr[0] - 0.5 * h * sr[0]; R.u = wr[1] - 0.5 * h * sr[1]; R.p = wr[2] - 0.5 * h * sr[2];
-        } else {   // the reference reconstructs the right ghost with +h/2 (grp_solver_EUL_source.c:154-158)
-            R.rho = wr[0] + 0.5 * h * sr[0]; R.u = wr[1] + 0.5 * h * sr[1]; R.p = wr[2] + 0.5 * h * sr[2];
-        }
-        L.s_rho = sl[0]; L.s_u = sl[1]; L.s_p = sl[2];
-        R.s_rho = sr[0]; R.s_u = sr[1]; R.s_p = sr[2];
-        const double c_L = sqrt(gamma * L.p / L.rho);
-        const double c_R = sqrt(gamma * R.p / R.rho);
-        hs = fmin(hs, h / (fabs(L.u) + fabs(c_L)));
-        hs = fmin(hs, h / (fabs(R.u) + fabs(c_R)));
+        sides(h, j == m, wl, sl, wr, sr, L, R);
+        // in range: the steps' own arithmetic (grp1d_fast.hpp); c_L and c_R serve the solver too
+        const bool in = gas_in_range(P.gas) && sides1_in_range(L, R) && h >= 0x1p-100 && h <= 0x1p100;
+        const Rcp rL = rcp_of(L.rho), rR = rcp_of(R.rho);
+        const double c_L = in ? sqrt_q(div_q(gamma * L.p, rL)) : sqrt(gamma * L.p / L.rho);
+        const double c_R = in ? sqrt_q(div_q(gamma * R.p, rR)) : sqrt(gamma * R.p / R.rho);
+        // the smaller of the two quotients is the one by the larger speed
+        const double speed = fmax(fabs(L.u) + fabs(c_L), fabs(R.u) + fabs(c_R));
+        hs = fmin(hs, in ? div_1(h, speed) : h / speed);
         const double eps = P.eps;
         if (L.p < eps || R.p < eps || L.rho < eps || R.rho < eps || !isfinite(L.s_p) || !isfinite(R.s_p) ||
             !isfinite(L.s_u) || !isfinite(R.s_u) || !isfinite(L.s_rho) || !isfinite(R.s_rho)) {
             flag(Ip, FLAG_ABORT);
         } else {
             double D[3], U[3];
-            grp_edir(D, U, L, R, P.gas, eps);
+            const bool done = in && grp_edir_q(D, U, L, R, rL, rR, c_L, c_R, P.gas, P.near2, eps);
+            if (__builtin_expect(__any(!done), 0)) {
+                if (!done) {
+                    double DU[6];
+                    redo_iface(Ip, eps, P.alpha, gamma, rho, u, p, s_rho, s_u, s_p, j, DU);
+                    for (int q = 0; q < 3; ++q) { D[q] = DU[q]; U[q] = DU[3 + q]; }
+                }
+            }
             if (U[2] < eps || U[0] < eps || !isfinite(U[1]) || !isfinite(U[2]) || !isfinite(U[0]) ||
                 !isfinite(D[1]) || !isfinite(D[2]) || !isfinite(D[0]))
                 flag(Ip, FLAG_STOP);
@@ -243,7 +304,7 @@ __device__ __forceinline__ double step_tau(const Inst &I, const Params &P, bool 
 }
 
 __device__ __forceinline__ void iface_flux(const double *mid, const double *dire, size_t n_if_all, size_t g,
-                                           double tau, double gamma, double F[3], double In[3])
+                                           double tau, double g_gm1, double F[3], double In[3])
 {
     double R = mid[g], U = mid[n_if_all + g], Pp = mid[2 * n_if_all + g];
     const double Rt = dire[g], Ut = dire[n_if_all + g], Pt = dire[2 * n_if_all + g];
@@ -252,7 +313,7 @@ __device__ __forceinline__ void iface_flux(const double *mid, const double *dire
     Pp += 0.5 * tau * Pt;
     F[0] = R * U;
     F[1] = F[0] * U + Pp;
-    F[2] = (gamma / (gamma - 1.0)) * Pp + 0.5 * F[0] * U;
+    F[2] = g_gm1 * Pp + 0.5 * F[0] * U;
     F[2] = F[2] * U;
     In[0] = R + 0.5 * tau * Rt;
     In[1] = U + 0.5 * tau * Ut;
@@ -279,21 +340,22 @@ __global__ void __launch_bounds__(BS) update_kernel(Tables T, int n_w, Inst *ins
     const double nu = tau / h;
     const size_t g = (size_t)I.ioff + j;
     double Fl[3], Il[3], Fr[3], Ir[3];
-    iface_flux(mid, dire, n_if_all, g, tau, gamma, Fl, Il);
-    iface_flux(mid, dire, n_if_all, g + 1, tau, gamma, Fr, Ir);
+    iface_flux(mid, dire, n_if_all, g, tau, P.gas.g_gm1, Fl, Il);
+    iface_flux(mid, dire, n_if_all, g + 1, tau, P.gas.g_gm1, Fr, Ir);
     const size_t o = (size_t)I.coff + j;
     const double r0 = rho[o], u0 = u[o], e0 = e[o];
     const double Mom = r0 * u0 - nu * (Fr[1] - Fl[1]);
     const double Ene = r0 * e0 - nu * (Fr[2] - Fl[2]);
     const double r1 = r0 - nu * (Fr[0] - Fl[0]);
-    const double u1 = Mom / r1;
-    const double e1 = Ene / r1;
+    double u1, e1, u1_;
+    quot3(Mom, Mom, Ene, r1, u1, u1_, e1);
     const double p1 = (Ene - 0.5 * Mom * u1) * (gamma - 1.0);
     rho[o] = r1; u[o] = u1; e[o] = e1; p[o] = p1;
     if (p1 < P.eps || r1 < P.eps) atomicOr(&I.uflags, FLAG_STOP);
-    s_u[o] = (Ir[1] - Il[1]) / h;
-    s_p[o] = (Ir[2] - Il[2]) / h;
-    s_rho[o] = (Ir[0] - Il[0]) / h;
+    const double dI[3] = {Ir[0] - Il[0], Ir[1] - Il[1], Ir[2] - Il[2]};
+    double sn[3];
+    quot4<3>(dI, I.div_h, sn);
+    s_rho[o] = sn[0]; s_u[o] = sn[1]; s_p[o] = sn[2];
 }
 
 // end of a step (grp_solver_EUL_source.c:218-233, 279-283): the step's tau
@@ -497,11 +559,13 @@ extern "C" int hgrp1d_create(hgrp1d **out, int n_inst, const int *cells, const d
     c->P.tau_fixed = config[16];
     c->P.alpha = config[41];
     c->P.gas = make_gas(config[6]);
+    c->P.near2 = near_threshold(c->P.eps);
     c->host_inst.resize(n_inst);
     for (int i = 0; i < n_inst; ++i) {
         Inst &I = c->host_inst[i];
         memset(&I, 0, sizeof I);
         I.coff = c->coff[i]; I.ioff = c->ioff[i]; I.m = cells[i]; I.bc = bc; I.h = h[i];
+        I.div_h = recip_div(h[i]);
     }
     const size_t nb = 7 * nc + 6 * ni + 4 * nc;
     hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
