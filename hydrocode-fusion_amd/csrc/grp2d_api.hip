@@ -21,6 +21,7 @@
 #include "grp_device.hpp"
 #include "sweep2d.hpp"
 #include "unsplit2d.hpp"
+#include "layout2d.hpp"
 
 namespace hgrp {
 hipError_t launch_sweep_x(const SweepArgs &a, int variant, hipStream_t st);
@@ -156,13 +157,6 @@ extern "C" int hgrp2d_destroy(hgrp2d *c)
     return 0;
 }
 
-static int copy_rows_in(hgrp2d *c, double *dst, const double *src)
-{
-    HCHECK(hipMemcpy2DAsync(dst, (size_t)c->ld * 8, src, (size_t)c->n * 8, (size_t)c->n * 8, (size_t)c->m,
-                            hipMemcpyHostToDevice, c->stream));
-    return 0;
-}
-
 extern "C" int hgrp2d_upload(hgrp2d *c, const double *rho, const double *u, const double *v,
                              const double *p, const double *e)
 {
@@ -171,37 +165,8 @@ extern "C" int hgrp2d_upload(hgrp2d *c, const double *rho, const double *u, cons
     c->two_fluid = false;                 // a new state needs its volume fraction again
     const int m = c->m, n = c->n;
     const double gamma = c->cfg[6];
-    const size_t mn = (size_t)m * n;
-    std::vector<double> E;
-    if (!e) {
-        E.resize(mn);
-        for (size_t k = 0; k < mn; ++k) {
-            double t = 0.5 * u[k] * u[k] + p[k] / (gamma - 1.0) / rho[k];
-            t += 0.5 * v[k] * v[k];
-            E[k] = t;
-        }
-        e = E.data();
-    }
     const double *src[5] = {rho, u, v, p, e};
-    for (int f = 0; f < 5; ++f) {
-        int rc = copy_rows_in(c, c->st[0][f], src[f]);
-        if (rc) return rc;
-    }
-    // BC -1 ghosts come from the initial data (bound_cond_slope_limiter_x.c:37-46)
-    std::vector<double> b((size_t)2 * n * 4 + (size_t)2 * m * 4);
-    double *xl = b.data(), *xh = xl + (size_t)n * 4, *yl = xh + (size_t)n * 4, *yh = yl + (size_t)m * 4;
-    const double *q4[4] = {rho, u, v, p};
-    for (int i = 0; i < n; ++i)
-        for (int q = 0; q < 4; ++q) {
-            xl[(size_t)i * 4 + q] = q4[q][i];
-            xh[(size_t)i * 4 + q] = q4[q][(size_t)(m - 1) * n + i];
-        }
-    for (int j = 0; j < m; ++j)
-        for (int q = 0; q < 4; ++q) {
-            yl[(size_t)j * 4 + q] = q4[q][(size_t)j * n];
-            yh[(size_t)j * 4 + q] = q4[q][(size_t)j * n + n - 1];
-        }
-    HCHECK(hipMemcpyAsync(c->bnd[0], b.data(), b.size() * 8, hipMemcpyHostToDevice, c->stream));
+    HCHECK(upload_state(src, c->st[1][0], c->st[0][0], c->bnd[0], (size_t)m * c->ld, m, n, c->ld, gamma, c->stream));
     // frozen CFL reduction over the initial data (grp_solver_2D_split_EUL_source.c:183-191)
     const unsigned long long inf_bits = 0x7ff0000000000000ull;
     HCHECK(hipMemcpyAsync(c->cfl_bits, &inf_bits, 8, hipMemcpyHostToDevice, c->stream));
@@ -221,11 +186,7 @@ extern "C" int hgrp2d_download(hgrp2d *c, double *rho, double *u, double *v, dou
 {
     if (!c) return ARG_ERROR - 1;
     double *dst[5] = {rho, u, v, p, e};
-    for (int f = 0; f < 5; ++f) {
-        if (!dst[f]) continue;
-        HCHECK(hipMemcpy2DAsync(dst[f], (size_t)c->n * 8, c->st[c->cs][f], (size_t)c->ld * 8, (size_t)c->n * 8,
-                                (size_t)c->m, hipMemcpyDeviceToHost, c->stream));
-    }
+    HCHECK(download_planes(dst, 5, c->st[c->cs][0], c->st[1 - c->cs][0], (size_t)c->m * c->ld, c->m, c->n, c->ld, c->stream));
     HCHECK(hipStreamSynchronize(c->stream));
     return 0;
 }
@@ -287,8 +248,7 @@ extern "C" int hgrp2d_set_fluids(hgrp2d *c, double gamma_b, const double *frac_a
         }
     }
     HCHECK(hipMemsetAsync(c->tf_block, 0, 6 * cells * sizeof(double), c->stream));
-    HCHECK(hipMemcpy2DAsync(c->fa[c->cs], (size_t)c->ld * 8, frac_a, (size_t)c->n * 8, (size_t)c->n * 8,
-                            (size_t)c->m, hipMemcpyHostToDevice, c->stream));
+    HCHECK(upload_plane(frac_a, c->fa[1 - c->cs], c->fa[c->cs], c->m, c->n, c->ld, c->stream));
     c->two.a = make_gas(c->cfg[6]);
     c->two.b = make_gas(gamma_b);
     HCHECK(launch_energy_tf(c->st[c->cs][0], c->st[c->cs][1], c->st[c->cs][2], c->st[c->cs][3], c->fa[c->cs],
@@ -310,8 +270,7 @@ extern "C" int hgrp2d_set_fluids(hgrp2d *c, double gamma_b, const double *frac_a
 extern "C" int hgrp2d_download_fraction(hgrp2d *c, double *frac_a)
 {
     if (!c || !frac_a || !c->two_fluid) return ARG_ERROR - 1;
-    HCHECK(hipMemcpy2DAsync(frac_a, (size_t)c->n * 8, c->fa[c->cs], (size_t)c->ld * 8, (size_t)c->n * 8, (size_t)c->m,
-                            hipMemcpyDeviceToHost, c->stream));
+    HCHECK(download_planes(&frac_a, 1, c->fa[c->cs], c->fa[1 - c->cs], 0, c->m, c->n, c->ld, c->stream));
     HCHECK(hipStreamSynchronize(c->stream));
     return 0;
 }

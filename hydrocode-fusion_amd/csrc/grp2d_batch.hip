@@ -31,6 +31,7 @@
 #include "grp_device.hpp"
 #include "sweep2d.hpp"
 #include "sweep2d_body.hpp"
+#include "layout2d.hpp"
 
 namespace hgrp {
 
@@ -455,43 +456,15 @@ extern "C" int hgrp2db_upload(hgrp2db *c, const double *rho, const double *u, co
     const unsigned long long inf_bits = 0x7ff0000000000000ull;
     std::vector<unsigned long long> infs((size_t)c->count, inf_bits);
     BCHECK(hipMemcpyAsync(c->cfl_bits, infs.data(), infs.size() * 8, hipMemcpyHostToDevice, c->stream));
-    std::vector<std::vector<double>> keep;          // host buffers alive until the copies are done
     size_t off = 0;
     for (int i = 0; i < c->count; ++i) {
         const int m = c->m[i], n = c->n[i];
-        const size_t mn = (size_t)m * n;
-        const double *r = rho + off, *uu = u + off, *vv = v + off, *pp = p + off;
-        keep.emplace_back(mn);
-        std::vector<double> &E = keep.back();
-        for (size_t k = 0; k < mn; ++k) {
-            double t = 0.5 * uu[k] * uu[k] + pp[k] / (gamma - 1.0) / r[k];
-            t += 0.5 * vv[k] * vv[k];
-            E[k] = t;
-        }
         const BatchGrid &g = c->grids[i];
-        const double *src[5] = {r, uu, vv, pp, E.data()};
-        for (int f = 0; f < 5; ++f)
-            BCHECK(hipMemcpy2DAsync(g.st[0] + (size_t)f * g.plane, (size_t)g.ld * 8, src[f], (size_t)n * 8,
-                                    (size_t)n * 8, (size_t)m, hipMemcpyHostToDevice, c->stream));
-        // BC -1 ghosts from the initial data (bound_cond_slope_limiter_x.c:37-46)
-        keep.emplace_back((size_t)8 * (m + n));
-        std::vector<double> &b = keep.back();
-        double *xl = b.data(), *xh = xl + (size_t)n * 4, *yl = xh + (size_t)n * 4, *yh = yl + (size_t)m * 4;
-        const double *q4[4] = {r, uu, vv, pp};
-        for (int ii = 0; ii < n; ++ii)
-            for (int q = 0; q < 4; ++q) {
-                xl[(size_t)ii * 4 + q] = q4[q][ii];
-                xh[(size_t)ii * 4 + q] = q4[q][(size_t)(m - 1) * n + ii];
-            }
-        for (int j = 0; j < m; ++j)
-            for (int q = 0; q < 4; ++q) {
-                yl[(size_t)j * 4 + q] = q4[q][(size_t)j * n];
-                yh[(size_t)j * 4 + q] = q4[q][(size_t)j * n + n - 1];
-            }
-        BCHECK(hipMemcpyAsync((void *)g.bnd[0], b.data(), b.size() * 8, hipMemcpyHostToDevice, c->stream));
+        const double *src[5] = {rho + off, u + off, v + off, p + off, nullptr};
+        BCHECK(upload_state(src, g.st[1], g.st[0], (double *)g.bnd[0], g.plane, m, n, g.ld, gamma, c->stream));
         BCHECK(launch_cfl(g.st[0], g.st[0] + g.plane, g.st[0] + 2 * g.plane, g.st[0] + 3 * g.plane, m, n, g.ld, gamma,
                           fmin(c->hx[i], c->hy[i]), c->cfl_bits + i, c->stream));
-        off += mn;
+        off += (size_t)m * n;
     }
     std::vector<unsigned long long> bits((size_t)c->count);
     BCHECK(hipMemcpyAsync(bits.data(), c->cfl_bits, bits.size() * 8, hipMemcpyDeviceToHost, c->stream));
@@ -700,12 +673,9 @@ extern "C" int hgrp2db_download(hgrp2db *c, double *rho, double *u, double *v, d
     size_t off = 0;
     for (int i = 0; i < c->count; ++i) {
         const BatchGrid &g = c->grids[i];
-        const double *src = g.st[c->res_cs[i]];
-        for (int f = 0; f < 5; ++f) {
-            if (!dst[f]) continue;
-            BCHECK(hipMemcpy2DAsync(dst[f] + off, (size_t)g.n * 8, src + (size_t)f * g.plane, (size_t)g.ld * 8,
-                                    (size_t)g.n * 8, (size_t)g.m, hipMemcpyDeviceToHost, c->stream));
-        }
+        double *to[5];
+        for (int f = 0; f < 5; ++f) to[f] = dst[f] ? dst[f] + off : nullptr;
+        BCHECK(download_planes(to, 5, g.st[c->res_cs[i]], g.st[1 - c->res_cs[i]], g.plane, g.m, g.n, g.ld, c->stream));
         off += (size_t)g.m * g.n;
     }
     BCHECK(hipStreamSynchronize(c->stream));

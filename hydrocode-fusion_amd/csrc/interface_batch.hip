@@ -196,22 +196,29 @@ struct DevBuf {
 int run_batch(const void *const *hin, const size_t *in_bytes, int nin, void *hout, size_t out_bytes,
               void (*launch)(void *const *din, void *dout, void *ctx), void *ctx)
 {
-    DevBuf bufs[4], ob;
+    // one allocation for the inputs and the results: each costs a call as much
+    // as the copies of a small batch
+    DevBuf buf;
     void *din[4] = {nullptr, nullptr, nullptr, nullptr};
-    for (int q = 0; q < nin; ++q) {
-        if (hipMalloc(&bufs[q].p, in_bytes[q] ? in_bytes[q] : 8) != hipSuccess) return -2;
-        if (in_bytes[q] && hipMemcpy(bufs[q].p, hin[q], in_bytes[q], hipMemcpyHostToDevice) != hipSuccess) return -3;
-        din[q] = bufs[q].p;
+    size_t total = 0, at[5];
+    for (int q = 0; q <= nin; ++q) {
+        at[q] = total;
+        total += ((q < nin ? in_bytes[q] : out_bytes) + 255) / 256 * 256;
     }
-    if (hipMalloc(&ob.p, out_bytes ? out_bytes : 8) != hipSuccess) return -2;
-    launch(din, ob.p, ctx);
+    if (hipMalloc(&buf.p, total ? total : 8) != hipSuccess) return -2;
+    for (int q = 0; q < nin; ++q) {
+        din[q] = (char *)buf.p + at[q];
+        if (in_bytes[q] && hipMemcpy(din[q], hin[q], in_bytes[q], hipMemcpyHostToDevice) != hipSuccess) return -3;
+    }
+    void *dout = (char *)buf.p + at[nin];
+    launch(din, dout, ctx);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e != hipSuccess) {
         fprintf(stderr, "hydrogrp: batch kernel failed: %s\n", hipGetErrorString(e));
         return -(int)e - 1;
     }
-    if (out_bytes && hipMemcpy(hout, ob.p, out_bytes, hipMemcpyDeviceToHost) != hipSuccess) return -3;
+    if (out_bytes && hipMemcpy(hout, dout, out_bytes, hipMemcpyDeviceToHost) != hipSuccess) return -3;
     return 0;
 }
 
