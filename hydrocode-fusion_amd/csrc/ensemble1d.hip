@@ -212,6 +212,11 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) if
                                                    const double *s_u, const double *s_p, double *mid, double *dire,
                                                    size_t n_if_all)
 {
+    __shared__ double tab[POW_TAB];
+    TabLoad<BS> tl;
+    tl.load(threadIdx.x);
+    tl.store(threadIdx.x, tab);
+    __syncthreads();
     const int wv = wave_index<BS>();
     if (wv >= n_w) return;
     const int2 we = T.w_if[wv];
@@ -264,7 +269,7 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) if
             flag(Ip, FLAG_ABORT);
         } else {
             double D[3], U[3];
-            const bool done = in && grp_edir_q(D, U, L, R, rL, rR, c_L, c_R, P.gas, P.near2, eps);
+            const bool done = in && grp_edir_q(D, U, L, R, rL, rR, c_L, c_R, P.gas, P.near2, eps, tab);
             if (__builtin_expect(__any(!done), 0)) {
                 if (!done) {
                     double DU[6];

@@ -201,14 +201,14 @@ __device__ __attribute__((noinline)) static StarQ star_ieee(double g_L, double g
 // the right side.  D[6], U[6] = rho u v p z_a phi; ws[2] wave speeds; us[6] =
 // rho_star_L u_star rho_star_R p_star c_star_L c_star_R.  tol, p_guess and
 // CONV as riemann_exact's (the reference: tol = eps, no guess, its own rule).
-// FAST: the exact Riemann solve in the steps' arithmetic (riemann_q, the same
-// star state), riemann_exact out of line where a side is out of its range: the
-// Newton iteration is most of the solver's divisions (an unsplit step, 257 x
-// 190: .132 -> .104 ms; 1024^2: .469 -> .387).
+// FAST: the exact Riemann solve in the steps' arithmetic (riemann_q with the
+// pow tables tab, the same star state), riemann_exact out of line where a side
+// is out of its range: the Newton iteration is most of the solver's divisions
+// (an unsplit step, 257 x 190: .132 -> .104 ms; 1024^2: .469 -> .387).
 template <bool CONV = false, bool FAST = false>
 __device__ __forceinline__ void grp_g2d(double D[6], double U[6], double ws[2], double us[6], G2Side L, G2Side R,
                                         double lu, double lv, double eps, double atc, double tol,
-                                        double p_guess = -1.0)
+                                        double p_guess = -1.0, const double *tab = nullptr)
 {
     double u_star, p_star, speed_L, speed_R;
     const double dist = sqrt((L.rho - R.rho) * (L.rho - R.rho) + (L.u - R.u) * (L.u - R.u)
@@ -224,7 +224,7 @@ __device__ __forceinline__ void grp_g2d(double D[6], double U[6], double ws[2], 
             bool in = gas_in_range(L.G) && gas_in_range(R.G) && fmin(L.p, R.p) >= 0x1p-100 && L.p + R.p <= 0x1p100 &&
                       fmin(L.c, R.c) >= 0x1p-100 && fabs(L.u) + fabs(R.u) + L.c + R.c <= 0x1p100;
             if (in)
-                in = riemann_q<CONV>(L.G, R.G, L.u, R.u, rcp_of(L.p), rcp_of(R.p), L.c, R.c, eps, tol, p_guess, st);
+                in = riemann_q<CONV>(L.G, R.G, L.u, R.u, rcp_of(L.p), rcp_of(R.p), L.c, R.c, eps, tol, p_guess, st, tab);
             if (!in) st = star_ieee<CONV>(L.G.g, R.G.g, L.u, R.u, L.p, R.p, L.c, R.c, eps, tol, p_guess);
         } else {
             const StarResult r = riemann_exact<CONV>(L.G, R.G, L.u, R.u, L.p, R.p, L.c, R.c, eps, tol, 500, p_guess);
@@ -367,7 +367,7 @@ __device__ __forceinline__ G2Side g2_side(const Side &S, const double T[4], cons
 template <bool CONV = false>
 __device__ __forceinline__ int grp_2d_flux_g2d(Side L, Side R, const double TL[4], const double TR[4], const Gas &G,
                                                double n_x, double n_y, double tau, double eps, double F[4],
-                                               double I[4], double tol, double p_guess = -1.0)
+                                               double I[4], double tol, double p_guess, const double *tab)
 {
     const double u = L.u * n_x + L.v * n_y;
     const double u_R = R.u * n_x + R.v * n_y;
@@ -382,7 +382,7 @@ __device__ __forceinline__ int grp_2d_flux_g2d(Side L, Side R, const double TL[4
     L.u = u; R.u = u_R; L.d_u = d_u; R.d_u = d_u_R;
     double dire[6], mid[6], ws[2], us[6];
     grp_g2d<CONV, true>(dire, mid, ws, us, g2_side(L, TLr, G, -1.0), g2_side(R, TRr, G, 1.0), 0.0, 0.0, eps, eps, tol,
-                        p_guess);
+                        p_guess, tab);
     return flux_from_mid_n(mid, dire, G, n_x, n_y, tau, eps, F, I);
 }
 

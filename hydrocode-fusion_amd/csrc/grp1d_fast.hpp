@@ -20,18 +20,18 @@ HGRP_HD bool sides1_in_range(const Side1 &L, const Side1 &R)
 // the axis inside the rarefaction next to side S (grp_edir's sonic branches)
 // false where there is no sonic point (a vacuum that the iteration left)
 template <int SIGN>
-HGRP_HD bool edir_sonic_q(double D[3], double U[3], const Side1 &S, const Rcp &rho, double c, const Gas &G)
+HGRP_HD bool edir_sonic_q(double D[3], double U[3], const Side1 &S, const Rcp &rho, double c, const Gas &G, const double *P)
 {
     const Rcp gm1 = {G.gm1(), G.y_gm1}, rg = {G.g, G.inv_g};
     const double t = div_q(2.0 * c, gm1);
     U[1] = G.z * (SIGN < 0 ? S.u + t : S.u - t);
     if (!((SIGN < 0 ? U[1] : -U[1]) >= 0x1p-200)) return false;
-    U[2] = div_1(div_q(U[1] * U[1] * S.rho, rg), pow_in_range(log_in_range(S.p), G.inv_g));
-    U[2] = pow_in_range(log_in_range(U[2]), G.g_gm1);
+    U[2] = div_1(div_q(U[1] * U[1] * S.rho, rg), pow_in_range(log_in_range(S.p, P), G.inv_g, P));
+    U[2] = pow_in_range(log_in_range(U[2], P), G.g_gm1, P);
     const Rcp rU = rcp_of(U[1]);
     U[0] = div_q(div_q(G.g * U[2], rU), rU);
-    const DD l = log_in_range(div_1(SIGN < 0 ? U[1] : -U[1], c));
-    const double pw_a = pow_in_range(l, G.e_a), pw_b = pow_in_range(l, G.e_b);
+    const DD l = log_in_range(div_1(SIGN < 0 ? U[1] : -U[1], c), P);
+    const double pw_a = pow_in_range(l, G.e_a, P), pw_b = pow_in_range(l, G.e_b, P);
     const double e = S.s_p - S.s_rho * c * c;
     D[1] = div_q(0.5 * (pw_a * (1.0 + G.z) + pw_b * G.z), {0.5 + G.z, 2.0 * G.y_op2z});
     D[1] = div_q(div_q(D[1] * e, gm1), rho);
@@ -46,7 +46,7 @@ HGRP_HD bool edir_sonic_q(double D[3], double U[3], const Side1 &S, const Rcp &r
 // one side's row a u_t + b p_t = d in the non-sonic case; pw_b as in grp_edir
 template <int SIGN>
 HGRP_HD void edir_row_q(const Side1 &S, const Rcp &rho, double c, double p_star, double u_star, const Rcp &rs, const Rcp &cs,
-                        int fan, double shk, const Gas &G, double &a, double &b, double &d, double &pw_b)
+                        int fan, double shk, const Gas &G, double &a, double &b, double &d, double &pw_b, const double *P)
 {
     if (fan) {
         const Rcp gm1 = {G.gm1(), G.y_gm1};
@@ -54,9 +54,9 @@ HGRP_HD void edir_row_q(const Side1 &S, const Rcp &rho, double c, double p_star,
         const double inv = recip_q(rs);
         b = div_q(SIGN < 0 ? inv : -inv, cs);
         const Rcp rc = rcp_of(c);
-        const DD l = log_in_range(div_q(cs.b, rc));
-        const double pw_a = pow_in_range(l, G.e_a);
-        pw_b = pow_in_range(l, G.e_b);
+        const DD l = log_in_range(div_q(cs.b, rc), P);
+        const double pw_a = pow_in_range(l, G.e_a, P);
+        pw_b = pow_in_range(l, G.e_b, P);
         d = div_q(0.5 * (pw_a * (1.0 + G.z) + pw_b * G.z), {0.5 + G.z, 2.0 * G.y_op2z});
         d = div_q(div_q(d * (S.s_p - S.s_rho * c * c), gm1), rho);
         const double r = div_q(div_q(div_q(G.g * S.s_p, rc) - c * S.s_rho, gm1), rho);
@@ -82,7 +82,7 @@ HGRP_HD void edir_row_q(const Side1 &S, const Rcp &rho, double c, double p_star,
 // near2: the acoustic switch on the squared distance; c_L, c_R: sqrt(gamma p / rho).
 // False, with nothing to use, where the interface is for grp_edir.
 HGRP_HD bool grp_edir_q(double D[3], double U[3], const Side1 &L, const Side1 &R, const Rcp &rL, const Rcp &rR, double c_L,
-                        double c_R, const Gas &G, double near2, double eps)
+                        double c_R, const Gas &G, double near2, double eps, const double *P)
 {
     const double dist2 = (L.u - R.u) * (L.u - R.u) + (L.p - R.p) * (L.p - R.p);
     if (dist2 < near2) {
@@ -109,12 +109,12 @@ HGRP_HD bool grp_edir_q(double D[3], double U[3], const Side1 &L, const Side1 &R
     const bool rough = any_lane(tiny(L.u) || tiny(R.u) || tiny(L.s_u) || tiny(R.s_u));
     const Rcp pL = rcp_of(L.p), pR = rcp_of(R.p);
     StarQ st;
-    if (!riemann_q<false, 50>(G, G, L.u, R.u, pL, pR, c_L, c_R, eps, eps, -1.0, st)) return false;
+    if (!riemann_q<false, 50>(G, G, L.u, R.u, pL, pR, c_L, c_R, eps, eps, -1.0, st, P)) return false;
     const double u = st.u, p = st.p, z = G.z;
     const double rs_L = p > L.p ? div_1(L.rho * (p + z * L.p), L.p + z * p)
-                                : L.rho * pow_in_range(log_in_range(div_q(p, pL)), G.inv_g);
+                                : L.rho * pow_in_range(log_in_range(div_q(p, pL), P), G.inv_g, P);
     const double rs_R = p > R.p ? div_1(R.rho * (p + z * R.p), R.p + z * p)
-                                : R.rho * pow_in_range(log_in_range(div_q(p, pR)), G.inv_g);
+                                : R.rho * pow_in_range(log_in_range(div_q(p, pR), P), G.inv_g, P);
     const Rcp qL = rcp_of(rs_L), qR = rcp_of(rs_R);
     const Rcp kL = rcp_of(sqrt_q(div_q(G.g * p, qL))), kR = rcp_of(sqrt_q(div_q(G.g * p, qR)));
     // shock speeds; where the density does not change by an ulp the quotient is IEEE's infinity or NaN
@@ -134,12 +134,12 @@ HGRP_HD bool grp_edir_q(double D[3], double U[3], const Side1 &L, const Side1 &R
         return true;
     }
     if (s_R < 0.0) { edir_upwind(D, U, R.rho, R.u, R.p, R.s_rho, R.s_u, R.s_p, G); return true; }
-    if (st.crw0 && u - kL.b > 0.0) return edir_sonic_q<-1>(D, U, L, rL, c_L, G);
-    if (st.crw1 && u + kR.b < 0.0) return edir_sonic_q<+1>(D, U, R, rR, c_R, G);
+    if (st.crw0 && u - kL.b > 0.0) return edir_sonic_q<-1>(D, U, L, rL, c_L, G, P);
+    if (st.crw1 && u + kR.b < 0.0) return edir_sonic_q<+1>(D, U, R, rR, c_R, G, P);
 
     double a_L, b_L, d_L, w_L, a_R, b_R, d_R, w_R;
-    edir_row_q<-1>(L, rL, c_L, p, u, qL, kL, st.crw0, s_L, G, a_L, b_L, d_L, w_L);
-    edir_row_q<+1>(R, rR, c_R, p, u, qR, kR, st.crw1, s_R, G, a_R, b_R, d_R, w_R);
+    edir_row_q<-1>(L, rL, c_L, p, u, qL, kL, st.crw0, s_L, G, a_L, b_L, d_L, w_L, P);
+    edir_row_q<+1>(R, rR, c_R, p, u, qR, kR, st.crw1, s_R, G, a_R, b_R, d_R, w_R, P);
     const Rcp ra = rcp_of(a_L);
     const double p_t = div_r(div_r(d_L * a_R, ra, rough) - d_R, rcp_of(div_q(b_L * a_R, ra) - b_R), rough);
     const double u_t = div_r(d_L - b_L * p_t, ra, rough);

@@ -120,10 +120,11 @@ __global__ void __launch_bounds__(64 * W, MINW) batch_x_kernel(BatchSweep b)
     __shared__ double xf[W][4][64];
     __shared__ double xi[W][4][64];
     __shared__ double xe[W][64];
+    __shared__ double tab[POW_TAB];
     const int4 t = b.tiles[blockIdx.x];
     if (b.grids[t.x].halted) return;                    // the whole block
     const SweepArgs a = batch_args(b, t.x);
-    line_sweep<0, W, NM>(a, BatchArgs{t.x}, t.y, t.z, xa, xb, xf, xi, xe);
+    line_sweep<0, W, NM>(a, BatchArgs{t.x}, t.y, t.z, xa, xb, xf, xi, xe, tab);
 }
 
 // the X sweep walking K chunks of W rows per block (line_sweep_chunks): the
@@ -136,10 +137,11 @@ __global__ void __launch_bounds__(64 * W, MINW) batch_x_chunks_kernel(BatchSweep
     __shared__ double xf[W][4][64];
     __shared__ double xi[W][4][64];
     __shared__ double xe[W][64];
-    __shared__ double xc[2][8][64];                     // the last face of the previous chunk: F, I
+    __shared__ double xc[8][64];                        // the last face of the previous chunk: F, I
+    __shared__ double tab[POW_TAB];
     const int4 t = b.tiles[blockIdx.x];
     if (b.grids[t.x].halted) return;                    // the whole block
-    line_sweep_chunks<0, W, NM, K>(BatchArgs{t.x}, t.y, t.z, xa, xb, xf, xi, xe, xc);
+    line_sweep_chunks<0, W, NM, K>(BatchArgs{t.x}, t.y, t.z, xa, xb, xf, xi, xe, xc, tab);
 }
 
 template <int MINW, int NM, int G>
@@ -148,11 +150,12 @@ __global__ void __launch_bounds__(256, MINW) batch_y_kernel(BatchSweep b)
     constexpr bool LEARNED = NM == NM_LEARNED;
     __shared__ uint32_t mlp_lds[LEARNED ? 4 : 1][LEARNED ? 64 * 8 : 1];
     __shared__ double stash[4][5][64];
+    __shared__ double tab[POW_TAB];
     const int4 t = b.tiles[blockIdx.x];                 // grid, first wave of the block, chunks per row group
     if (b.grids[t.x].halted) return;
     const SweepArgs a = batch_args(b, t.x);
     const int wv = (threadIdx.x >> 6) & 3;
-    y_sweep<MINW, NM, G>(a, BatchArgs{t.x}, (long)t.y + wv, t.z, stash[wv], mlp_lds[wv]);
+    y_sweep<MINW, NM, G>(a, BatchArgs{t.x}, (long)t.y + wv, t.z, stash[wv], mlp_lds[wv], tab);
 }
 
 // the one-grid launch variants (sweep2d.hip) X 0..4 and Y 0..4: X 0 = 8 rows

@@ -80,7 +80,7 @@ HGRP_HD bool gas_in_range(const Gas &G) { return G.gm1() >= 0x1p-20 && G.g <= 0x
 // log(p/p_s) on the rarefaction branch, 1/sqrt(1 + nu (p - p_s)/p_s) in hi on
 // the shock branch.
 template <int SIGN>
-HGRP_HD double curve_q(double p, double u_s, const Rcp &p_s, double c_s, const Gas &G, DD *keep)
+HGRP_HD double curve_q(double p, double u_s, const Rcp &p_s, double c_s, const Gas &G, DD *keep, const double *P)
 {
     double w;
     if (p > p_s.b) {
@@ -89,15 +89,15 @@ HGRP_HD double curve_q(double p, double u_s, const Rcp &p_s, double c_s, const G
         keep->hi = s.y;
         w = div_q(div_q(div_q(dp * c_s, {G.g, G.inv_g}), p_s), s);
     } else {
-        *keep = log_in_range(div_q(p, p_s));
-        w = pow_in_range(*keep, G.mu) - 1.0;
+        *keep = log_in_range(div_q(p, p_s), P);
+        w = pow_in_range(*keep, G.mu, P) - 1.0;
         w = div_q(2.0 * c_s * w, {G.gm1(), G.y_gm1});
     }
     return SIGN < 0 ? u_s - w : u_s + w;
 }
 
 // dv/dp along the 3-wave (the 1-wave's is its negative) at the pressure of the last curve_q
-HGRP_HD double slope_q(double p, const Rcp &p_s, double c_s, const Gas &G, const DD &keep)
+HGRP_HD double slope_q(double p, const Rcp &p_s, double c_s, const Gas &G, const DD &keep, const double *P)
 {
     const double t2 = div_q(div_q(c_s, {G.g, G.inv_g}), p_s);
     if (p > p_s.b) {
@@ -105,7 +105,7 @@ HGRP_HD double slope_q(double p, const Rcp &p_s, double c_s, const Gas &G, const
         const double t3 = div_q(0.5 * t2 * G.nu, p_s);
         return t2 * t1 - t3 * (p - p_s.b) * cube(t1);
     }
-    return recip_1(pow_in_range(keep, G.nu)) * t2;
+    return recip_1(pow_in_range(keep, G.nu, P)) * t2;
 }
 
 struct StarQ {
@@ -116,11 +116,11 @@ struct StarQ {
 // riemann_exact with at most N steps; false where the pressure leaves the range (or is not a number)
 template <bool CONV, int N = 500>
 HGRP_HD bool riemann_q(const Gas &GL, const Gas &GR, double u_L, double u_R, const Rcp &p_L, const Rcp &p_R,
-                       double c_L, double c_R, double eps, double tol, double p_guess, StarQ &out)
+                       double c_L, double c_R, double eps, double tol, double p_guess, StarQ &out, const double *P)
 {
     DD bL = {0.0, 0.0}, bR = {0.0, 0.0};
-    const double u_LR = curve_q<-1>(p_R.b, u_L, p_L, c_L, GL, &bL);
-    const double u_RL = curve_q<+1>(p_L.b, u_R, p_R, c_R, GR, &bR);
+    const double u_LR = curve_q<-1>(p_R.b, u_L, p_L, c_L, GL, &bL, P);
+    const double u_RL = curve_q<+1>(p_L.b, u_R, p_R, c_R, GR, &bR, P);
     out.crw1 = (u_LR > u_R + eps) ? 0 : 1;
     out.crw0 = (u_RL > u_L - eps) ? 1 : 0;
     if (fabs(u_L - u_R) < tol && fabs(p_L.b - p_R.b) < tol) {
@@ -142,14 +142,14 @@ HGRP_HD bool riemann_q(const Gas &GL, const Gas &GR, double u_L, double u_R, con
                 p = 0.5 * p0;
             }
         } else {
-            k1 = -slope_q(p, p_L, c_L, GL, bL);
-            k3 = slope_q(p, p_R, c_R, GR, bR);
+            k1 = -slope_q(p, p_L, c_L, GL, bL, P);
+            k3 = slope_q(p, p_R, c_R, GR, bR, P);
             const double p_new = p + div_1(v_R - v_L, k1 - k3);
             p = (p_new < 0.0) ? 0.5 * p : p_new;
         }
         if (__builtin_expect(!(p > 0x1p-300 && p < 0x1p300), 0)) return false;
-        v_L = curve_q<-1>(p, u_L, p_L, c_L, GL, &bL);
-        v_R = curve_q<+1>(p, u_R, p_R, c_R, GR, &bR);
+        v_L = curve_q<-1>(p, u_L, p_L, c_L, GL, &bL, P);
+        v_R = curve_q<+1>(p, u_R, p_R, c_R, GR, &bR, P);
         const double gap = fabs(v_L - v_R);
         if (st == 1 || st == 4) ++done;
         if (st == 3 || st == 5) ++n;
@@ -181,13 +181,13 @@ HGRP_HD bool riemann_q(const Gas &GL, const Gas &GR, double u_L, double u_R, con
 // head.  SIGN -1: the 1-wave, +1: the 3-wave.
 template <int SIGN>
 HGRP_HD void behind_q(double rho, double u, const Rcp &p, double c, double p_star, int fan, const Gas &G, double &rs,
-                      double &cs, double &speed)
+                      double &cs, double &speed, const double *P)
 {
     const double x = div_q(p_star, p);
     if (fan) {
-        const DD l = log_in_range(x);
-        rs = rho * pow_in_range(l, G.inv_g);
-        cs = c * pow_in_range(l, G.e_cs);
+        const DD l = log_in_range(x, P);
+        rs = rho * pow_in_range(l, G.inv_g, P);
+        cs = c * pow_in_range(l, G.e_cs, P);
         speed = SIGN < 0 ? u - c : u + c;
     } else {
         rs = div_1(rho * (p_star + G.z * p.b), p.b + G.z * p_star);
@@ -200,10 +200,10 @@ HGRP_HD void behind_q(double rho, double u, const Rcp &p, double c, double p_sta
 // (1 + z) x^e_a + z x^e_b over 1 + 2 z, times TdS, minus / plus c x^e_a dI: the
 // derivative along a rarefaction's characteristic; *xb receives x^e_b
 template <int SIGN>
-HGRP_HD double fan_line_q(double x, double c, const Gas &G, double TdS, double dI, double *xb)
+HGRP_HD double fan_line_q(double x, double c, const Gas &G, double TdS, double dI, double *xb, const double *P)
 {
-    const DD l = log_in_range(x);
-    const double a = pow_in_range(l, G.e_a), b = pow_in_range(l, G.e_b);
+    const DD l = log_in_range(x, P);
+    const double a = pow_in_range(l, G.e_a, P), b = pow_in_range(l, G.e_b, P);
     *xb = b;
     double d = G.opz() * a + G.z * b;
     d = div_q(d, {G.op2z(), G.y_op2z}) * TdS;
@@ -229,7 +229,7 @@ struct LineQ {
 };
 template <int SIGN>
 HGRP_HD void line_q(const Rcp &rho, double p, double c, double d_rho, double d_u, double d_p, double p_star,
-                    double rs, double cs, int fan, const Gas &G, LineQ &o)
+                    double rs, double cs, int fan, const Gas &G, LineQ &o, const double *P)
 {
     const Rcp rrs = rcp_of(rs);
     if (fan) {
@@ -238,7 +238,7 @@ HGRP_HD void line_q(const Rcp &rho, double p, double c, double d_rho, double d_u
         o.a = 1.0;
         const double inv = recip_q(rrs);
         o.b = div_1(SIGN < 0 ? inv : -inv, cs);
-        o.d = fan_line_q<SIGN>(div_1(cs, c), c, G, TdS, dI, &o.xb);
+        o.d = fan_line_q<SIGN>(div_1(cs, c), c, G, TdS, dI, &o.xb, P);
         o.Ss = o.S = 0.0;
     } else {
         const double ss = sqrt_q(div_q(0.5 * (G.gp1() * p + G.gm1() * p_star), rrs));
@@ -272,7 +272,7 @@ HGRP_HD void line_q(const Rcp &rho, double p, double c, double d_rho, double d_u
 template <bool TRANS, bool TF, bool CONV>
 HGRP_HD bool grp_q1d_q(double D[4], double U[4], const Side &L, const Side &R, const double TL[4], const double TR[4],
                        const Gas &GL, const Gas &GR, double near2, double eps, double tol, double p_guess,
-                       const double *FA, double *FO)
+                       const double *FA, double *FO, const double *P)
 {
     const Rcp rL = rcp_of(L.rho), rR = rcp_of(R.rho);
     const double c_L = sqrt_q(div_q(GL.g * L.p, rL)), c_R = sqrt_q(div_q(GR.g * R.p, rR));
@@ -291,9 +291,9 @@ HGRP_HD bool grp_q1d_q(double D[4], double U[4], const Side &L, const Side &R, c
     } else {
         rough = any_lane(tiny(L.u) || tiny(R.u) || tiny(L.d_u) || tiny(R.d_u));
         const Rcp pL = rcp_of(L.p), pR = rcp_of(R.p);
-        if (!riemann_q<CONV>(GL, GR, L.u, R.u, pL, pR, c_L, c_R, eps, tol, p_guess, st)) return false;
-        behind_q<-1>(L.rho, L.u, pL, c_L, st.p, st.crw0, GL, rs_L, cs_L, speed_L);
-        behind_q<+1>(R.rho, R.u, pR, c_R, st.p, st.crw1, GR, rs_R, cs_R, speed_R);
+        if (!riemann_q<CONV>(GL, GR, L.u, R.u, pL, pR, c_L, c_R, eps, tol, p_guess, st, P)) return false;
+        behind_q<-1>(L.rho, L.u, pL, c_L, st.p, st.crw0, GL, rs_L, cs_L, speed_L, P);
+        behind_q<+1>(R.rho, R.u, pR, c_R, st.p, st.crw1, GR, rs_R, cs_R, speed_R, P);
     }
     const double u_star = st.u, p_star = st.p;
 
@@ -364,16 +364,16 @@ HGRP_HD bool grp_q1d_q(double D[4], double U[4], const Side &L, const Side &R, c
         if (!(C >= 0x1p-200)) return false;                // no sonic point (a vacuum that the iteration left)
         const Rcp rC = rcp_of(C);
         const double x = div_1(C, c);
-        U[3] = pow_in_range(log_in_range(x), G.e_sonic) * p;
+        U[3] = pow_in_range(log_in_range(x, P), G.e_sonic, P) * p;
         U[0] = div_q(div_q(G.g * U[3], rC), rC);
         U[2] = in0 ? L.v : R.v;
         double TdS, dI, xb;
         if (in0) {
             invariants_q<-1>(rho, c, L.d_rho, L.d_u, L.d_p, G, TdS, dI);
-            D[1] = fan_line_q<-1>(x, c, G, TdS, dI, &xb);
+            D[1] = fan_line_q<-1>(x, c, G, TdS, dI, &xb, P);
         } else {
             invariants_q<+1>(rho, c, R.d_rho, R.d_u, R.d_p, G, TdS, dI);
-            D[1] = fan_line_q<+1>(x, c, G, TdS, dI, &xb);
+            D[1] = fan_line_q<+1>(x, c, G, TdS, dI, &xb, P);
         }
         D[3] = U[0] * U[1] * D[1];
         D[0] = U[0] * U[1] * xb * TdS * G.gm1();
@@ -382,8 +382,8 @@ HGRP_HD bool grp_q1d_q(double D[4], double U[4], const Side &L, const Side &R, c
         if constexpr (TF) { FO[0] = in0 ? FA[0] : FA[2]; FO[1] = -U[1] * (in0 ? FA[1] : FA[3]) * U[0] / rho.b; }
     } else {                                              // non-sonic
         LineQ l, r;
-        line_q<-1>(rL, L.p, c_L, L.d_rho, L.d_u, L.d_p, p_star, rs_L, cs_L, st.crw0, GL, l);
-        line_q<+1>(rR, R.p, c_R, R.d_rho, R.d_u, R.d_p, p_star, rs_R, cs_R, st.crw1, GR, r);
+        line_q<-1>(rL, L.p, c_L, L.d_rho, L.d_u, L.d_p, p_star, rs_L, cs_L, st.crw0, GL, l, P);
+        line_q<+1>(rR, R.p, c_R, R.d_rho, R.d_u, R.d_p, p_star, rs_R, cs_R, st.crw1, GR, r, P);
         const Rcp det = rcp_of(l.a * r.b - l.b * r.a);
         const double u_t = div_r(r.b * l.d - l.b * r.d, det, rough);
         const double p_t = div_r(l.a * r.d - r.a * l.d, det, rough);
@@ -456,7 +456,7 @@ inline double near_threshold(double eps)
 template <int DIR, bool CONV>
 __device__ __forceinline__ bool flux_split_q(const Side &L, const Side &R, const Gas &G, double near2, double tau,
                                              double eps, double F[4], double I[4], double tol, double p_guess,
-                                             int *code)
+                                             int *code, const double *P)
 {
     if (!(gas_in_range(G) && sides_in_range(L, R))) return false;
     Side l = L, r = R;
@@ -465,7 +465,7 @@ __device__ __forceinline__ bool flux_split_q(const Side &L, const Side &R, const
         r.u = R.v; r.v = -R.u; r.d_u = R.d_v; r.d_v = -R.d_u;
     }
     double D[4], U[4];
-    if (!grp_q1d_q<false, false, CONV>(D, U, l, r, nullptr, nullptr, G, G, near2, eps, tol, p_guess, nullptr, nullptr))
+    if (!grp_q1d_q<false, false, CONV>(D, U, l, r, nullptr, nullptr, G, G, near2, eps, tol, p_guess, nullptr, nullptr, P))
         return false;
     *code = flux_from_mid<DIR>(U, D, G, tau, eps, F, I);
     return true;
@@ -476,7 +476,7 @@ __device__ __forceinline__ bool flux_split_q(const Side &L, const Side &R, const
 template <bool CONV>
 __device__ __forceinline__ bool flux_transversal_q(const Side &L, const Side &R, const double TL[4], const double TR[4],
                                                    const Gas &G, int dir, double near2, double tau, double eps, double F[4],
-                                                   double I[4], double tol, double p_guess, int *code)
+                                                   double I[4], double tol, double p_guess, int *code, const double *P)
 {
     const double t = ((fabs(TL[0]) + fabs(TL[1])) + (fabs(TL[2]) + fabs(TL[3]))) +
                      ((fabs(TR[0]) + fabs(TR[1])) + (fabs(TR[2]) + fabs(TR[3])));
@@ -490,7 +490,7 @@ __device__ __forceinline__ bool flux_transversal_q(const Side &L, const Side &R,
         tr[1] = TR[2]; tr[2] = -TR[1];
     }
     double D[4], U[4];
-    if (!grp_q1d_q<true, false, CONV>(D, U, l, r, tl, tr, G, G, near2, eps, tol, p_guess, nullptr, nullptr)) return false;
+    if (!grp_q1d_q<true, false, CONV>(D, U, l, r, tl, tr, G, G, near2, eps, tol, p_guess, nullptr, nullptr, P)) return false;
     *code = flux_from_mid_n(U, D, G, dir ? 0.0 : 1.0, dir ? 1.0 : 0.0, tau, eps, F, I);
     return true;
 }
@@ -536,7 +536,7 @@ __device__ __forceinline__ bool two_in_range(const TwoGas &T)
 template <int DIR, bool CONV>
 __device__ __forceinline__ bool flux_two_fluid_q(const Side &L, const Side &R, const TwoGas &T, const double FA[4],
                                                  double near2, double tau, double eps, double F[4], double I[4],
-                                                 double FZ[3], double tol, double p_guess, int *code)
+                                                 double FZ[3], double tol, double p_guess, int *code, const double *P)
 {
     constexpr double n_x = DIR == 0 ? 1.0 : 0.0, n_y = DIR == 0 ? 0.0 : 1.0;
     // reconstructed fractions leave [0, 1] by rounding only
@@ -554,7 +554,7 @@ __device__ __forceinline__ bool flux_two_fluid_q(const Side &L, const Side &R, c
         r.u = R.v; r.v = -R.u; r.d_u = R.d_v; r.d_v = -R.d_u;
     }
     double dire[4], mid[4], fo[2];
-    if (!grp_q1d_q<false, true, CONV>(dire, mid, l, r, nullptr, nullptr, GL, GR, near2, eps, tol, p_guess, FA, fo))
+    if (!grp_q1d_q<false, true, CONV>(dire, mid, l, r, nullptr, nullptr, GL, GR, near2, eps, tol, p_guess, FA, fo, P))
         return false;
     *code = star_dire_bad(mid, dire, eps);
     if (*code) {

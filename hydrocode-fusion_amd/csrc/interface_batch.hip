@@ -37,8 +37,8 @@ __global__ void __launch_bounds__(128) flux_batch_kernel(const double *L, const 
     double F[4], I[4];
     int code = 0;
     const bool in = l[0] - 1.0 >= 0x1p-20 && l[0] <= 0x1p20;
-    const bool done = in && (dir == 0 ? flux_split_q<0, false>(SL, SR, make_gas_q(l[0]), near2, tau, eps, F, I, eps, -1.0, &code)
-                                      : flux_split_q<1, false>(SL, SR, make_gas_q(l[0]), near2, tau, eps, F, I, eps, -1.0, &code));
+    const bool done = in && (dir == 0 ? flux_split_q<0, false>(SL, SR, make_gas_q(l[0]), near2, tau, eps, F, I, eps, -1.0, &code, powtab::TAB)
+                                      : flux_split_q<1, false>(SL, SR, make_gas_q(l[0]), near2, tau, eps, F, I, eps, -1.0, &code, powtab::TAB));
     if (!done)
         code = dir == 0 ? flux_ieee<0>(l, r, tau, eps, F, I) : flux_ieee<1>(l, r, tau, eps, F, I);
     double *o = out + (size_t)k * 9;

@@ -30,7 +30,8 @@ __global__ void __launch_bounds__(64 * W, MINW) sweep_x_rows_kernel(SweepArgs a)
     __shared__ double xf[W][4][64];   // fluxes
     __shared__ double xi[W][4][64];   // interface values at t + tau
     __shared__ double xe[W][64];      // E of the owned cell (read back for the update)
-    line_sweep<0, W, NM>(a, KernargArgs{}, blockIdx.x, blockIdx.y, xa, xb, xf, xi, xe);
+    __shared__ double tab[POW_TAB];
+    line_sweep<0, W, NM>(a, KernargArgs{}, blockIdx.x, blockIdx.y, xa, xb, xf, xi, xe, tab);
 }
 
 // X sweep walking K chunks of W cell rows per block (line_sweep with K > 1).
@@ -42,9 +43,10 @@ __global__ void __launch_bounds__(64 * W, MINW) sweep_x_chunks_kernel(SweepArgs 
     __shared__ double xf[W][4][64];
     __shared__ double xi[W][4][64];
     __shared__ double xe[W][64];
-    __shared__ double xc[2][8][64];   // the last face of the previous chunk: F, I
+    __shared__ double xc[8][64];      // the last face of the previous chunk: F, I
+    __shared__ double tab[POW_TAB];
     (void)a;                          // read through KernargArgs, chunk by chunk
-    line_sweep_chunks<0, W, NM, K>(KernargArgs{}, blockIdx.x, blockIdx.y, xa, xb, xf, xi, xe, xc);
+    line_sweep_chunks<0, W, NM, K>(KernargArgs{}, blockIdx.x, blockIdx.y, xa, xb, xf, xi, xe, xc, tab);
 }
 
 // Y sweep (y_sweep): blocks of 4 waves, wave index = global wave number.
@@ -54,9 +56,10 @@ __global__ void __launch_bounds__(256, MINW) sweep_y_kernel(SweepArgs a, int chu
     constexpr bool LEARNED = NM == NM_LEARNED;
     __shared__ uint32_t mlp_lds[LEARNED ? 4 : 1][LEARNED ? 64 * 8 : 1];
     __shared__ double stash[4][5][64];   // each wave's cell values and E, read back for the update
+    __shared__ double tab[POW_TAB];
     const int wv = (threadIdx.x >> 6) & 3;
     const long wave = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    y_sweep<MINW, NM, G>(a, KernargArgs{}, wave, chunks, stash[wv], mlp_lds[wv]);
+    y_sweep<MINW, NM, G>(a, KernargArgs{}, wave, chunks, stash[wv], mlp_lds[wv], tab);
 }
 
 // min over cells of min(h_x, h_y) / (|c| + |u| + |v|)  (grp_solver_2D_split_EUL_source.c:185-191).

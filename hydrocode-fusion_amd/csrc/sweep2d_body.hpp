@@ -199,10 +199,12 @@ __device__ __attribute__((noinline)) int redo_face(const SweepArgs *ap, int line
 // argument block again (see reload_args).
 template <int DIR, int NM, int MINW, class Src>
 __device__ __forceinline__ void solve_interface(const SweepArgs &a, const Src &src, const Side &SL, const Side &SR,
-                                                int line, int f, double F[4], double I[4], double p_guess = -1.0)
+                                                int line, int f, double F[4], double I[4], const double *tab,
+                                                double p_guess = -1.0)
 {
     int code = ifvar_bad(SL, SR, a.eps) ? 1 : 0, bad = 0;
-    const bool done = flux_split_q<DIR, NM != NM_REF>(SL, SR, a.gas, a.near2, a.tau, a.eps, F, I, a.tol, p_guess, &bad);
+    const bool done = flux_split_q<DIR, NM != NM_REF>(SL, SR, a.gas, a.near2, a.tau, a.eps, F, I, a.tol, p_guess, &bad,
+                                                   tab);
     if (__builtin_expect(__any(!done), 0)) {
         if (!done) {
             const SweepArgs ar = src.get();
@@ -252,9 +254,9 @@ __device__ __forceinline__ double interface_guess(const SweepArgs &a, bool activ
 // c0 - 1 + w (w = 0 .. W-1) of the 64 lines of group bx.  Wave w solves the
 // face right of its cell; waves 1 .. W-1 update their cells with the face left
 // of them, and wave 0 too when `carried` (with the face the previous chunk's
-// last wave left in xc[(k - 1) & 1]); with `carry` the last wave leaves its
-// face in xc[k & 1].  Returns false when the sweep is halted (only checked
-// with `first`).
+// last wave left in xf and xi, which wave 0 keeps in xc).  tab: the pow tables,
+// filled in the `first` chunk.  Returns false when the sweep is halted (only
+// checked with `first`).
 // lane, w: the thread's lane and wave (threadIdx.x & 63, threadIdx.x >> 6).
 // The global loads of a chunk for the thread's own cell c = c0 - 1 + w: its
 // values, previous slopes and E.
@@ -282,10 +284,10 @@ __device__ __forceinline__ void chunk_loads(const SweepArgs &a, int lane, int w,
 }
 
 template <int DIR, int W, int NM, class Src>
-__device__ __forceinline__ bool line_chunk(const SweepArgs &a, const Src &src, int lane, int w, int bx, int c0, int k,
-                                          bool first, bool carried, bool carry, double (*xa)[4][64],
+__device__ __forceinline__ bool line_chunk(const SweepArgs &a, const Src &src, int lane, int w, int bx, int c0, bool first,
+                                          bool carried, double (*xa)[4][64],
                                           double (*xb)[4][64], double (*xf)[4][64], double (*xi)[4][64],
-                                          double (*xe)[64], double (*xc)[8][64])
+                                          double (*xe)[64], double (*xc)[64], double *tab)
 {
     const int line = bx * 64 + lane;
     const bool col = line < (DIR == 0 ? a.n : a.m);
@@ -296,7 +298,7 @@ __device__ __forceinline__ bool line_chunk(const SweepArgs &a, const Src &src, i
 
     // every global load of the chunk up front, before the first LDS store:
     // the owned cell's values, previous slopes and E, then the end waves'
-    // extra cells
+    // extra cells, and in the first chunk the pow tables
     const bool own = col && c >= 0 && c < m;
     double v[4], vl[4], vr[4], sp[4], e_c;
     {
@@ -314,6 +316,14 @@ __device__ __forceinline__ bool line_chunk(const SweepArgs &a, const Src &src, i
         L.value(c + 2, vrr);
         L.prev_slopes(c + 1, sp1);
     }
+    if (first) {
+        TabLoad<64 * W> t;
+        t.load(w * 64 + lane);
+        t.store(w * 64 + lane, tab);
+    }
+    if (carried && w == 0)                        // the face on its left, before the last wave writes its next one
+#pragma unroll
+        for (int q = 0; q < 4; ++q) { xc[q][lane] = xf[W - 1][q][lane]; xc[4 + q][lane] = xi[W - 1][q][lane]; }
 #pragma unroll
     for (int q = 0; q < 4; ++q) xa[w][q][lane] = v[q];
     xe[w][lane] = e_c;
@@ -362,13 +372,10 @@ __device__ __forceinline__ bool line_chunk(const SweepArgs &a, const Src &src, i
         // none of it is held across the solve
         const Side SL = recon(v, s, hh, true);
         const Side SR = recon(vr, sr, hh, false);
-        solve_interface<DIR, NM, 4>(src.get(), src, SL, SR, line, f, F, I, pg);
+        solve_interface<DIR, NM, 4>(src.get(), src, SL, SR, line, f, F, I, tab, pg);
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q) { xf[w][q][lane] = F[q]; xi[w][q][lane] = I[q]; }
-    if (carry && w == W - 1)                      // the next chunk's first face
-#pragma unroll
-        for (int q = 0; q < 4; ++q) { xc[k & 1][q][lane] = F[q]; xc[k & 1][4 + q][lane] = I[q]; }
     __syncthreads();
     if (own && (w >= 1 || carried)) {
         // the cell's values and E come back from LDS, so no register holds them across the solve
@@ -380,7 +387,7 @@ __device__ __forceinline__ bool line_chunk(const SweepArgs &a, const Src &src, i
             for (int q = 0; q < 4; ++q) { Fl[q] = xf[w - 1][q][lane]; Il[q] = xi[w - 1][q][lane]; }
         } else {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) { Fl[q] = xc[(k - 1) & 1][q][lane]; Il[q] = xc[(k - 1) & 1][4 + q][lane]; }
+            for (int q = 0; q < 4; ++q) { Fl[q] = xc[q][lane]; Il[q] = xc[4 + q][lane]; }
         }
 #pragma unroll
         for (int q = 0; q < 4; ++q) vc[q] = xa[w][q][lane];
@@ -395,26 +402,28 @@ __device__ __forceinline__ bool line_chunk(const SweepArgs &a, const Src &src, i
 template <int DIR, int W, int NM, class Src>
 __device__ __forceinline__ void line_sweep(const SweepArgs &a, const Src &src, int bx, int by, double (*xa)[4][64],
                                            double (*xb)[4][64], double (*xf)[4][64], double (*xi)[4][64],
-                                           double (*xe)[64])
+                                           double (*xe)[64], double *tab)
 {
-    (void)line_chunk<DIR, W, NM>(a, src, threadIdx.x & 63, threadIdx.x >> 6, bx, by * (W - 1), 0, true, false, false,
-                                 xa, xb, xf, xi, xe, nullptr);
+    (void)line_chunk<DIR, W, NM>(a, src, threadIdx.x & 63, threadIdx.x >> 6, bx, by * (W - 1), true, false, xa, xb, xf,
+                                 xi, xe, nullptr, tab);
 }
 
 // The same walking K chunks of W cells along the block's lines (by (K W - 1)
 // onwards): the first chunk's wave 0 is the halo cell as above, and in every
 // later chunk wave 0 updates its cell too, with the face that the previous
-// chunk's last wave solved (xc, double-buffered); a block then solves K W faces
-// for K W - 1 cells instead of W for W - 1.  Every LDS slot a chunk writes before
-// its first barrier is read by the previous chunk only before that chunk's last
-// barrier, so the chunks need no barrier between them.  The argument block is
+// chunk's last wave solved (wave 0 moves it to xc before the first barrier; the
+// last wave writes xf and xi again only after the second); a block then solves
+// K W faces for K W - 1 cells instead of W for W - 1.  What the other waves write
+// before a chunk's first barrier, the previous chunk reads only before its last
+// one, so the chunks need no barrier between them.  With the pow tables a block
+// takes 77 KiB of LDS: two still fit a CU.  The argument block is
 // read again for each chunk, and the lane and wave indices pass through an
 // empty asm each time, so that neither the arguments nor the LDS addresses
 // derived from them are held across the chunks' solves.
 template <int DIR, int W, int NM, int K, class Src>
 __device__ __forceinline__ void line_sweep_chunks(const Src &src, int bx, int by, double (*xa)[4][64],
                                                   double (*xb)[4][64], double (*xf)[4][64], double (*xi)[4][64],
-                                                  double (*xe)[64], double (*xc)[8][64])
+                                                  double (*xe)[64], double (*xc)[64], double *tab)
 {
     const int s0 = by * (K * W - 1);
     for (int k = 0; k < K; ++k) {
@@ -425,7 +434,7 @@ __device__ __forceinline__ void line_sweep_chunks(const Src &src, int bx, int by
         int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         __asm__ volatile("" : "+v"(lane));
         __asm__ volatile("" : "+s"(w));
-        if (!line_chunk<DIR, W, NM>(a, src, lane, w, bx, c0, k, k == 0, k > 0, k + 1 < K, xa, xb, xf, xi, xe, xc))
+        if (!line_chunk<DIR, W, NM>(a, src, lane, w, bx, c0, k == 0, k > 0, xa, xb, xf, xi, xe, xc, tab))
             return;
     }
 }
@@ -436,18 +445,17 @@ __device__ __forceinline__ void line_sweep_chunks(const Src &src, int bx, int by
 // smaller G stacks rows, so that a front lying along y (constant i) meets
 // fewer waves, each with more lanes on it.
 // wave: the wave's index in the grid's sweep (a group of 64/G rows, one run
-// of G - 1 cells); st, mlp: this wave's LDS slots; src gives the argument
-// block again after the solve.
+// of G - 1 cells); st, mlp: this wave's LDS slots; tab: the block's, for the
+// pow tables; src gives the argument block again after the solve.
 template <int MINW, int NM, int G, class Src>
 __device__ __forceinline__ void y_sweep(const SweepArgs &a, const Src &src, long wave, int chunks,
-                                        double (*st)[64], uint32_t *mlp)
+                                        double (*st)[64], uint32_t *mlp, double *tab)
 {
     static_assert(G == 64 || G == 32 || G == 16 || G == 8, "lanes per row");
     constexpr int ROWS = 64 / G;
     constexpr bool LEARNED = NM == NM_LEARNED;
     const int lane = threadIdx.x & 63, k = lane % G;
     const int jg = (int)(wave / chunks);
-    if (jg * ROWS >= a.m) return;                      // uniform per wave
     const int j = jg * ROWS + lane / G;
     const bool rowv = j < a.m;
     const int c0 = (int)(wave % chunks) * (G - 1);
@@ -477,8 +485,14 @@ __device__ __forceinline__ void y_sweep(const SweepArgs &a, const Src &src, long
         L.value(c + 2, wrr);
         L.prev_slopes(c + 1, sp1);
     }
-    // the predecessor's status is read while the loads above are in flight
+    TabLoad<256> t;
+    t.load(threadIdx.x);
+    // the predecessor's status is read while the loads above are in flight; the
+    // whole block returns together
     if (sweep_halted(a)) return;
+    t.store(threadIdx.x, tab);
+    __syncthreads();
+    if (jg * ROWS >= a.m) return;                      // uniform per wave
     // each lane reads back only its own slots: no barrier needed
 #pragma unroll
     for (int q = 0; q < 4; ++q) st[q][lane] = w[q];
@@ -525,7 +539,7 @@ __device__ __forceinline__ void y_sweep(const SweepArgs &a, const Src &src, long
         // none of it is held across the solve
         const Side SL = recon(w, s, hh, true);
         const Side SR = recon(wr, sr, hh, false);
-        solve_interface<1, NM, MINW>(src.get(), src, SL, SR, j, f, F, I, pg);
+        solve_interface<1, NM, MINW>(src.get(), src, SL, SR, j, f, F, I, tab, pg);
     }
     double Fl[4], Il[4];
 #pragma unroll

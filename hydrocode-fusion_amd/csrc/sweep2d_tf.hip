@@ -186,7 +186,7 @@ __device__ __attribute__((noinline)) int redo_face_tf(const SweepArgs *ap, int l
 template <int DIR, int NM>
 __device__ __forceinline__ void solve_interface_tf(const SweepArgs &a, const double wl[NQ], const double sl[NQ],
                                                    const double wr[NQ], const double sr[NQ], int line, int f, double F[4],
-                                                   double I[4], double Z[3], double p_guess = -1.0)
+                                                   double I[4], double Z[3], const double *tab, double p_guess = -1.0)
 {
     Side SL, SR;
     double FA[4];
@@ -194,7 +194,7 @@ __device__ __forceinline__ void solve_interface_tf(const SweepArgs &a, const dou
     recon_tf(wr, sr, a.hh, false, SR, FA[2], FA[3]);
     int code = ifvar_bad(SL, SR, a.eps) ? 1 : 0, bad = 0;
     const bool done = flux_two_fluid_q<DIR, NM != NM_REF>(SL, SR, a.two, FA, a.near2, a.tau, a.eps, F, I, Z, a.tol,
-                                                          p_guess, &bad);
+                                                          p_guess, &bad, tab);
     if (__builtin_expect(__any(!done), 0)) {
         if (!done) {
             const SweepArgs ar = reload_args<SweepArgs>();
@@ -259,6 +259,7 @@ __global__ void __launch_bounds__(64 * W, (W + 3) / 4) sweep_x_tf_kernel(SweepAr
     __shared__ double xz[W][3][64];    // u_n a, u_n at t + tau/2; a at t + tau
     __shared__ double xi[W][4][64];    // interface values at t + tau
     __shared__ double xe[W][64];       // E of the owned row
+    __shared__ double tab[POW_TAB];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int i = blockIdx.x * 64 + lane;
     const bool col = i < a.n;
@@ -284,6 +285,9 @@ __global__ void __launch_bounds__(64 * W, (W + 3) / 4) sweep_x_tf_kernel(SweepAr
         L.value(c + 2, vrr);
         L.prev_slopes(c + 1, sp1);
     }
+    TabLoad<64 * W> tl;
+    tl.load(threadIdx.x);
+    tl.store(threadIdx.x, tab);
 #pragma unroll
     for (int q = 0; q < NQ; ++q) xa[w][q][lane] = v[q];
     xe[w][lane] = e_c;
@@ -323,7 +327,7 @@ __global__ void __launch_bounds__(64 * W, (W + 3) / 4) sweep_x_tf_kernel(SweepAr
     if constexpr (LEARNED)   // xf[w] is not written before the solve: it holds the network inputs
         pg = interface_guess_tf<0>(a, col && f <= m, v, s, vr, sr, (uint32_t *)&xf[w][0][0]);
     if (col && f <= m)
-        solve_interface_tf<0, NM>(a, v, s, vr, sr, i, f, F, I, Z, pg);
+        solve_interface_tf<0, NM>(a, v, s, vr, sr, i, f, F, I, Z, tab, pg);
 #pragma unroll
     for (int q = 0; q < 4; ++q) { xf[w][q][lane] = F[q]; xi[w][q][lane] = I[q]; }
 #pragma unroll
@@ -352,10 +356,10 @@ __global__ void __launch_bounds__(256, 3) sweep_y_tf_kernel(SweepArgs a, int chu
     constexpr int ROWS = 64 / G;
     __shared__ double stash[4][NQ + 1][64];
     __shared__ uint32_t mlp_lds[LEARNED ? 4 : 1][LEARNED ? 64 * 8 : 1];
+    __shared__ double tab[POW_TAB];
     const int lane = threadIdx.x & 63, k = lane % G;
     const long wave = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const int jg = (int)(wave / chunks);
-    if (jg * ROWS >= a.m) return;
     const int j = jg * ROWS + lane / G;
     const bool rowv = j < a.m;
     const int c0 = (int)(wave % chunks) * (G - 1);
@@ -379,8 +383,14 @@ __global__ void __launch_bounds__(256, 3) sweep_y_tf_kernel(SweepArgs a, int chu
         L.value(c + 2, wrr);
         L.prev_slopes(c + 1, sp1);
     }
-    // the predecessor's status is read while the loads above are in flight
+    TabLoad<256> tl;
+    tl.load(threadIdx.x);
+    // the predecessor's status is read while the loads above are in flight; the
+    // whole block returns together
     if (tf_halted(a)) return;
+    tl.store(threadIdx.x, tab);
+    __syncthreads();
+    if (jg * ROWS >= a.m) return;
     double(*st)[64] = stash[(threadIdx.x >> 6) & 3];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) st[q][lane] = w[q];
@@ -417,7 +427,7 @@ __global__ void __launch_bounds__(256, 3) sweep_y_tf_kernel(SweepArgs a, int chu
     double pg = -1.0;
     if constexpr (LEARNED) pg = interface_guess_tf<1>(a, face, w, s, wr, sr, mlp_lds[(threadIdx.x >> 6) & 3]);
     if (face)
-        solve_interface_tf<1, NM>(a, w, s, wr, sr, j, f, F, I, Z, pg);
+        solve_interface_tf<1, NM>(a, w, s, wr, sr, j, f, F, I, Z, tab, pg);
     double Fl[4], Il[4], Zl[3];
 #pragma unroll
     for (int q = 0; q < 4; ++q) { Fl[q] = __shfl_up(F[q], 1); Il[q] = __shfl_up(I[q], 1); }

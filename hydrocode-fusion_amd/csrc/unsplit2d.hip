@@ -169,15 +169,15 @@ __device__ __attribute__((noinline)) int redo_face_t(const UnsplitArgs *ap, int 
 template <int NM, bool G2>
 __device__ __forceinline__ void solve_t(const UnsplitArgs &a, int dir, const Side &SL, const Side &SR,
                                         const double TL[4], const double TR[4], int c, int ci, double F[4], double I[4],
-                                        double p_guess)
+                                        double p_guess, const double *tab)
 {
     int code = ifvar_bad_t(SL, SR, TL, TR, a.eps) ? 1 : 0, bad = 0;
     const double n_x = dir ? 0.0 : 1.0, n_y = dir ? 1.0 : 0.0;
     if constexpr (G2) {
-        bad = grp_2d_flux_g2d<NM != NM_REF>(SL, SR, TL, TR, a.gas, n_x, n_y, a.tau, a.eps, F, I, a.tol, p_guess);
+        bad = grp_2d_flux_g2d<NM != NM_REF>(SL, SR, TL, TR, a.gas, n_x, n_y, a.tau, a.eps, F, I, a.tol, p_guess, tab);
     } else {
         const bool done = flux_transversal_q<NM != NM_REF>(SL, SR, TL, TR, a.gas, dir, a.near2, a.tau, a.eps, F, I, a.tol,
-                                                           p_guess, &bad);
+                                                           p_guess, &bad, tab);
         if (__builtin_expect(__any(!done), 0)) {
             if (!done) {
                 const UnsplitArgs ar = reload_args<UnsplitArgs>();
@@ -224,8 +224,9 @@ template <int W, int NM, bool G2>
 __device__ __forceinline__ void unsplit_step_body(const UnsplitArgs &a)
 {
     __shared__ double sd[W][12][64];     // side data of row c: value, x-slope, y-slope
-    __shared__ double fx[W - 1][8][64];  // x-interface c+1: flux, values at t + tau
+    __shared__ double fx[W - 1][8][62];  // x-interface c+1 of lanes 1..62: flux, values at t + tau
     __shared__ double gy[W - 2][8][64];  // y-interfaces of the updated rows: flux, values at t + tau
+    __shared__ double tab[POW_TAB];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int m = a.m, n = a.n;
     const int i0 = blockIdx.x * 62, ci = i0 - 1 + lane;
@@ -234,6 +235,9 @@ __device__ __forceinline__ void unsplit_step_body(const UnsplitArgs &a)
     const bool xin = c >= 0 && c < m, yin = ci >= 0 && ci < n;
     {
         double v[4] = {1.0, 0.0, 0.0, 1.0}, s[4] = {0.0, 0.0, 0.0, 0.0}, t[4] = {0.0, 0.0, 0.0, 0.0};
+        TabLoad<64 * W> tl;
+        tl.load(threadIdx.x);
+        tl.store(threadIdx.x, tab);
         if (c <= m && ci <= n && (xin || yin)) G.side(c, ci, v, s, t);   // a cell or a ghost, not a corner
 #pragma unroll
         for (int q = 0; q < 4; ++q) { sd[w][q][lane] = v[q]; sd[w][4 + q][lane] = s[q]; sd[w][8 + q][lane] = t[q]; }
@@ -295,11 +299,11 @@ __device__ __forceinline__ void unsplit_step_body(const UnsplitArgs &a)
         // the argument block is read again for the solve, so no scalar register holds it across
         if (active) {
             sides();
-            solve_t<NM, G2>(reload_args<UnsplitArgs>(), dir, SL, SR, TL, TR, dir ? yc : c, dir ? ycell : ci, F, I, pg);
+            solve_t<NM, G2>(reload_args<UnsplitArgs>(), dir, SL, SR, TL, TR, dir ? yc : c, dir ? ycell : ci, F, I, pg, tab);
         }
-        if (dir == 0 && w <= W - 2) {
+        if (dir == 0 && w <= W - 2 && lane >= 1 && lane <= 62) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) { fx[w][q][lane] = F[q]; fx[w][4 + q][lane] = I[q]; }
+            for (int q = 0; q < 4; ++q) { fx[w][q][lane - 1] = F[q]; fx[w][4 + q][lane - 1] = I[q]; }
         }
         if (dir == 1 && w >= 1 && w <= W - 2) {
 #pragma unroll
@@ -317,8 +321,8 @@ __device__ __forceinline__ void unsplit_step_body(const UnsplitArgs &a)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             vc[q] = sd[w][q][lane];
-            Fl[q] = fx[w - 1][q][lane]; Ixl[q] = fx[w - 1][4 + q][lane];
-            Fr[q] = fx[w][q][lane];     Ixr[q] = fx[w][4 + q][lane];
+            Fl[q] = fx[w - 1][q][lane - 1]; Ixl[q] = fx[w - 1][4 + q][lane - 1];
+            Fr[q] = fx[w][q][lane - 1];     Ixr[q] = fx[w][4 + q][lane - 1];
             Gl[q] = gy[w - 1][q][lane - 1]; Iyl[q] = gy[w - 1][4 + q][lane - 1];
             Gy[q] = gy[w - 1][q][lane];     Iy[q] = gy[w - 1][4 + q][lane];
         }
@@ -370,6 +374,7 @@ __device__ __forceinline__ void unsplit_strip_body(const UnsplitArgs &a, int R)
     __shared__ double fl[8][64];       // x-interface r: flux, values at t + tau
     __shared__ double gb[8][64];       // y-interfaces of row r: flux, values at t + tau
     __shared__ uint32_t mlp_lds[NM == NM_LEARNED ? 64 * 8 : 1];   // network inputs
+    __shared__ double tab[POW_TAB];
     if (a.prev != nullptr) {
         const SweepStatus p0 = a.prev[0], p1 = a.prev[1];
         if (p0.fail_key != 0ull || p0.flags != 0u || p1.fail_key != 0ull) {
@@ -392,6 +397,9 @@ __device__ __forceinline__ void unsplit_strip_body(const UnsplitArgs &a, int R)
 #pragma unroll
         for (int q = 0; q < 4; ++q) { sd[buf][q][lane] = v[q]; sd[buf][4 + q][lane] = s[q]; sd[buf][8 + q][lane] = t[q]; }
     };
+    TabLoad<64> tl;
+    tl.load(lane);
+    tl.store(lane, tab);
     int cb = 0;
     put_side(cb, r0 - 1);
 #pragma unroll 1
@@ -433,7 +441,7 @@ __device__ __forceinline__ void unsplit_strip_body(const UnsplitArgs &a, int R)
             }
             double Fo[4] = {0.0, 0.0, 0.0, 0.0}, Io[4] = {0.0, 0.0, 0.0, 0.0};
             const double pg = unsplit_guess<NM>(a, active, 1 - pass, SL, SR, mlp_lds);
-            if (active) solve_t<NM, G2>(reload_args<UnsplitArgs>(), 1 - pass, SL, SR, TL, TR, r, ci, Fo, Io, pg);
+            if (active) solve_t<NM, G2>(reload_args<UnsplitArgs>(), 1 - pass, SL, SR, TL, TR, r, ci, Fo, Io, pg, tab);
             if (pass == 0) {
 #pragma unroll
                 for (int q = 0; q < 4; ++q) { gb[q][lane] = Fo[q]; gb[4 + q][lane] = Io[q]; }
@@ -497,8 +505,8 @@ __global__ void __launch_bounds__(64, 2) unsplit_strip_g2d_kernel(UnsplitArgs a,
 // Two forms: the tile (TILE_W waves, TILE_W - 2 updated rows per block) and the
 // strip (one wave per block walking down its rows).  The context picks one
 // (hgrp2d_set_unsplit_form, hgrp2d_tune) or takes the default (form 0: the tile).
-// The tile is 12 waves tall: 156 KiB of LDS (140 with the learned guess, whose
-// y results then share the side data's slots), one block per CU, 168 VGPRs
+// The tile is 12 waves tall: 160 KiB of LDS (with the pow tables; the network
+// inputs lie in the x results' slots), one block per CU, 168 VGPRs
 // (15-18 spilled; 39-77 in the G2D and learned forms) for 3 waves per SIMD.
 // Against 8 waves (6 rows, 100 KiB, 192 VGPRs, 2 waves per SIMD) its halo rows
 // are 1 in 6 instead of 1 in 4: at 1024^2 the whole run takes 602 instead of

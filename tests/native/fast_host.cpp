@@ -19,7 +19,7 @@ static int both(const double *l, const double *r, double tau, double eps, double
     ieee[0] = grp_2d_flux<DIR, CONV>(a, b, G, tau, eps, F, I, tol, guess);
     for (int q = 0; q < 4; ++q) { ieee[1 + q] = F[q]; ieee[5 + q] = I[q]; }
     int code = 0;
-    if (!flux_split_q<DIR, CONV>(a, b, G, near_threshold(eps), tau, eps, F, I, tol, guess, &code)) return 0;
+    if (!flux_split_q<DIR, CONV>(a, b, G, near_threshold(eps), tau, eps, F, I, tol, guess, &code, powtab::TAB)) return 0;
     fast[0] = code;
     for (int q = 0; q < 4; ++q) { fast[1 + q] = F[q]; fast[5 + q] = I[q]; }
     return 1;
@@ -54,7 +54,7 @@ extern "C" int fh_transversal_many(const double *L, const double *R, int n, doub
         o[0] = grp_2d_flux_n(a, b, l + 11, r + 11, G, dir ? 0.0 : 1.0, dir ? 1.0 : 0.0, tau, eps, o + 1, o + 5, eps);
         int code = 0;
         if (!flux_transversal_q<false>(a, b, l + 11, r + 11, G, dir, near_threshold(eps), tau, eps, f + 1, f + 5, eps, -1.0,
-                                       &code)) {
+                                       &code, powtab::TAB)) {
             f[0] = NAN;
             continue;
         }
@@ -80,10 +80,12 @@ extern "C" int fh_two_fluid_many(const double *L, const double *R, const double 
         bool ok;
         if (dir == 0) {
             o[0] = grp_2d_flux_tf<0, true>(a, b, T, fa, tau, eps, o + 1, o + 5, o + 9, 1e-12);
-            ok = flux_two_fluid_q<0, true>(a, b, T, fa, near_threshold(eps), tau, eps, f + 1, f + 5, f + 9, 1e-12, -1.0, &code);
+            ok = flux_two_fluid_q<0, true>(a, b, T, fa, near_threshold(eps), tau, eps, f + 1, f + 5, f + 9, 1e-12, -1.0, &code,
+                                             powtab::TAB);
         } else {
             o[0] = grp_2d_flux_tf<1, true>(a, b, T, fa, tau, eps, o + 1, o + 5, o + 9, 1e-12);
-            ok = flux_two_fluid_q<1, true>(a, b, T, fa, near_threshold(eps), tau, eps, f + 1, f + 5, f + 9, 1e-12, -1.0, &code);
+            ok = flux_two_fluid_q<1, true>(a, b, T, fa, near_threshold(eps), tau, eps, f + 1, f + 5, f + 9, 1e-12, -1.0, &code,
+                                             powtab::TAB);
         }
         f[0] = ok ? code : NAN;
         took += ok;
@@ -104,7 +106,7 @@ extern "C" int fh_edir_many(const double *L, const double *R, int n, double eps,
         const Rcp rL = rcp_of(a.rho), rR = rcp_of(b.rho);
         if (sides1_in_range(a, b) &&
             grp_edir_q(f, f + 3, a, b, rL, rR, sqrt_q(div_q(G.g * a.p, rL)), sqrt_q(div_q(G.g * b.p, rR)), G,
-                       near_threshold(eps), eps))
+                       near_threshold(eps), eps, powtab::TAB))
             ++took;
         else
             for (int q = 0; q < 6; ++q) f[q] = o[q];
