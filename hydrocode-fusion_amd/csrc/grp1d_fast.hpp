@@ -109,12 +109,13 @@ HGRP_HD bool grp_edir_q(double D[3], double U[3], const Side1 &L, const Side1 &R
     const bool rough = any_lane(tiny(L.u) || tiny(R.u) || tiny(L.s_u) || tiny(R.s_u));
     const Rcp pL = rcp_of(L.p), pR = rcp_of(R.p);
     StarQ st;
-    if (!riemann_q<false, 50>(G, G, L.u, R.u, pL, pR, c_L, c_R, eps, eps, -1.0, st, P)) return false;
+    Keep wL, wR;
+    if (!riemann_q<false, 50>(G, G, L.u, R.u, pL, pR, c_L, c_R, eps, eps, -1.0, st, wL, wR, P)) return false;
     const double u = st.u, p = st.p, z = G.z;
     const double rs_L = p > L.p ? div_1(L.rho * (p + z * L.p), L.p + z * p)
-                                : L.rho * pow_in_range(log_in_range(div_q(p, pL), P), G.inv_g, P);
+                                : L.rho * pow_in_range(wL.m != 0.0 ? wL.l : log_in_range(div_q(p, pL), P), G.inv_g, P);
     const double rs_R = p > R.p ? div_1(R.rho * (p + z * R.p), R.p + z * p)
-                                : R.rho * pow_in_range(log_in_range(div_q(p, pR), P), G.inv_g, P);
+                                : R.rho * pow_in_range(wR.m != 0.0 ? wR.l : log_in_range(div_q(p, pR), P), G.inv_g, P);
     const Rcp qL = rcp_of(rs_L), qR = rcp_of(rs_R);
     const Rcp kL = rcp_of(sqrt_q(div_q(G.g * p, qL))), kR = rcp_of(sqrt_q(div_q(G.g * p, qR)));
     // shock speeds; where the density does not change by an ulp the quotient is IEEE's infinity or NaN

@@ -76,36 +76,43 @@ HGRP_HD double div_r(double a, const Rcp &r, bool rough) { return rough ? a / r.
 HGRP_HD bool gas_in_range(const Gas &G) { return G.gm1() >= 0x1p-20 && G.g <= 0x1p20; }
 
 // ---- the exact Riemann solve ---------------------------------------------------------
-// What the wave curve leaves for the Newton slope at the same pressure:
-// log(p/p_s) on the rarefaction branch, 1/sqrt(1 + nu (p - p_s)/p_s) in hi on
-// the shock branch.
+// What the wave curve leaves for the Newton slope at the same pressure and, from
+// the last one, for the state behind the wave: on the rarefaction branch
+// l = log(p/p_s) and m = (p/p_s)^mu; on the shock branch m = 0 and
+// l.hi = 1/sqrt(1 + nu (p - p_s)/p_s).
+struct Keep {
+    DD l;
+    double m;
+};
 template <int SIGN>
-HGRP_HD double curve_q(double p, double u_s, const Rcp &p_s, double c_s, const Gas &G, DD *keep, const double *P)
+HGRP_HD double curve_q(double p, double u_s, const Rcp &p_s, double c_s, const Gas &G, Keep *keep, const double *P)
 {
     double w;
     if (p > p_s.b) {
         const double dp = p - p_s.b;
         const Rcp s = sqrt_rcp(1.0 + div_q(G.nu * dp, p_s));
-        keep->hi = s.y;
+        keep->l.hi = s.y;
+        keep->m = 0.0;
         w = div_q(div_q(div_q(dp * c_s, {G.g, G.inv_g}), p_s), s);
     } else {
-        *keep = log_in_range(div_q(p, p_s), P);
-        w = pow_in_range(*keep, G.mu, P) - 1.0;
+        keep->l = log_in_range(div_q(p, p_s), P);
+        keep->m = pow_in_range(keep->l, G.mu, P);
+        w = keep->m - 1.0;
         w = div_q(2.0 * c_s * w, {G.gm1(), G.y_gm1});
     }
     return SIGN < 0 ? u_s - w : u_s + w;
 }
 
 // dv/dp along the 3-wave (the 1-wave's is its negative) at the pressure of the last curve_q
-HGRP_HD double slope_q(double p, const Rcp &p_s, double c_s, const Gas &G, const DD &keep, const double *P)
+HGRP_HD double slope_q(double p, const Rcp &p_s, double c_s, const Gas &G, const Keep &keep, const double *P)
 {
     const double t2 = div_q(div_q(c_s, {G.g, G.inv_g}), p_s);
     if (p > p_s.b) {
-        const double t1 = keep.hi;
+        const double t1 = keep.l.hi;
         const double t3 = div_q(0.5 * t2 * G.nu, p_s);
         return t2 * t1 - t3 * (p - p_s.b) * cube(t1);
     }
-    return recip_1(pow_in_range(keep, G.nu, P)) * t2;
+    return recip_1(pow_in_range(keep.l, G.nu, P)) * t2;
 }
 
 struct StarQ {
@@ -113,25 +120,18 @@ struct StarQ {
     int crw0, crw1;
 };
 
-// riemann_exact with at most N steps; false where the pressure leaves the range (or is not a number)
-template <bool CONV, int N = 500>
-HGRP_HD bool riemann_q(const Gas &GL, const Gas &GR, double u_L, double u_R, const Rcp &p_L, const Rcp &p_R,
-                       double c_L, double c_R, double eps, double tol, double p_guess, StarQ &out, const double *P)
+// The iteration: the star pressure p, the curves' velocities v_L and v_R at it,
+// the star velocity u.
+template <bool CONV, int N>
+HGRP_HD bool newton_q(const Gas &GL, const Gas &GR, double u_L, double u_R, const Rcp &p_L, const Rcp &p_R, double c_L,
+                      double c_R, double tol, double p_guess, double &p, double &v_L, double &v_R, double &u, Keep &kL,
+                      Keep &kR, const double *P)
 {
-    DD bL = {0.0, 0.0}, bR = {0.0, 0.0};
-    const double u_LR = curve_q<-1>(p_R.b, u_L, p_L, c_L, GL, &bL, P);
-    const double u_RL = curve_q<+1>(p_L.b, u_R, p_R, c_R, GR, &bR, P);
-    out.crw1 = (u_LR > u_R + eps) ? 0 : 1;
-    out.crw0 = (u_RL > u_L - eps) ? 1 : 0;
-    if (fabs(u_L - u_R) < tol && fabs(p_L.b - p_R.b) < tol) {
-        out.p = 0.5 * (p_L.b + p_R.b);
-        out.u = 0.5 * (u_L + u_R);
-        return true;
-    }
     // the states of riemann_exact's loop: 0 the curves at the learned guess, 1 steps from it,
     // 2 the curves at the reference's guess, 3 steps from it, 4 and 5 the converge rule's extra steps
     int st = p_guess > 0.0 ? 0 : 2, n = 0, done = 0;
-    double p = p_guess, v_L = 0.0, v_R = 0.0, k1 = 0.0, k3 = 0.0;
+    double k1 = 0.0, k3 = 0.0;
+    p = p_guess;
     for (;;) {
         if (st == 0 || st == 2) {
             k1 = div_q(div_q(-c_L, p_L), {GL.g, GL.inv_g});
@@ -142,14 +142,14 @@ HGRP_HD bool riemann_q(const Gas &GL, const Gas &GR, double u_L, double u_R, con
                 p = 0.5 * p0;
             }
         } else {
-            k1 = -slope_q(p, p_L, c_L, GL, bL, P);
-            k3 = slope_q(p, p_R, c_R, GR, bR, P);
+            k1 = -slope_q(p, p_L, c_L, GL, kL, P);
+            k3 = slope_q(p, p_R, c_R, GR, kR, P);
             const double p_new = p + div_1(v_R - v_L, k1 - k3);
             p = (p_new < 0.0) ? 0.5 * p : p_new;
         }
         if (__builtin_expect(!(p > 0x1p-300 && p < 0x1p300), 0)) return false;
-        v_L = curve_q<-1>(p, u_L, p_L, c_L, GL, &bL, P);
-        v_R = curve_q<+1>(p, u_R, p_R, c_R, GR, &bR, P);
+        v_L = curve_q<-1>(p, u_L, p_L, c_L, GL, &kL, P);
+        v_R = curve_q<+1>(p, u_R, p_R, c_R, GR, &kR, P);
         const double gap = fabs(v_L - v_R);
         if (st == 1 || st == 4) ++done;
         if (st == 3 || st == 5) ++n;
@@ -171,8 +171,72 @@ HGRP_HD bool riemann_q(const Gas &GL, const Gas &GR, double u_L, double u_R, con
             break;
         }
     }
-    out.p = p;
-    out.u = div_1(k1 * (v_R - v_L), k1 - k3) + v_L;
+    u = div_1(k1 * (v_R - v_L), k1 - k3) + v_L;
+    return true;
+}
+
+// Which of the waves are shocks, from the end of the Newton iteration: the
+// reference asks whether v_L(q) - v_R(q) =: g(q) exceeds eps at q = p_R (the
+// 3-wave) and p_L (the 1-wave), two more wave curves.  Here g(p) is known at the
+// last p.  Along either curve |v'| falls with the pressure, p |v'| rises (for
+// the rarefaction it is a power -nu > -1, for the shock its logarithmic slope
+// lies between -1 and -1/2), and |v'| = c/(gamma p) at the side's own pressure;
+// so between q and p the slope of g lies between A/pm and A/pn, where A sums
+// c/gamma over the sides, pm is the largest of the three pressures and pn the
+// smaller side's.  The margin M covers the rounding of the curves here and there
+// (pressure ratios up to 1024).  False where that does not decide: the curves do.
+// With the states behind the waves taken from the last curves (Keep) a step
+// goes, at 1024^2, from .374 to .355 ms, 4096^2 learned 4.54 -> 4.34, two fluids
+// 2048 x 512 .566 -> .522.
+struct WaveTest {
+    double A, M, g, p, pm, pn;
+};
+HGRP_HD bool wave_type(const WaveTest &w, double q, double eps, int &fan)
+{
+    const double d = w.p - q, t = d * w.A;
+    const bool shock = d > 0.0 && t + (w.g - eps - w.M) * w.pm > 0.0;
+    fan = !shock;
+    return shock || t + (w.g - eps + w.M) * (d > 0.0 ? w.pn : w.pm) < 0.0;
+}
+
+// riemann_exact with at most N steps; kL, kR: of the curves at the star pressure
+// (m = 0 where there is none).  False where the pressure leaves the range (or is
+// not a number).
+template <bool CONV, int N = 500>
+HGRP_HD bool riemann_q(const Gas &GL, const Gas &GR, double u_L, double u_R, const Rcp &p_L, const Rcp &p_R,
+                       double c_L, double c_R, double eps, double tol, double p_guess, StarQ &out, Keep &kL, Keep &kR,
+                       const double *P)
+{
+    const bool equal = fabs(u_L - u_R) < tol && fabs(p_L.b - p_R.b) < tol;
+    bool sure = false;
+    kL = kR = {{0.0, 0.0}, 0.0};
+    if (equal) {
+        out.p = 0.5 * (p_L.b + p_R.b);
+        out.u = 0.5 * (u_L + u_R);
+    } else {
+        double v_L = 0.0, v_R = 0.0, p;
+        if (!newton_q<CONV, N>(GL, GR, u_L, u_R, p_L, p_R, c_L, c_R, tol, p_guess, p, v_L, v_R, out.u, kL, kR, P))
+            return false;
+        out.p = p;
+        const double top = fmax(p_L.b, p_R.b);
+        WaveTest w;
+        w.pn = fmin(p_L.b, p_R.b);
+        w.pm = fmax(top, p);
+        w.p = p;
+        w.g = v_L - v_R;
+        w.A = c_L * GL.inv_g + c_R * GR.inv_g;
+        w.M = 0x1p-46 * (fabs(u_L) + fabs(u_R) + fabs(v_L) + fabs(v_R) + eps + c_L * (GL.y_gm1 + 64.0) +
+                         c_R * (GR.y_gm1 + 64.0));
+        const bool s0 = wave_type(w, p_L.b, eps, out.crw0), s1 = wave_type(w, p_R.b, eps, out.crw1);
+        sure = s0 && s1 && top <= 1024.0 * w.pn;
+    }
+    if (__builtin_expect(!sure, 0)) {
+        Keep t;
+        const double u_LR = curve_q<-1>(p_R.b, u_L, p_L, c_L, GL, &t, P);
+        const double u_RL = curve_q<+1>(p_L.b, u_R, p_R, c_R, GR, &t, P);
+        out.crw1 = (u_LR > u_R + eps) ? 0 : 1;
+        out.crw0 = (u_RL > u_L - eps) ? 1 : 0;
+    }
     return true;
 }
 
@@ -180,19 +244,22 @@ HGRP_HD bool riemann_q(const Gas &GL, const Gas &GR, double u_L, double u_R, con
 // The state behind a wave (rho and c next to the contact) and the speed of its
 // head.  SIGN -1: the 1-wave, +1: the 3-wave.
 template <int SIGN>
-HGRP_HD void behind_q(double rho, double u, const Rcp &p, double c, double p_star, int fan, const Gas &G, double &rs,
-                      double &cs, double &speed, const double *P)
+HGRP_HD void behind_q(double rho, double u, const Rcp &p, double c, double p_star, int fan, const Keep &k,
+                      const Gas &G, double &rs, double &cs, double &speed, const double *P)
 {
-    const double x = div_q(p_star, p);
     if (fan) {
-        const DD l = log_in_range(x, P);
-        rs = rho * pow_in_range(l, G.inv_g, P);
-        cs = c * pow_in_range(l, G.e_cs, P);
+        Keep a = k;
+        if (a.m == 0.0) {
+            a.l = log_in_range(div_q(p_star, p), P);
+            a.m = pow_in_range(a.l, G.mu, P);
+        }
+        rs = rho * pow_in_range(a.l, G.inv_g, P);
+        cs = c * a.m;                                     // e_cs is mu
         speed = SIGN < 0 ? u - c : u + c;
     } else {
         rs = div_1(rho * (p_star + G.z * p.b), p.b + G.z * p_star);
         cs = sqrt_q(div_1(G.g * p_star, rs));
-        const double s = c * sqrt_q(div_q(0.5 * (G.gp1() * x + G.gm1()), {G.g, G.inv_g}));
+        const double s = c * sqrt_q(div_q(0.5 * (G.gp1() * div_q(p_star, p) + G.gm1()), {G.g, G.inv_g}));
         speed = SIGN < 0 ? u - s : u + s;
     }
 }
@@ -291,9 +358,10 @@ HGRP_HD bool grp_q1d_q(double D[4], double U[4], const Side &L, const Side &R, c
     } else {
         rough = any_lane(tiny(L.u) || tiny(R.u) || tiny(L.d_u) || tiny(R.d_u));
         const Rcp pL = rcp_of(L.p), pR = rcp_of(R.p);
-        if (!riemann_q<CONV>(GL, GR, L.u, R.u, pL, pR, c_L, c_R, eps, tol, p_guess, st, P)) return false;
-        behind_q<-1>(L.rho, L.u, pL, c_L, st.p, st.crw0, GL, rs_L, cs_L, speed_L, P);
-        behind_q<+1>(R.rho, R.u, pR, c_R, st.p, st.crw1, GR, rs_R, cs_R, speed_R, P);
+        Keep kL, kR;
+        if (!riemann_q<CONV>(GL, GR, L.u, R.u, pL, pR, c_L, c_R, eps, tol, p_guess, st, kL, kR, P)) return false;
+        behind_q<-1>(L.rho, L.u, pL, c_L, st.p, st.crw0, kL, GL, rs_L, cs_L, speed_L, P);
+        behind_q<+1>(R.rho, R.u, pR, c_R, st.p, st.crw1, kR, GR, rs_R, cs_R, speed_R, P);
     }
     const double u_star = st.u, p_star = st.p;
 

@@ -54,6 +54,34 @@ def test_same_bits_as_the_ieee_solver(fast, gamma, direction, conv):
     assert np.array_equal(f[on], i[on])
 
 
+@pytest.mark.parametrize("gamma", [1.4, 1.05, 3.0])
+@pytest.mark.parametrize("conv", [0, 1])
+def test_waves_at_the_shock_threshold(fast, gamma, conv):
+    """One wave vanishes up to a few eps: the state on its far side lies on the
+    other wave's curve, moved by velocities around eps (the reference's
+    threshold between shock and rarefaction) and by none; strong and weak other
+    waves, pressure ratios past the bound of the estimate among them."""
+    n, rng = 20000, np.random.default_rng(5)
+    L, R = np.zeros((n, 15)), np.zeros((n, 15))
+    side = rng.random(n) < 0.5                                    # the wave that vanishes: the 3-wave, else the 1-wave
+    rho, p, u = rng.uniform(0.1, 3, n), rng.uniform(0.1, 3, n), rng.uniform(-1, 1, n)
+    x = np.where(rng.random(n) < 0.5, 10.0 ** rng.uniform(-2, 4, n), 1 + 10.0 ** rng.uniform(-9, -1, n) * rng.choice([-1, 1], n))
+    c = np.sqrt(gamma * p / rho)
+    shock = c / gamma * (x - 1) / np.sqrt(1 + (gamma + 1) / (2 * gamma) * np.maximum(x - 1, 0))
+    w = np.where(x > 1, shock, 2 * c / (gamma - 1) * (x ** ((gamma - 1) / (2 * gamma)) - 1))
+    off = 1e-9 * rng.choice([0, 1, -1, 0.999999, 1.000001], n) + rng.choice([0, 1e-15, 3e-10], n) * rng.uniform(-3, 3, n)
+    for A, own in ((L, side), (R, ~side)):
+        A[:, 0] = gamma
+        A[:, 3] = np.where(own, rho, rng.uniform(0.1, 3, n))
+        A[:, 6] = np.where(own, p, p * x)
+        A[:, 4] = np.where(own, u, np.where(side, u - w, u + w) + off)
+        A[:, 7:11] = rng.uniform(-1, 1, (n, 4))
+    took, f, i = _both(fast, L, R, 0, conv, np.full(n, -1.0))
+    on = ~np.isnan(f[:, 0])
+    assert took == on.sum() > 0.99 * n
+    assert np.array_equal(f[on], i[on])
+
+
 def _tails(n, seed, jump):
     """Interfaces ahead of a front: uniform pressure to within its rounding and
     velocities of every magnitude down to the denormals; `jump`: a contact too."""
