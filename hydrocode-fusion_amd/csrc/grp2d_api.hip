@@ -28,6 +28,7 @@ hipError_t launch_sweep_x(const SweepArgs &a, int variant, hipStream_t st);
 hipError_t launch_sweep_y(const SweepArgs &a, int variant, hipStream_t st);
 const char *sweep_kernel_name(int dir, int variant, int nm);
 int sweep_variants(int dir);
+int default_sweep(int dir, int m, int n);
 hipError_t launch_sweep_x_tf(const SweepArgs &a, hipStream_t st);
 const char *sweep_tf_kernel_name(int dir, int nm);
 hipError_t launch_sweep_y_tf(const SweepArgs &a, hipStream_t st);
@@ -103,6 +104,8 @@ extern "C" int hgrp2d_create(hgrp2d **out, int m, int n, const double *config)
     hgrp2d *c = (hgrp2d *)calloc(1, sizeof(hgrp2d));
     if (!c) return ARG_ERROR - 5;
     c->m = m; c->n = n; c->ld = (int)pitch_of(n);
+    c->xv = default_sweep(0, m, n);
+    c->yv = default_sweep(1, m, n);
     memcpy(c->cfg, config, sizeof c->cfg);
     const size_t cells = (size_t)m * c->ld;
     const size_t nb = (size_t)(2 * 5 + 2 * 4 + 2 * 4) * cells + 2 * (size_t)n * 4 + 2 * (size_t)m * 4;

@@ -112,36 +112,19 @@ struct BatchArgs {
     __device__ SweepArgs get() const { return batch_args(reload_args<BatchSweep>(), gi); }
 };
 
-template <int W, int MINW, int NM>
-__global__ void __launch_bounds__(64 * W, MINW) batch_x_kernel(BatchSweep b)
+// tile: grid, first wave of the block, waves along the fast direction
+template <int MINW, int NM, int G>
+__global__ void __launch_bounds__(256, MINW) batch_x_kernel(BatchSweep b)
 {
-    __shared__ double xa[W][4][64];
-    __shared__ double xb[W][4][64];
-    __shared__ double xf[W][4][64];
-    __shared__ double xi[W][4][64];
-    __shared__ double xe[W][64];
+    constexpr bool LEARNED = NM == NM_LEARNED;
+    __shared__ uint32_t mlp_lds[LEARNED ? 4 : 1][LEARNED ? 64 * 8 : 1];
+    __shared__ double stash[4][5][64];
     __shared__ double tab[POW_TAB];
     const int4 t = b.tiles[blockIdx.x];
     if (b.grids[t.x].halted) return;                    // the whole block
     const SweepArgs a = batch_args(b, t.x);
-    line_sweep<0, W, NM>(a, BatchArgs{t.x}, t.y, t.z, xa, xb, xf, xi, xe, tab);
-}
-
-// the X sweep walking K chunks of W rows per block (line_sweep_chunks): the
-// tile's row block is by (K W - 1) rows
-template <int W, int MINW, int NM, int K>
-__global__ void __launch_bounds__(64 * W, MINW) batch_x_chunks_kernel(BatchSweep b)
-{
-    __shared__ double xa[W][4][64];
-    __shared__ double xb[W][4][64];
-    __shared__ double xf[W][4][64];
-    __shared__ double xi[W][4][64];
-    __shared__ double xe[W][64];
-    __shared__ double xc[8][64];                        // the last face of the previous chunk: F, I
-    __shared__ double tab[POW_TAB];
-    const int4 t = b.tiles[blockIdx.x];
-    if (b.grids[t.x].halted) return;                    // the whole block
-    line_sweep_chunks<0, W, NM, K>(BatchArgs{t.x}, t.y, t.z, xa, xb, xf, xi, xe, xc, tab);
+    const int wv = (threadIdx.x >> 6) & 3;
+    wave_sweep<0, MINW, NM, G>(a, BatchArgs{t.x}, (long)t.y + wv, t.z, stash[wv], mlp_lds[wv], tab);
 }
 
 template <int MINW, int NM, int G>
@@ -151,29 +134,23 @@ __global__ void __launch_bounds__(256, MINW) batch_y_kernel(BatchSweep b)
     __shared__ uint32_t mlp_lds[LEARNED ? 4 : 1][LEARNED ? 64 * 8 : 1];
     __shared__ double stash[4][5][64];
     __shared__ double tab[POW_TAB];
-    const int4 t = b.tiles[blockIdx.x];                 // grid, first wave of the block, chunks per row group
+    const int4 t = b.tiles[blockIdx.x];
     if (b.grids[t.x].halted) return;
     const SweepArgs a = batch_args(b, t.x);
     const int wv = (threadIdx.x >> 6) & 3;
-    y_sweep<MINW, NM, G>(a, BatchArgs{t.x}, (long)t.y + wv, t.z, stash[wv], mlp_lds[wv], tab);
+    wave_sweep<1, MINW, NM, G>(a, BatchArgs{t.x}, (long)t.y + wv, t.z, stash[wv], mlp_lds[wv], tab);
 }
 
-// the one-grid launch variants (sweep2d.hip) X 0..4 and Y 0..4: X 0 = 8 rows
-// at 4 waves/SIMD, 1 = 8 rows at the compiler's budget, 2 = 16 rows, 3 and 4 =
-// 8 rows walking 4 and 8 chunks (31 and 63 rows per block); Y 0..4 = 16, 32,
-// 64, 8 lanes per row at 4 waves/SIMD, 64 at the compiler's budget
-static int x_cells_per_block(int v) { return v == 2 ? 15 : v == 3 ? 31 : v == 4 ? 63 : 7; }
-static int y_lanes_b(int v) { return v == 1 ? 32 : (v == 2 || v == 4) ? 64 : v == 3 ? 8 : 16; }
-
+// the one-grid launch variants (sweep_shape), X 0..4 and Y 0..4
 template <int NM>
 static void launch_bx(const BatchSweep &b, int v, int blocks, hipStream_t st)
 {
     switch (v) {
-    case 1: hipLaunchKernelGGL((batch_x_kernel<8, 1, NM>), dim3(blocks), dim3(512), 0, st, b); break;
-    case 2: hipLaunchKernelGGL((batch_x_kernel<16, 4, NM>), dim3(blocks), dim3(1024), 0, st, b); break;
-    case 3: hipLaunchKernelGGL((batch_x_chunks_kernel<8, 4, NM, 4>), dim3(blocks), dim3(512), 0, st, b); break;
-    case 4: hipLaunchKernelGGL((batch_x_chunks_kernel<8, 4, NM, 8>), dim3(blocks), dim3(512), 0, st, b); break;
-    default: hipLaunchKernelGGL((batch_x_kernel<8, 4, NM>), dim3(blocks), dim3(512), 0, st, b); break;
+    case 1: hipLaunchKernelGGL((batch_x_kernel<4, NM, 32>), dim3(blocks), dim3(256), 0, st, b); break;
+    case 2: hipLaunchKernelGGL((batch_x_kernel<4, NM, 8>), dim3(blocks), dim3(256), 0, st, b); break;
+    case 3: hipLaunchKernelGGL((batch_x_kernel<3, NM, 16>), dim3(blocks), dim3(256), 0, st, b); break;
+    case 4: hipLaunchKernelGGL((batch_x_kernel<3, NM, 8>), dim3(blocks), dim3(256), 0, st, b); break;
+    default: hipLaunchKernelGGL((batch_x_kernel<4, NM, 16>), dim3(blocks), dim3(256), 0, st, b); break;
     }
 }
 
@@ -184,7 +161,7 @@ static void launch_by(const BatchSweep &b, int v, int blocks, hipStream_t st)
     case 1: hipLaunchKernelGGL((batch_y_kernel<4, NM, 32>), dim3(blocks), dim3(256), 0, st, b); break;
     case 2: hipLaunchKernelGGL((batch_y_kernel<4, NM, 64>), dim3(blocks), dim3(256), 0, st, b); break;
     case 3: hipLaunchKernelGGL((batch_y_kernel<4, NM, 8>), dim3(blocks), dim3(256), 0, st, b); break;
-    case 4: hipLaunchKernelGGL((batch_y_kernel<1, NM, 64>), dim3(blocks), dim3(256), 0, st, b); break;
+    case 4: hipLaunchKernelGGL((batch_y_kernel<3, NM, 16>), dim3(blocks), dim3(256), 0, st, b); break;
     default: hipLaunchKernelGGL((batch_y_kernel<4, NM, 16>), dim3(blocks), dim3(256), 0, st, b); break;
     }
 }
@@ -434,16 +411,8 @@ static int build_tiles(hgrp2db *c, int dir, int v)
     pre.assign(1, 0);
     for (int r = 0; r < c->count; ++r) {
         const int i = c->order[r], m = c->m[i], n = c->n[i];
-        if (dir == 0) {
-            const int rows = x_cells_per_block(v);
-            for (int by = 0; by < (m + rows - 1) / rows; ++by)
-                for (int bx = 0; bx < (n + 63) / 64; ++bx) t.push_back(make_int4(i, bx, by, 0));
-        } else {
-            const int G = y_lanes_b(v), rows = 64 / G;
-            const int chunks = (n + G - 2) / (G - 1);
-            const long waves = (long)((m + rows - 1) / rows) * chunks;
-            for (long w = 0; w < waves; w += 4) t.push_back(make_int4(i, (int)w, chunks, 0));
-        }
+        const WaveGrid w = wave_grid(dir, m, n, sweep_shape(dir, v).G);
+        for (long k = 0; k < w.blocks; ++k) t.push_back(make_int4(i, (int)(4 * k), w.per_row, 0));
         pre.push_back((int)t.size());
     }
     BCHECK(hipMalloc((void **)&c->tiles_d[dir][v], std::max<size_t>(t.size(), 1) * sizeof(int4)));

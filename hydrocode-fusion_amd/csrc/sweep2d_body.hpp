@@ -238,230 +238,77 @@ __device__ __forceinline__ double interface_guess(const SweepArgs &a, bool activ
     return learned_guess_wave(a.mlp, want, SL.rho, uL, SL.p, SR.rho, uR, SR.p, a.gas.g, a.gas.g, lds);
 }
 
-// Line-parallel sweep along DIR: a block of W waves covers 64 consecutive
-// grid lines of the sweep direction (lane: line; DIR 0: x-line i, DIR 1:
-// y-line j) and the cells c0-1 .. c0+W-2 along them (wave w: cell c = c0-1+w).
-// Neighbours along the sweep live in the next wave, so values, slopes and then
-// fluxes are exchanged through LDS (one array each: three barriers per block).
-// Wave w solves interface c+1 (between cells c and c+1); waves 1..W-1 update
-// cells c0 .. c0+W-2.  The 64 lanes of a wave lie across the sweep, so an
-// interface front (a shock or contact crossing the lines) is met by the whole
-// wave together and the GRP branches stay coherent.  Used for DIR 0, where the
-// lanes read consecutive doubles.  (For DIR 1 each lane would read its own row,
-// stride ld: on MI355X that form ran as fast as sweep_y_kernel at 1024^2 and
-// 3x slower at 4096^2, where the rows no longer stay in cache.)
-// One chunk of a line-parallel sweep: the block's waves own cells
-// c0 - 1 + w (w = 0 .. W-1) of the 64 lines of group bx.  Wave w solves the
-// face right of its cell; waves 1 .. W-1 update their cells with the face left
-// of them, and wave 0 too when `carried` (with the face the previous chunk's
-// last wave left in xf and xi, which wave 0 keeps in xc).  tab: the pow tables,
-// filled in the `first` chunk.  Returns false when the sweep is halted (only
-// checked with `first`).
-// lane, w: the thread's lane and wave (threadIdx.x & 63, threadIdx.x >> 6).
-// The global loads of a chunk for the thread's own cell c = c0 - 1 + w: its
-// values, previous slopes and E.
-struct ChunkIn {
-    double v[4], sp[4], e_c;
+// How a grid is laid over waves of 64/G grid lines of G cells (wave_sweep): the
+// waves along the fast direction (dir 1: runs of G - 1 cells of a line; dir 0:
+// groups of 64/G lines, whole blocks of them) and the blocks of 4 waves.
+struct WaveGrid {
+    int per_row;
+    long blocks;
 };
-
-template <int DIR, int W>
-__device__ __forceinline__ void chunk_loads(const SweepArgs &a, int lane, int w, int bx, int c0, ChunkIn &in)
+inline WaveGrid wave_grid(int dir, int m, int n, int G)
 {
-    const int line = bx * 64 + lane;
-    const bool col = line < (DIR == 0 ? a.n : a.m);
-    const Line<DIR> L(a, col ? line : 0);
-    const int m = L.cnt;
-    const int c = c0 - 1 + w;
-    const bool own = col && c >= 0 && c < m;
-    in.v[0] = 1.0; in.v[1] = 0.0; in.v[2] = 0.0; in.v[3] = 1.0;
-    in.sp[0] = in.sp[1] = in.sp[2] = in.sp[3] = 0.0;
-    in.e_c = 0.0;
-    if (col && c <= m) L.value(c, in.v);
-    if (own) {
-        L.prev_slopes(c, in.sp);
-        in.e_c = a.st[L.at(c) + 4 * a.plane];
+    const int lines = 64 / G;
+    if (dir == 0) {
+        const int groups = (n + 4 * lines - 1) / (4 * lines) * 4;
+        return {groups, (long)(groups / 4) * ((m + G - 2) / (G - 1))};
     }
+    const int runs = (n + G - 2) / (G - 1);
+    return {runs, ((long)((m + lines - 1) / lines) * runs + 3) / 4};
 }
 
-template <int DIR, int W, int NM, class Src>
-__device__ __forceinline__ bool line_chunk(const SweepArgs &a, const Src &src, int lane, int w, int bx, int c0, bool first,
-                                          bool carried, double (*xa)[4][64],
-                                          double (*xb)[4][64], double (*xf)[4][64], double (*xi)[4][64],
-                                          double (*xe)[64], double (*xc)[64], double *tab)
+// Launch variants: lanes along a line and the register budget (waves per SIMD).
+// Four waves cost some 45 spilled registers and are 3-5 % faster than three
+// (none spilled) once a grid gives every SIMD more than three waves (a step of
+// 512^2 .144 against .151 ms, 1024^2 .326 against .336); below that the budget of
+// three is 3 % faster (384^2 .107 against .110, 127 x 329 .072 against .075), so
+// that is a smaller grid's default.
+// G = 16: the repeated face is 1 in 16 and a front along the lines still meets
+// few waves; G = 8 repeats 1 in 8 (1024^2: X .120 ms), G = 32 reads X lines in
+// 16-byte pieces (4096^2 learned: X 1.64 ms against 1.36).
+struct SweepShape {
+    int G, minw;
+};
+inline SweepShape sweep_shape(int dir, int variant)
 {
-    const int line = bx * 64 + lane;
-    const bool col = line < (DIR == 0 ? a.n : a.m);
-    const Line<DIR> L(a, col ? line : 0);
-    const int m = L.cnt;                          // cells along the sweep
-    const int c = c0 - 1 + w;                     // owned cell; -1 and m are ghosts
-    const double hh = a.hh;
-
-    // every global load of the chunk up front, before the first LDS store:
-    // the owned cell's values, previous slopes and E, then the end waves'
-    // extra cells, and in the first chunk the pow tables
-    const bool own = col && c >= 0 && c < m;
-    double v[4], vl[4], vr[4], sp[4], e_c;
-    {
-        ChunkIn in;
-        chunk_loads<DIR, W>(a, lane, w, bx, c0, in);
-        e_c = in.e_c;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) { v[q] = in.v[q]; sp[q] = in.sp[q]; }
-    }
-    if (col && w == 0 && c >= 0) L.value(c - 1, vl);
-    // the last wave also limits cell c + 1 (the right side of its interface): its loads go out now too
-    double vrr[4], sp1[4];
-    if (col && w == W - 1 && c + 1 <= m) L.value(c + 1, vr);
-    if (col && w == W - 1 && c + 1 < m) {
-        L.value(c + 2, vrr);
-        L.prev_slopes(c + 1, sp1);
-    }
-    if (first) {
-        TabLoad<64 * W> t;
-        t.load(w * 64 + lane);
-        t.store(w * 64 + lane, tab);
-    }
-    if (carried && w == 0)                        // the face on its left, before the last wave writes its next one
-#pragma unroll
-        for (int q = 0; q < 4; ++q) { xc[q][lane] = xf[W - 1][q][lane]; xc[4 + q][lane] = xi[W - 1][q][lane]; }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) xa[w][q][lane] = v[q];
-    xe[w][lane] = e_c;
-    const bool next_own = col && w == W - 1 && c + 1 < m;
-    // the predecessor's status is read while the loads above are in flight
-    // (they stay in bounds either way); the whole block returns together
-    if (first && sweep_halted(a)) return false;
-    __syncthreads();
-    if (w > 0)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) vl[q] = xa[w - 1][q][lane];
-    if (w < W - 1)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) vr[q] = xa[w + 1][q][lane];
-
-    double s[4] = {0.0, 0.0, 0.0, 0.0}, sr[4] = {0.0, 0.0, 0.0, 0.0};
-    if (own) L.limited_sp(vl, v, vr, sp, s);
-    if (next_own) L.limited_sp(v, vr, vrr, sp1, sr);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) xb[w][q][lane] = s[q];
-    __syncthreads();
-    if (w < W - 1)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) sr[q] = xb[w + 1][q][lane];
-    // the ghosts' slopes from the boundary cells' (the lane has them by now)
-    if (col && (c == -1 || c + 1 == m)) {
-        double g[4];
-        L.ghost_slope_near(c == -1, c == -1 ? sr : s, g);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            if (c == -1) s[q] = g[q]; else sr[q] = g[q];
-        }
-    }
-
-    double F[4] = {0.0, 0.0, 0.0, 0.0}, I[4] = {0.0, 0.0, 0.0, 0.0};
-    const int f = c + 1;
-    double pg = -1.0;
-    if constexpr (NM == NM_LEARNED) {
-        // xf[w] is not written before the solve: it holds this wave's network inputs
-        const Side SL = recon(v, s, hh, true);
-        const Side SR = recon(vr, sr, hh, false);
-        pg = interface_guess<DIR>(src.get(), col && f <= m, SL, SR, (uint32_t *)&xf[w][0][0]);
-    }
-    if (col && f <= m) {
-        // the argument block is read again here and after the solve, so that
-        // none of it is held across the solve
-        const Side SL = recon(v, s, hh, true);
-        const Side SR = recon(vr, sr, hh, false);
-        solve_interface<DIR, NM, 4>(src.get(), src, SL, SR, line, f, F, I, tab, pg);
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) { xf[w][q][lane] = F[q]; xi[w][q][lane] = I[q]; }
-    __syncthreads();
-    if (own && (w >= 1 || carried)) {
-        // the cell's values and E come back from LDS, so no register holds them across the solve
-        const SweepArgs ar = src.get();
-        const Line<DIR> Lr(ar, line);
-        double Fl[4], Il[4], vc[4];
-        if (w >= 1) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) { Fl[q] = xf[w - 1][q][lane]; Il[q] = xi[w - 1][q][lane]; }
-        } else {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) { Fl[q] = xc[q][lane]; Il[q] = xc[4 + q][lane]; }
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) vc[q] = xa[w][q][lane];
-        Lr.update_e(c, vc, xe[w][lane], Fl, F, Il, I);
-    }
-    return true;
+    static const SweepShape x[6] = {{16, 4}, {32, 4}, {8, 4}, {16, 3}, {8, 3}, {32, 3}};
+    static const SweepShape y[5] = {{16, 4}, {32, 4}, {64, 4}, {8, 4}, {16, 3}};
+    return dir == 0 ? x[variant] : y[variant];
+}
+inline int default_variant(int dir, int m, int n)
+{
+    return wave_grid(dir, m, n, 16).blocks <= 3 * 256 ? (dir == 0 ? 3 : 4) : 0;
 }
 
-// Line-parallel sweep of one block: (bx, by) its group of 64 lines and its
-// run of W - 1 cells (by (W - 1) onwards, wave 0 holding the halo cell); src
-// gives the argument block again after the solve.
-template <int DIR, int W, int NM, class Src>
-__device__ __forceinline__ void line_sweep(const SweepArgs &a, const Src &src, int bx, int by, double (*xa)[4][64],
-                                           double (*xb)[4][64], double (*xf)[4][64], double (*xi)[4][64],
-                                           double (*xe)[64], double *tab)
+// Wave-parallel sweep along DIR: a wave holds 64/G grid lines of G lanes each;
+// the lane at place k of a line owns cell c0-1+k, computes interface c0+k and
+// updates cell c0-1+k for k >= 1 (G-1 cells per line).  Neighbours are lanes of
+// the same wave, so no wave waits for another once the pow tables are there: a
+// row of waves that hands its faces on through LDS waits 40 % of the time at
+// its three barriers (X of 4096^2: 1.56 ms against 1.36 with the learned guess,
+// 1.83 against 1.50 without; 1024^2 .123 against .109).
+// DIR 1: the lanes of a line are consecutive (and so are its cells in memory);
+// DIR 0: the lines are (lane k 64/G + l: line l, so 64/G consecutive i), and a
+// block's waves take neighbouring lines, so that together they read whole cache
+// lines.  Stacked lines let a front that lies along them meet few waves, each
+// with many lanes on it.
+// wave: the wave's index in the grid's sweep, per_row as wave_grid's; st, mlp:
+// this wave's LDS slots; tab: the block's, for the pow tables; src gives the
+// argument block again after the solve.
+template <int DIR, int MINW, int NM, int G, class Src>
+__device__ __forceinline__ void wave_sweep(const SweepArgs &a, const Src &src, long wave, int per_row,
+                                           double (*st)[64], uint32_t *mlp, double *tab)
 {
-    (void)line_chunk<DIR, W, NM>(a, src, threadIdx.x & 63, threadIdx.x >> 6, bx, by * (W - 1), true, false, xa, xb, xf,
-                                 xi, xe, nullptr, tab);
-}
-
-// The same walking K chunks of W cells along the block's lines (by (K W - 1)
-// onwards): the first chunk's wave 0 is the halo cell as above, and in every
-// later chunk wave 0 updates its cell too, with the face that the previous
-// chunk's last wave solved (wave 0 moves it to xc before the first barrier; the
-// last wave writes xf and xi again only after the second); a block then solves
-// K W faces for K W - 1 cells instead of W for W - 1.  What the other waves write
-// before a chunk's first barrier, the previous chunk reads only before its last
-// one, so the chunks need no barrier between them.  With the pow tables a block
-// takes 77 KiB of LDS: two still fit a CU.  The argument block is
-// read again for each chunk, and the lane and wave indices pass through an
-// empty asm each time, so that neither the arguments nor the LDS addresses
-// derived from them are held across the chunks' solves.
-template <int DIR, int W, int NM, int K, class Src>
-__device__ __forceinline__ void line_sweep_chunks(const Src &src, int bx, int by, double (*xa)[4][64],
-                                                  double (*xb)[4][64], double (*xf)[4][64], double (*xi)[4][64],
-                                                  double (*xe)[64], double (*xc)[64], double *tab)
-{
-    const int s0 = by * (K * W - 1);
-    for (int k = 0; k < K; ++k) {
-        const SweepArgs a = src.get();
-        const int c0 = s0 + k * W;
-        if (c0 - 1 >= (DIR == 0 ? a.m : a.n)) break;   // uniform: the chunk lies past the last cell
-        int lane = threadIdx.x & 63;
-        int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-        __asm__ volatile("" : "+v"(lane));
-        __asm__ volatile("" : "+s"(w));
-        if (!line_chunk<DIR, W, NM>(a, src, lane, w, bx, c0, k == 0, k > 0, xa, xb, xf, xi, xe, xc, tab))
-            return;
-    }
-}
-
-// Y sweep: a wave holds 64/G y-lines (rows j) of G lanes each; lane k of a
-// row owns cell c0-1+k, computes interface c0+k and updates cell c0-1+k for
-// k >= 1 (G-1 cells per row).  With G = 64 a wave is one stretch of one line;
-// smaller G stacks rows, so that a front lying along y (constant i) meets
-// fewer waves, each with more lanes on it.
-// wave: the wave's index in the grid's sweep (a group of 64/G rows, one run
-// of G - 1 cells); st, mlp: this wave's LDS slots; tab: the block's, for the
-// pow tables; src gives the argument block again after the solve.
-template <int MINW, int NM, int G, class Src>
-__device__ __forceinline__ void y_sweep(const SweepArgs &a, const Src &src, long wave, int chunks,
-                                        double (*st)[64], uint32_t *mlp, double *tab)
-{
-    static_assert(G == 64 || G == 32 || G == 16 || G == 8, "lanes per row");
-    constexpr int ROWS = 64 / G;
+    static_assert(G == 64 || G == 32 || G == 16 || G == 8, "lanes per line");
+    constexpr int LINES = 64 / G, STEP = DIR == 0 ? LINES : 1;   // STEP: lanes between neighbours along the sweep
     constexpr bool LEARNED = NM == NM_LEARNED;
-    const int lane = threadIdx.x & 63, k = lane % G;
-    const int jg = (int)(wave / chunks);
-    const int j = jg * ROWS + lane / G;
-    const bool rowv = j < a.m;
-    const int c0 = (int)(wave % chunks) * (G - 1);
-    const int n = a.n;
+    const int lane = threadIdx.x & 63, k = DIR == 0 ? lane / LINES : lane % G;
+    const int slow = (int)(wave / per_row), fast = (int)(wave % per_row);
+    const int j = (DIR == 0 ? fast : slow) * LINES + (DIR == 0 ? lane % LINES : lane / G);
+    const bool rowv = j < (DIR == 0 ? a.n : a.m);
+    const int c0 = (DIR == 0 ? slow : fast) * (G - 1);
+    const int n = DIR == 0 ? a.m : a.n;                // cells along the sweep
     const int c = c0 - 1 + k;
-    const Line<1> L(a, rowv ? j : 0);
+    const Line<DIR> L(a, rowv ? j : 0);
     const double hh = a.hh;
 
     const bool own = rowv && c >= 0 && c < n;
@@ -492,7 +339,7 @@ __device__ __forceinline__ void y_sweep(const SweepArgs &a, const Src &src, long
     if (sweep_halted(a)) return;
     t.store(threadIdx.x, tab);
     __syncthreads();
-    if (jg * ROWS >= a.m) return;                      // uniform per wave
+    if (!__any(rowv) || c0 >= n) return;               // a wave past the last line or cell
     // each lane reads back only its own slots: no barrier needed
 #pragma unroll
     for (int q = 0; q < 4; ++q) st[q][lane] = w[q];
@@ -500,7 +347,7 @@ __device__ __forceinline__ void y_sweep(const SweepArgs &a, const Src &src, long
     // neighbours along the row from the next lanes; a row's end lanes take the loaded ones
     double wl[4], wr[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) { wl[q] = __shfl_up(w[q], 1); wr[q] = __shfl_down(w[q], 1); }
+    for (int q = 0; q < 4; ++q) { wl[q] = __shfl_up(w[q], STEP); wr[q] = __shfl_down(w[q], STEP); }
     if (first)
 #pragma unroll
         for (int q = 0; q < 4; ++q) wl[q] = wl_e[q];
@@ -513,7 +360,7 @@ __device__ __forceinline__ void y_sweep(const SweepArgs &a, const Src &src, long
 
     double sr[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) sr[q] = __shfl_down(s[q], 1);
+    for (int q = 0; q < 4; ++q) sr[q] = __shfl_down(s[q], STEP);
     if (last_own) L.limited_sp(w, wr, wrr, sp1, sr);
     // the ghosts' slopes from the boundary cells'
     if (rowv && (c == -1 || c + 1 == n)) {
@@ -532,21 +379,21 @@ __device__ __forceinline__ void y_sweep(const SweepArgs &a, const Src &src, long
     if constexpr (LEARNED) {
         const Side SL = recon(w, s, hh, true);
         const Side SR = recon(wr, sr, hh, false);
-        pg = interface_guess<1>(src.get(), face, SL, SR, mlp);
+        pg = interface_guess<DIR>(src.get(), face, SL, SR, mlp);
     }
     if (face) {
         // the argument block is read again here and after the solve, so that
         // none of it is held across the solve
         const Side SL = recon(w, s, hh, true);
         const Side SR = recon(wr, sr, hh, false);
-        solve_interface<1, NM, MINW>(src.get(), src, SL, SR, j, f, F, I, tab, pg);
+        solve_interface<DIR, NM, MINW>(src.get(), src, SL, SR, j, f, F, I, tab, pg);
     }
     double Fl[4], Il[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) { Fl[q] = __shfl_up(F[q], 1); Il[q] = __shfl_up(I[q], 1); }
+    for (int q = 0; q < 4; ++q) { Fl[q] = __shfl_up(F[q], STEP); Il[q] = __shfl_up(I[q], STEP); }
     if (k >= 1 && own) {
         const SweepArgs ar = src.get();
-        const Line<1> Lr(ar, j);
+        const Line<DIR> Lr(ar, j);
         double wc[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) wc[q] = st[q][lane];

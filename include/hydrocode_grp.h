@@ -161,12 +161,12 @@ int hgrp2d_set_unsplit_form(hgrp2d *ctx, int form);
 #define HGRP_SOLVER_G2D 1
 int hgrp2d_set_interface_solver(hgrp2d *ctx, int solver);
 
-/* Launch variants of the X sweep (0..4) and the Y sweep (0..4) (no counterpart
- * in the reference).  X: 0 = 8 cell rows per block at 4 waves/SIMD (the
- * default), 1 = 8 rows at the compiler's register budget, 2 = 16 rows, 3 and 4
- * = 8 rows walking 4 and 8 chunks along the lines (fewer repeated solves).  Y: 0 =
- * 4 rows of 16 lanes per wave (the default), 1 = 2 x 32, 2 = 1 x 64, 3 = 8 x 8,
- * 4 = 1 x 64 at the compiler's register budget.  Results do not depend on them. */
+/* Launch variants of the X sweep (0..5) and the Y sweep (0..4) (no counterpart
+ * in the reference): a wave holds 64/G grid lines of G lanes along the sweep, at
+ * a register budget for w waves per SIMD.  X: 0 = G 16, w 4; 1 = 32, 4; 2 = 8, 4;
+ * 3 = 16, 3; 4 = 8, 3; 5 = 32, 3.  Y: 0 = 16, 4; 1 = 32, 4; 2 = 64, 4; 3 = 8, 4;
+ * 4 = 16, 3.  The defaults are G 16 with w 4, on grids too small to give every
+ * SIMD more than three waves with w 3.  Results do not depend on them. */
 int hgrp2d_set_sweeps(hgrp2d *ctx, int x_variant, int y_variant);
 
 /* Sweep autotuner: times every X variant, then every Y variant, over `steps`
