@@ -99,4 +99,22 @@ __device__ __forceinline__ Side recon(const double w[4], const double s[4], doub
     return f;
 }
 
+// How a grid is laid over waves of 64/G grid lines of G cells (wave_sweep): the
+// waves along the fast direction (dir 1: runs of G - 1 cells of a line; dir 0:
+// groups of 64/G lines, whole blocks of them) and the blocks of 4 waves.
+struct WaveGrid {
+    int per_row;
+    long blocks;
+};
+inline WaveGrid wave_grid(int dir, int m, int n, int G)
+{
+    const int lines = 64 / G;
+    if (dir == 0) {
+        const int groups = (n + 4 * lines - 1) / (4 * lines) * 4;
+        return {groups, (long)(groups / 4) * ((m + G - 2) / (G - 1))};
+    }
+    const int runs = (n + G - 2) / (G - 1);
+    return {runs, ((long)((m + lines - 1) / lines) * runs + 3) / 4};
+}
+
 }  // namespace hgrp

@@ -238,24 +238,6 @@ __device__ __forceinline__ double interface_guess(const SweepArgs &a, bool activ
     return learned_guess_wave(a.mlp, want, SL.rho, uL, SL.p, SR.rho, uR, SR.p, a.gas.g, a.gas.g, lds);
 }
 
-// How a grid is laid over waves of 64/G grid lines of G cells (wave_sweep): the
-// waves along the fast direction (dir 1: runs of G - 1 cells of a line; dir 0:
-// groups of 64/G lines, whole blocks of them) and the blocks of 4 waves.
-struct WaveGrid {
-    int per_row;
-    long blocks;
-};
-inline WaveGrid wave_grid(int dir, int m, int n, int G)
-{
-    const int lines = 64 / G;
-    if (dir == 0) {
-        const int groups = (n + 4 * lines - 1) / (4 * lines) * 4;
-        return {groups, (long)(groups / 4) * ((m + G - 2) / (G - 1))};
-    }
-    const int runs = (n + G - 2) / (G - 1);
-    return {runs, ((long)((m + lines - 1) / lines) * runs + 3) / 4};
-}
-
 // Launch variants: lanes along a line and the register budget (waves per SIMD).
 // Four waves cost some 45 spilled registers and are 3-5 % faster than three
 // (none spilled) once a grid gives every SIMD more than three waves (a step of

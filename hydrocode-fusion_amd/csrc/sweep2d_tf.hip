@@ -246,126 +246,25 @@ __device__ __forceinline__ bool tf_halted(const SweepArgs &a)
     return false;
 }
 
-// X sweep, row-parallel (the layout of sweep_x_rows_kernel with five quantities):
-// W waves per block, W - 1 cell rows updated; one block fills a CU at W / 4
-// waves per SIMD
-template <int W, int NM>
-__global__ void __launch_bounds__(64 * W, (W + 3) / 4) sweep_x_tf_kernel(SweepArgs a)
+// Both sweeps in the wave form of the single-fluid ones (wave_sweep): G = 16
+// cells of 4 lines per wave, a register budget for three waves per SIMD (some
+// 50 registers spilled; a step of 2048 x 512 .414 ms, at two waves .467, at four
+// .541).  The X sweep as rows of waves that hand faces on through LDS took .170
+// ms, this form .137.
+template <int DIR, int NM, int G>
+__device__ __forceinline__ void wave_sweep_tf(const SweepArgs &a, int per_row, double (*st)[64], uint32_t *mlp, double *tab)
 {
     constexpr bool LEARNED = NM == NM_LEARNED;
-    __shared__ double xa[W][NQ][64];   // values
-    __shared__ double xb[W][NQ][64];   // slopes
-    __shared__ double xf[W][4][64];    // fluxes
-    __shared__ double xz[W][3][64];    // u_n a, u_n at t + tau/2; a at t + tau
-    __shared__ double xi[W][4][64];    // interface values at t + tau
-    __shared__ double xe[W][64];       // E of the owned row
-    __shared__ double tab[POW_TAB];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int i = blockIdx.x * 64 + lane;
-    const bool col = i < a.n;
-    const int m = a.m;
-    const int j0 = blockIdx.y * (W - 1);
-    const int c = j0 - 1 + w;
-    const LineTF<0> L(a, col ? i : 0);
-
-    const bool own = col && c >= 0 && c < m;
-    double v[NQ] = {1.0, 0.0, 0.0, 1.0, 1.0}, vl[NQ], vr[NQ], sp[NQ] = {0.0, 0.0, 0.0, 0.0, 0.0}, e_c = 0.0;
-    // every global load before the first LDS store: the owned cell, then the
-    // end waves' extra cells
-    if (col && c <= m) L.value(c, v);
-    if (own) {
-        L.prev_slopes(c, sp);
-        e_c = a.st[L.at(c) + 4 * a.plane];
-    }
-    if (col && w == 0 && c >= 0) L.value(c - 1, vl);
-    double vrr[NQ], sp1[NQ];
-    const bool next_own = col && w == W - 1 && c + 1 < m;
-    if (col && w == W - 1 && c + 1 <= m) L.value(c + 1, vr);
-    if (next_own) {
-        L.value(c + 2, vrr);
-        L.prev_slopes(c + 1, sp1);
-    }
-    TabLoad<64 * W> tl;
-    tl.load(threadIdx.x);
-    tl.store(threadIdx.x, tab);
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) xa[w][q][lane] = v[q];
-    xe[w][lane] = e_c;
-    // the predecessor's status is read while the loads above are in flight
-    // (they stay in bounds either way); the whole block returns together
-    if (tf_halted(a)) return;
-    __syncthreads();
-    if (w > 0)
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) vl[q] = xa[w - 1][q][lane];
-    if (w < W - 1)
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) vr[q] = xa[w + 1][q][lane];
-
-    double s[NQ] = {0.0, 0.0, 0.0, 0.0, 0.0}, sr[NQ] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    if (own) L.limited_sp(vl, v, vr, sp, s);
-    if (next_own) L.limited_sp(v, vr, vrr, sp1, sr);
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) xb[w][q][lane] = s[q];
-    __syncthreads();
-    if (w < W - 1)
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) sr[q] = xb[w + 1][q][lane];
-    // the ghosts' slopes from the boundary cells'
-    if (col && (c == -1 || c + 1 == m)) {
-        double g[NQ];
-        L.ghost_slope_near(c == -1, c == -1 ? sr : s, g);
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            if (c == -1) s[q] = g[q]; else sr[q] = g[q];
-        }
-    }
-
-    double F[4] = {0.0, 0.0, 0.0, 0.0}, I[4] = {0.0, 0.0, 0.0, 0.0}, Z[3] = {0.0, 0.0, 0.0};
-    const int f = c + 1;
-    double pg = -1.0;
-    if constexpr (LEARNED)   // xf[w] is not written before the solve: it holds the network inputs
-        pg = interface_guess_tf<0>(a, col && f <= m, v, s, vr, sr, (uint32_t *)&xf[w][0][0]);
-    if (col && f <= m)
-        solve_interface_tf<0, NM>(a, v, s, vr, sr, i, f, F, I, Z, tab, pg);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) { xf[w][q][lane] = F[q]; xi[w][q][lane] = I[q]; }
-#pragma unroll
-    for (int q = 0; q < 3; ++q) xz[w][q][lane] = Z[q];
-    __syncthreads();
-    if (own && w >= 1) {
-        double Fl[4], Il[4], Zl[3], vc[NQ];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) { Fl[q] = xf[w - 1][q][lane]; Il[q] = xi[w - 1][q][lane]; }
-#pragma unroll
-        for (int q = 0; q < 3; ++q) Zl[q] = xz[w - 1][q][lane];
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) vc[q] = xa[w][q][lane];
-        const SweepArgs ar = reload_args<SweepArgs>();   // not held across the solve
-        LineTF<0>(ar, i).update(c, vc, xe[w][lane], Fl, F, Zl, Z, Il, I);
-    }
-}
-
-// Y sweep: a wave owns 64 consecutive cells of a y-line (as sweep_y_kernel)
-template <int NM, int G = 16>
-__global__ void __launch_bounds__(256, 3) sweep_y_tf_kernel(SweepArgs a, int chunks)
-{
-    constexpr bool LEARNED = NM == NM_LEARNED;
-    // 64/G y-lines of G lanes per wave, as in sweep_y_kernel: lane k of a row
-    // owns cell c0-1+k and updates it for k >= 1
-    constexpr int ROWS = 64 / G;
-    __shared__ double stash[4][NQ + 1][64];
-    __shared__ uint32_t mlp_lds[LEARNED ? 4 : 1][LEARNED ? 64 * 8 : 1];
-    __shared__ double tab[POW_TAB];
-    const int lane = threadIdx.x & 63, k = lane % G;
+    constexpr int LINES = 64 / G, STEP = DIR == 0 ? LINES : 1;   // STEP: lanes between neighbours along the sweep
+    const int lane = threadIdx.x & 63, k = DIR == 0 ? lane / LINES : lane % G;
     const long wave = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int jg = (int)(wave / chunks);
-    const int j = jg * ROWS + lane / G;
-    const bool rowv = j < a.m;
-    const int c0 = (int)(wave % chunks) * (G - 1);
-    const int n = a.n;
+    const int slow = (int)(wave / per_row), fast = (int)(wave % per_row);
+    const int j = (DIR == 0 ? fast : slow) * LINES + (DIR == 0 ? lane % LINES : lane / G);
+    const bool rowv = j < (DIR == 0 ? a.n : a.m);
+    const int c0 = (DIR == 0 ? slow : fast) * (G - 1);
+    const int n = DIR == 0 ? a.m : a.n;                          // cells along the sweep
     const int c = c0 - 1 + k;
-    const LineTF<1> L(a, rowv ? j : 0);
+    const LineTF<DIR> L(a, rowv ? j : 0);
 
     const bool own = rowv && c >= 0 && c < n;
     double w[NQ] = {1.0, 0.0, 0.0, 1.0, 1.0}, sp[NQ] = {0.0, 0.0, 0.0, 0.0, 0.0}, e_c = 0.0;
@@ -390,14 +289,13 @@ __global__ void __launch_bounds__(256, 3) sweep_y_tf_kernel(SweepArgs a, int chu
     if (tf_halted(a)) return;
     tl.store(threadIdx.x, tab);
     __syncthreads();
-    if (jg * ROWS >= a.m) return;
-    double(*st)[64] = stash[(threadIdx.x >> 6) & 3];
+    if (!__any(rowv) || c0 >= n) return;                         // a wave past the last line or cell
 #pragma unroll
     for (int q = 0; q < NQ; ++q) st[q][lane] = w[q];
     st[NQ][lane] = e_c;
     double wl[NQ], wr[NQ];
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) { wl[q] = __shfl_up(w[q], 1); wr[q] = __shfl_down(w[q], 1); }
+    for (int q = 0; q < NQ; ++q) { wl[q] = __shfl_up(w[q], STEP); wr[q] = __shfl_down(w[q], STEP); }
     if (first)
 #pragma unroll
         for (int q = 0; q < NQ; ++q) wl[q] = wl_e[q];
@@ -409,7 +307,7 @@ __global__ void __launch_bounds__(256, 3) sweep_y_tf_kernel(SweepArgs a, int chu
     if (own) L.limited_sp(wl, w, wr, sp, s);
     double sr[NQ];
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) sr[q] = __shfl_down(s[q], 1);
+    for (int q = 0; q < NQ; ++q) sr[q] = __shfl_down(s[q], STEP);
     if (last_own) L.limited_sp(w, wr, wrr, sp1, sr);
     // the ghosts' slopes from the boundary cells'
     if (rowv && (c == -1 || c + 1 == n)) {
@@ -425,21 +323,43 @@ __global__ void __launch_bounds__(256, 3) sweep_y_tf_kernel(SweepArgs a, int chu
     const int f = c + 1;
     const bool face = rowv && f <= n;
     double pg = -1.0;
-    if constexpr (LEARNED) pg = interface_guess_tf<1>(a, face, w, s, wr, sr, mlp_lds[(threadIdx.x >> 6) & 3]);
+    if constexpr (LEARNED) pg = interface_guess_tf<DIR>(a, face, w, s, wr, sr, mlp);
     if (face)
-        solve_interface_tf<1, NM>(a, w, s, wr, sr, j, f, F, I, Z, tab, pg);
+        solve_interface_tf<DIR, NM>(a, w, s, wr, sr, j, f, F, I, Z, tab, pg);
     double Fl[4], Il[4], Zl[3];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) { Fl[q] = __shfl_up(F[q], 1); Il[q] = __shfl_up(I[q], 1); }
+    for (int q = 0; q < 4; ++q) { Fl[q] = __shfl_up(F[q], STEP); Il[q] = __shfl_up(I[q], STEP); }
 #pragma unroll
-    for (int q = 0; q < 3; ++q) Zl[q] = __shfl_up(Z[q], 1);
+    for (int q = 0; q < 3; ++q) Zl[q] = __shfl_up(Z[q], STEP);
     if (k >= 1 && own) {
         double wc[NQ];
 #pragma unroll
         for (int q = 0; q < NQ; ++q) wc[q] = st[q][lane];
         const SweepArgs ar = reload_args<SweepArgs>();   // not held across the solve
-        LineTF<1>(ar, j).update(c, wc, st[NQ][lane], Fl, F, Zl, Z, Il, I);
+        LineTF<DIR>(ar, j).update(c, wc, st[NQ][lane], Fl, F, Zl, Z, Il, I);
     }
+}
+
+template <int NM, int G>
+__global__ void __launch_bounds__(256, 3) sweep_x_tf_kernel(SweepArgs a, int per_row)
+{
+    constexpr bool LEARNED = NM == NM_LEARNED;
+    __shared__ double stash[4][NQ + 1][64];
+    __shared__ uint32_t mlp_lds[LEARNED ? 4 : 1][LEARNED ? 64 * 8 : 1];
+    __shared__ double tab[POW_TAB];
+    const int wv = (threadIdx.x >> 6) & 3;
+    wave_sweep_tf<0, NM, G>(a, per_row, stash[wv], mlp_lds[wv], tab);
+}
+
+template <int NM, int G>
+__global__ void __launch_bounds__(256, 3) sweep_y_tf_kernel(SweepArgs a, int per_row)
+{
+    constexpr bool LEARNED = NM == NM_LEARNED;
+    __shared__ double stash[4][NQ + 1][64];
+    __shared__ uint32_t mlp_lds[LEARNED ? 4 : 1][LEARNED ? 64 * 8 : 1];
+    __shared__ double tab[POW_TAB];
+    const int wv = (threadIdx.x >> 6) & 3;
+    wave_sweep_tf<1, NM, G>(a, per_row, stash[wv], mlp_lds[wv], tab);
 }
 
 // min over cells of min(h_x, h_y) / (|c| + |u| + |v|) with the mixture's gamma
@@ -502,38 +422,32 @@ hipError_t launch_energy_tf(const double *rho, const double *u, const double *v,
 // the two-fluid sweep kernel's name as profilers print it
 const char *sweep_tf_kernel_name(int dir, int nm)
 {
-    static const char *xn[3] = {"sweep_x_tf_kernel<12, 0>", "sweep_x_tf_kernel<12, 1>", "sweep_x_tf_kernel<12, 2>"};
+    static const char *xn[3] = {"sweep_x_tf_kernel<0, 16>", "sweep_x_tf_kernel<1, 16>", "sweep_x_tf_kernel<2, 16>"};
     static const char *yn[3] = {"sweep_y_tf_kernel<0, 16>", "sweep_y_tf_kernel<1, 16>", "sweep_y_tf_kernel<2, 16>"};
     if (nm < 0 || nm > 2 || dir < 0 || dir > 1) return "";
     return dir == 0 ? xn[nm] : yn[nm];
 }
 
-// Rows per block of the X sweep: 12 waves (11 rows updated) at 3 waves per SIMD,
-// 132 KiB of LDS
-constexpr int TF_X_W = 12;
-
 hipError_t launch_sweep_x_tf(const SweepArgs &a, hipStream_t st)
 {
-    constexpr int W = TF_X_W;
-    dim3 grid((a.n + 63) / 64, (a.m + W - 2) / (W - 1));
+    const WaveGrid w = wave_grid(0, a.m, a.n, 16);
+    const dim3 grid((unsigned)w.blocks), block(256);
     switch (newton_mode(a)) {
-    case NM_LEARNED: hipLaunchKernelGGL((sweep_x_tf_kernel<W, NM_LEARNED>), grid, dim3(64 * W), 0, st, a); break;
-    case NM_CONV: hipLaunchKernelGGL((sweep_x_tf_kernel<W, NM_CONV>), grid, dim3(64 * W), 0, st, a); break;
-    default: hipLaunchKernelGGL((sweep_x_tf_kernel<W, NM_REF>), grid, dim3(64 * W), 0, st, a); break;
+    case NM_LEARNED: hipLaunchKernelGGL((sweep_x_tf_kernel<NM_LEARNED, 16>), grid, block, 0, st, a, w.per_row); break;
+    case NM_CONV: hipLaunchKernelGGL((sweep_x_tf_kernel<NM_CONV, 16>), grid, block, 0, st, a, w.per_row); break;
+    default: hipLaunchKernelGGL((sweep_x_tf_kernel<NM_REF, 16>), grid, block, 0, st, a, w.per_row); break;
     }
     return hipGetLastError();
 }
 
 hipError_t launch_sweep_y_tf(const SweepArgs &a, hipStream_t st)
 {
-    // 4 rows of 16 lanes per wave (the default of the single-fluid Y sweep)
-    const int chunks = (a.n + 14) / 15;
-    const long waves = (long)((a.m + 3) / 4) * chunks;
-    const long blocks = (waves + 3) / 4;
+    const WaveGrid w = wave_grid(1, a.m, a.n, 16);
+    const dim3 grid((unsigned)w.blocks), block(256);
     switch (newton_mode(a)) {
-    case NM_LEARNED: hipLaunchKernelGGL(sweep_y_tf_kernel<NM_LEARNED>, dim3((unsigned)blocks), dim3(256), 0, st, a, chunks); break;
-    case NM_CONV: hipLaunchKernelGGL(sweep_y_tf_kernel<NM_CONV>, dim3((unsigned)blocks), dim3(256), 0, st, a, chunks); break;
-    default: hipLaunchKernelGGL(sweep_y_tf_kernel<NM_REF>, dim3((unsigned)blocks), dim3(256), 0, st, a, chunks); break;
+    case NM_LEARNED: hipLaunchKernelGGL((sweep_y_tf_kernel<NM_LEARNED, 16>), grid, block, 0, st, a, w.per_row); break;
+    case NM_CONV: hipLaunchKernelGGL((sweep_y_tf_kernel<NM_CONV, 16>), grid, block, 0, st, a, w.per_row); break;
+    default: hipLaunchKernelGGL((sweep_y_tf_kernel<NM_REF, 16>), grid, block, 0, st, a, w.per_row); break;
     }
     return hipGetLastError();
 }

@@ -40,3 +40,24 @@ def test_default_variant(hg, m, n, w):
         assert s.sweep_kernel(0) == f"sweep_x_kernel<{w}, 0, 16>" and s.sweep_kernel(1) == f"sweep_y_kernel<{w}, 0, 16>"
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("m,n", [(1, 1), (14, 15), (15, 16), (16, 17), (31, 4), (33, 46)])
+def test_two_fluid_layout_edges(hg, oracle, m, n):
+    """Cells that are all fluid a run as the single fluid, bit for bit."""
+    s0 = cases.smooth_random(m, n, m + 100 * n)
+    cfg = make_config(t_all=1.0, h_x=1 / m, h_y=1 / n, bc_x=-2, bc_y=-7, split=1)
+    out = []
+    for two in (False, True):
+        c = hg.Solver2D(m, n, cfg)
+        try:
+            c.upload(s0["rho"], s0["u"], s0["v"], s0["p"])
+            if two:
+                c.set_fluids(1.67, np.ones((m, n)))        # all of it fluid a: the single-fluid operations
+            c.bench(7)
+            out.append(np.asarray(c.download()).reshape(5, m, n))
+            if two:
+                assert np.array_equal(c.download_fraction().reshape(m, n), np.ones((m, n)))
+        finally:
+            c.close()
+    assert np.array_equal(out[0], out[1])
