@@ -18,31 +18,6 @@
 
 namespace hgrp {
 
-// X and Y sweeps (wave_sweep): blocks of 4 waves, wave index = global wave number.
-template <int MINW, int NM, int G>
-__global__ void __launch_bounds__(256, MINW) sweep_x_kernel(SweepArgs a, int per_row)
-{
-    constexpr bool LEARNED = NM == NM_LEARNED;
-    __shared__ uint32_t mlp_lds[LEARNED ? 4 : 1][LEARNED ? 64 * 8 : 1];
-    __shared__ double stash[4][5][64];   // each wave's cell values and E, read back for the update
-    __shared__ double tab[POW_TAB];
-    const int wv = (threadIdx.x >> 6) & 3;
-    const long wave = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    wave_sweep<0, MINW, NM, G>(a, KernargArgs{}, wave, per_row, stash[wv], mlp_lds[wv], tab);
-}
-
-template <int MINW, int NM, int G>
-__global__ void __launch_bounds__(256, MINW) sweep_y_kernel(SweepArgs a, int per_row)
-{
-    constexpr bool LEARNED = NM == NM_LEARNED;
-    __shared__ uint32_t mlp_lds[LEARNED ? 4 : 1][LEARNED ? 64 * 8 : 1];
-    __shared__ double stash[4][5][64];
-    __shared__ double tab[POW_TAB];
-    const int wv = (threadIdx.x >> 6) & 3;
-    const long wave = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    wave_sweep<1, MINW, NM, G>(a, KernargArgs{}, wave, per_row, stash[wv], mlp_lds[wv], tab);
-}
-
 // min over cells of min(h_x, h_y) / (|c| + |u| + |v|)  (grp_solver_2D_split_EUL_source.c:185-191).
 // fmin is exact, so the order of the reduction does not matter; positive
 // doubles order like their bit patterns, so a 64-bit atomicMin reduces them.
@@ -73,6 +48,9 @@ __global__ void __launch_bounds__(256) cfl_kernel(const double *rho, const doubl
 int sweep_variants(int dir) { return dir == 0 ? 6 : 5; }
 int default_sweep(int dir, int m, int n) { return default_variant(dir, m, n); }
 
+// the variants of three waves per SIMD (sweep2d_few.hip)
+hipError_t launch_sweep_few(int dir, const SweepArgs &a, int variant, hipStream_t st);
+
 template <int NM>
 static hipError_t launch_x(const SweepArgs &a, int v, hipStream_t st)
 {
@@ -81,9 +59,6 @@ static hipError_t launch_x(const SweepArgs &a, int v, hipStream_t st)
     switch (v) {
     case 1: hipLaunchKernelGGL((sweep_x_kernel<4, NM, 32>), grid, block, 0, st, a, w.per_row); break;
     case 2: hipLaunchKernelGGL((sweep_x_kernel<4, NM, 8>), grid, block, 0, st, a, w.per_row); break;
-    case 3: hipLaunchKernelGGL((sweep_x_kernel<3, NM, 16>), grid, block, 0, st, a, w.per_row); break;
-    case 4: hipLaunchKernelGGL((sweep_x_kernel<3, NM, 8>), grid, block, 0, st, a, w.per_row); break;
-    case 5: hipLaunchKernelGGL((sweep_x_kernel<3, NM, 32>), grid, block, 0, st, a, w.per_row); break;
     default: hipLaunchKernelGGL((sweep_x_kernel<4, NM, 16>), grid, block, 0, st, a, w.per_row); break;
     }
     return hipGetLastError();
@@ -98,7 +73,6 @@ static hipError_t launch_y(const SweepArgs &a, int v, hipStream_t st)
     case 1: hipLaunchKernelGGL((sweep_y_kernel<4, NM, 32>), grid, block, 0, st, a, w.per_row); break;
     case 2: hipLaunchKernelGGL((sweep_y_kernel<4, NM, 64>), grid, block, 0, st, a, w.per_row); break;
     case 3: hipLaunchKernelGGL((sweep_y_kernel<4, NM, 8>), grid, block, 0, st, a, w.per_row); break;
-    case 4: hipLaunchKernelGGL((sweep_y_kernel<3, NM, 16>), grid, block, 0, st, a, w.per_row); break;
     default: hipLaunchKernelGGL((sweep_y_kernel<4, NM, 16>), grid, block, 0, st, a, w.per_row); break;
     }
     return hipGetLastError();
@@ -106,6 +80,7 @@ static hipError_t launch_y(const SweepArgs &a, int v, hipStream_t st)
 
 hipError_t launch_sweep_x(const SweepArgs &a, int variant, hipStream_t st)
 {
+    if (sweep_shape(0, variant).minw == 3) return launch_sweep_few(0, a, variant, st);
     switch (newton_mode(a)) {
     case NM_LEARNED: return launch_x<NM_LEARNED>(a, variant, st);
     case NM_CONV: return launch_x<NM_CONV>(a, variant, st);
@@ -115,6 +90,7 @@ hipError_t launch_sweep_x(const SweepArgs &a, int variant, hipStream_t st)
 
 hipError_t launch_sweep_y(const SweepArgs &a, int variant, hipStream_t st)
 {
+    if (sweep_shape(1, variant).minw == 3) return launch_sweep_few(1, a, variant, st);
     switch (newton_mode(a)) {
     case NM_LEARNED: return launch_y<NM_LEARNED>(a, variant, st);
     case NM_CONV: return launch_y<NM_CONV>(a, variant, st);

@@ -239,11 +239,11 @@ __device__ __forceinline__ double interface_guess(const SweepArgs &a, bool activ
 }
 
 // Launch variants: lanes along a line and the register budget (waves per SIMD).
-// Four waves cost some 45 spilled registers and are 3-5 % faster than three
-// (none spilled) once a grid gives every SIMD more than three waves (a step of
-// 512^2 .144 against .151 ms, 1024^2 .326 against .336); below that the budget of
-// three is 3 % faster (384^2 .107 against .110, 127 x 329 .072 against .075), so
-// that is a smaller grid's default.
+// Four waves cost some 30 spilled registers and are 5-8 % faster than three (none
+// spilled) once a grid gives every SIMD more than three waves (a step of 512^2
+// .143 against .150 ms, 1024^2 .313 against .338); below that the budget of three
+// is 2-4 % faster (384^2 .1056 against .1073, 127 x 329 .072 against .075), so that
+// is a smaller grid's default.
 // G = 16: the repeated face is 1 in 16 and a front along the lines still meets
 // few waves; G = 8 repeats 1 in 8 (1024^2: X .120 ms), G = 32 reads X lines in
 // 16-byte pieces (4096^2 learned: X 1.64 ms against 1.36).
@@ -381,6 +381,31 @@ __device__ __forceinline__ void wave_sweep(const SweepArgs &a, const Src &src, l
         for (int q = 0; q < 4; ++q) wc[q] = st[q][lane];
         Lr.update_e(c, wc, st[4][lane], Fl, F, Il, I);
     }
+}
+
+// X and Y sweeps (wave_sweep): blocks of 4 waves, wave index = global wave number.
+template <int MINW, int NM, int G>
+__global__ void __launch_bounds__(256, MINW) sweep_x_kernel(SweepArgs a, int per_row)
+{
+    constexpr bool LEARNED = NM == NM_LEARNED;
+    __shared__ uint32_t mlp_lds[LEARNED ? 4 : 1][LEARNED ? 64 * 8 : 1];
+    __shared__ double stash[4][5][64];   // each wave's cell values and E, read back for the update
+    __shared__ double tab[POW_TAB];
+    const int wv = (threadIdx.x >> 6) & 3;
+    const long wave = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    wave_sweep<0, MINW, NM, G>(a, KernargArgs{}, wave, per_row, stash[wv], mlp_lds[wv], tab);
+}
+
+template <int MINW, int NM, int G>
+__global__ void __launch_bounds__(256, MINW) sweep_y_kernel(SweepArgs a, int per_row)
+{
+    constexpr bool LEARNED = NM == NM_LEARNED;
+    __shared__ uint32_t mlp_lds[LEARNED ? 4 : 1][LEARNED ? 64 * 8 : 1];
+    __shared__ double stash[4][5][64];
+    __shared__ double tab[POW_TAB];
+    const int wv = (threadIdx.x >> 6) & 3;
+    const long wave = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    wave_sweep<1, MINW, NM, G>(a, KernargArgs{}, wave, per_row, stash[wv], mlp_lds[wv], tab);
 }
 
 }  // namespace hgrp
