@@ -1,19 +1,14 @@
 // unsplit2d.hip -- the genuinely 2D GRP step (no dimension splitting), one
 // launch per time step.
 //
-//   unsplit_step_kernel  a block of W waves (W = TILE_W) covers 62 consecutive y-cells
-//                        (lanes: cells i0-1 .. i0+62) of the cell rows
-//                        j0-1 .. j0+W-2 (wave w: row j0-1+w).  Every lane forms
-//                        the "side data" of its cell -- value, limited x-slope,
-//                        limited y-slope, or the ghost's value and slopes at the
-//                        edges -- and parks it in LDS.  Waves 0..W-2 solve the
-//                        x-interface between their row and the next; waves
-//                        1..W-2 also solve the y-interfaces of the updated rows
-//                        (each half a pair of rows, 2 x 32 interfaces) and
-//                        update their 62 cells with both flux differences.
-//                        Rows j0-1 and j0+W-2 are halo rows; interface rows and
-//                        columns on tile edges are solved by both tiles,
-//                        everything else once.
+//   unsplit_step_kernel  a wave covers a tile of 7 x 8 cells.  It forms the "side
+//                        data" of the tile's cells and of those around it --
+//                        value, limited x-slope, limited y-slope, or the ghost's
+//                        value and slopes at the edges -- in its LDS slots, solves
+//                        the tile's y-interfaces, then its x-interfaces, one lane
+//                        an interface, and updates the cells with both flux
+//                        differences.  Interfaces on tile edges are solved by both
+//                        tiles, everything else once.
 //
 // Semantics follow src/finite_volume/grp_solver_2D_EUL_source.c:181-262,
 // src/inter_process/bound_cond_slope_limiter_{x,y}.c:27-129 (including the
@@ -220,59 +215,70 @@ __device__ __forceinline__ double unsplit_guess(const UnsplitArgs &a, bool activ
 
 }  // namespace
 
-template <int W, int NM, bool G2>
-__device__ __forceinline__ void unsplit_step_body(const UnsplitArgs &a)
+// Tile form: a wave owns a tile of 7 x 8 cells (rows along x, columns along y).
+// Its 8 x 8 x-interfaces fill the wave, its 7 x 9 y-interfaces all but a lane;
+// the side data of its 9 x 10 cells lie in the wave's own LDS slots, and the
+// faces go to the cells' lanes by shuffles, so no wave waits for another once
+// the pow tables are there.  (A tile of 12 waves, 10 rows of 62 cells, handed its
+// faces on through 160 KiB of LDS, one block to a CU, and waited 58 % of its time
+// at the barriers.  A step with it and with this: 300^2 .062 and .054 ms, 512^2
+// .108 and .092, 1024^2 .281 and .283, 4096^2 3.84 and 3.22; G2D 257 x 190 .089
+// and .049, 1024^2 .337 and .347.)
+constexpr int TILE_R = 7, TILE_C = 8, SIDE_C = TILE_C + 2, SIDES = (TILE_R + 2) * SIDE_C - 1;   // not the last corner
+
+template <int NM, bool G2>
+__device__ __forceinline__ void unsplit_step_body(const UnsplitArgs &a, int per_row)
 {
-    __shared__ double sd[W][12][64];     // side data of row c: value, x-slope, y-slope
-    __shared__ double fx[W - 1][8][62];  // x-interface c+1 of lanes 1..62: flux, values at t + tau
-    __shared__ double gy[W - 2][8][64];  // y-interfaces of the updated rows: flux, values at t + tau
+    constexpr bool LEARNED = NM == NM_LEARNED;
+    __shared__ double sides_lds[4][12][SIDES];   // value, x-slope, y-slope of the tile's cells and the ones around
     __shared__ double tab[POW_TAB];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int m = a.m, n = a.n;
-    const int i0 = blockIdx.x * 62, ci = i0 - 1 + lane;
-    const int j0 = blockIdx.y * (W - 2), c = j0 - 1 + w;
-    const Grid G(a);
-    const bool xin = c >= 0 && c < m, yin = ci >= 0 && ci < n;
+    __shared__ uint32_t mlp_lds[LEARNED ? 4 : 1][LEARNED ? 64 * 8 : 1];
+    const int lane = threadIdx.x & 63, wv = (threadIdx.x >> 6) & 3;
+    const long wave = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    const int j0 = (int)(wave / per_row) * TILE_R, i0 = (int)(wave % per_row) * TILE_C;
+    double(*sd)[SIDES] = sides_lds[wv];
+    // the lane's cell (row r, column k of the tile with its halo; updated for r >= 1) and x-interface,
+    // between rows r and r + 1
+    const int r = lane >> 3, k = (lane & 7) + 1, c = j0 - 1 + r, ci = i0 - 1 + k;
+    const bool own = r >= 1 && c < a.m && ci < a.n;
     {
-        double v[4] = {1.0, 0.0, 0.0, 1.0}, s[4] = {0.0, 0.0, 0.0, 0.0}, t[4] = {0.0, 0.0, 0.0, 0.0};
-        TabLoad<64 * W> tl;
+        const Grid G(a);
+        TabLoad<256> tl;
         tl.load(threadIdx.x);
-        tl.store(threadIdx.x, tab);
-        if (c <= m && ci <= n && (xin || yin)) G.side(c, ci, v, s, t);   // a cell or a ghost, not a corner
+#pragma unroll 1
+        for (int id = lane; id < SIDES; id += 64) {
+            const int sc = j0 - 1 + id / SIDE_C, si = i0 - 1 + id % SIDE_C;
+            double v[4] = {1.0, 0.0, 0.0, 1.0}, s[4] = {0.0, 0.0, 0.0, 0.0}, t[4] = {0.0, 0.0, 0.0, 0.0};
+            const bool xin = sc >= 0 && sc < a.m, yin = si >= 0 && si < a.n;
+            if (sc <= a.m && si <= a.n && (xin || yin)) G.side(sc, si, v, s, t);   // a cell or a ghost, not a corner
 #pragma unroll
-        for (int q = 0; q < 4; ++q) { sd[w][q][lane] = v[q]; sd[w][4 + q][lane] = s[q]; sd[w][8 + q][lane] = t[q]; }
-    }
-    // a failed step ends the run: later steps do nothing.  The status is read
-    // after the side loads went out (they stay in bounds either way); the
-    // whole block returns together.
-    if (a.prev != nullptr) {
-        const SweepStatus p0 = a.prev[0], p1 = a.prev[1];
-        if (p0.fail_key != 0ull || p0.flags != 0u || p1.fail_key != 0ull) {
-            if (threadIdx.x == 0) atomicOr(&a.status[0].flags, 2u);
-            return;
+            for (int q = 0; q < 4; ++q) { sd[q][id] = v[q]; sd[4 + q][id] = s[q]; sd[8 + q][id] = t[q]; }
         }
+        // a failed step ends the run: later steps do nothing.  The status is read
+        // after the side loads went out (they stay in bounds either way); the
+        // whole block returns together.
+        if (a.prev != nullptr) {
+            const SweepStatus p0 = a.prev[0], p1 = a.prev[1];
+            if (p0.fail_key != 0ull || p0.flags != 0u || p1.fail_key != 0ull) {
+                if (threadIdx.x == 0) atomicOr(&a.status[0].flags, 2u);
+                return;
+            }
+        }
+        tl.store(threadIdx.x, tab);
     }
     __syncthreads();
+    if (j0 >= a.m) return;                                   // a wave past the last tile
 
     // dir 1: y-interfaces of the updated rows (flux_generator_y.c:42-121), normal derivative =
-    //        y-slope, transversal = -(x-slope); wave w takes half a row pair (2 rows x 32
-    //        interfaces), so a front lying along y meets half as many waves as with one
-    //        64-lane row per wave;
-    // dir 0: x-interface f = c + 1 between rows c and c + 1 (flux_generator_x.c:42-121),
-    //        the right side from the next wave.
-    // One solve site for both, so the GRP code and its registers are laid out once.  The x-pass
-    // comes last: until a wave has solved its x-interfaces its slots of fx are free, and both
-    // passes' network inputs (the learned guess) lie there.
-    const int f = c + 1;
-    const int task = w - 1;                                  // waves 1 .. W-2
-    const int yr = 1 + 2 * (task >> 1) + (lane >> 5);        // tile row of this lane's y-interface
-    const int yt = ((task & 1) << 5) + (lane & 31);          // between tile lanes yt and yt + 1
-    const int yc = j0 - 1 + yr, ycell = i0 - 1 + yt;
+    //        y-slope, transversal = -(x-slope);
+    // dir 0: x-interface f = c + 1 between rows c and c + 1 (flux_generator_x.c:42-121).
+    // One solve site for both, so the GRP code and its registers are laid out once.
+    const int yr = lane / (TILE_C + 1) + 1, yk = lane % (TILE_C + 1), yc = j0 - 1 + yr, ycell = i0 - 1 + yk;
+    double dG[4];
 #pragma unroll 1
     for (int dir = 1; dir >= 0; --dir) {
-        const bool active = dir ? w >= 1 && w <= W - 2 && yc >= 0 && yc < m && yt <= 62 && ycell <= n - 1
-                                : w <= W - 2 && lane >= 1 && lane <= 62 && yin && f <= m;
-        const int r0 = dir ? yr : w, k0 = dir ? yt : lane, r1 = dir ? yr : w + 1, k1 = dir ? yt + 1 : lane;
+        const bool active = dir ? lane < TILE_R * (TILE_C + 1) && yc < a.m && ycell < a.n : c < a.m && ci < a.n;
+        const int id0 = dir ? yr * SIDE_C + yk : r * SIDE_C + k, id1 = dir ? id0 + 1 : id0 + SIDE_C;
         Side SL, SR;
         double TL[4], TR[4];
         // the two cells' side data: value, normal and transversal slope
@@ -282,8 +288,8 @@ __device__ __forceinline__ void unsplit_step_body(const UnsplitArgs &a)
             double vl[4], sl[4], vr[4], sr[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                vl[q] = sd[r0][q][k0]; sl[q] = sd[r0][sn + q][k0]; TL[q] = sd[r0][st + q][k0];
-                vr[q] = sd[r1][q][k1]; sr[q] = sd[r1][sn + q][k1]; TR[q] = sd[r1][st + q][k1];
+                vl[q] = sd[q][id0]; sl[q] = sd[sn + q][id0]; TL[q] = sd[st + q][id0];
+                vr[q] = sd[q][id1]; sr[q] = sd[sn + q][id1]; TR[q] = sd[st + q][id1];
             }
             if (dir)
 #pragma unroll
@@ -292,72 +298,77 @@ __device__ __forceinline__ void unsplit_step_body(const UnsplitArgs &a)
             SR = recon(vr, sr, hh, false);
         };
         double F[4] = {0.0, 0.0, 0.0, 0.0}, I[4] = {0.0, 0.0, 0.0, 0.0}, pg = -1.0;
-        if constexpr (NM == NM_LEARNED) {   // a call: the sides are read again after it, not held across
+        if constexpr (LEARNED) {   // a call: the sides are read again after it, not held across
             if (active) sides();
-            pg = unsplit_guess<NM>(a, active, dir, SL, SR, (uint32_t *)&fx[w < W - 1 ? w : 0][0][0]);
+            pg = unsplit_guess<NM>(a, active, dir, SL, SR, mlp_lds[wv]);
         }
         // the argument block is read again for the solve, so no scalar register holds it across
         if (active) {
             sides();
             solve_t<NM, G2>(reload_args<UnsplitArgs>(), dir, SL, SR, TL, TR, dir ? yc : c, dir ? ycell : ci, F, I, pg, tab);
         }
-        if (dir == 0 && w <= W - 2 && lane >= 1 && lane <= 62) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) { fx[w][q][lane - 1] = F[q]; fx[w][4 + q][lane - 1] = I[q]; }
-        }
-        if (dir == 1 && w >= 1 && w <= W - 2) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) { gy[yr - 1][q][yt] = F[q]; gy[yr - 1][4 + q][yt] = I[q]; }
-        }
-    }
-    __syncthreads();
-
-    // combined update and slope refresh (grp_solver_2D_EUL_source.c:231-262)
-    if (w >= 1 && w <= W - 2 && xin && yin && lane >= 1 && lane <= 62) {
         const UnsplitArgs a = reload_args<UnsplitArgs>();
-        const size_t o = G.at(c, ci);
-        const double e_c = a.st[o + 4 * a.plane];
-        double vc[4], Fl[4], Ixl[4], Fr[4], Ixr[4], Gy[4], Iy[4], Gl[4], Iyl[4];
+        const size_t o = (size_t)c * (size_t)a.ld + (size_t)ci, P = a.plane;
+        if (dir) {   // the y-faces on both sides of the lane's cell
+            const int hi = r >= 1 ? (r - 1) * (TILE_C + 1) + k : 1;
+            double dI[4], tn[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                dG[q] = __shfl(F[q], hi) - __shfl(F[q], hi - 1);
+                dI[q] = __shfl(I[q], hi) - __shfl(I[q], hi - 1);
+            }
+            if (own) {
+                quot4(dI, a.div_hy, tn);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) a.t_o[o + q * P] = tn[q];
+            }
+            continue;
+        }
+        // combined update and slope refresh (grp_solver_2D_EUL_source.c:231-262)
+        double dF[4], dI[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            vc[q] = sd[w][q][lane];
-            Fl[q] = fx[w - 1][q][lane - 1]; Ixl[q] = fx[w - 1][4 + q][lane - 1];
-            Fr[q] = fx[w][q][lane - 1];     Ixr[q] = fx[w][4 + q][lane - 1];
-            Gl[q] = gy[w - 1][q][lane - 1]; Iyl[q] = gy[w - 1][4 + q][lane - 1];
-            Gy[q] = gy[w - 1][q][lane];     Iy[q] = gy[w - 1][4 + q][lane];
+            dF[q] = F[q] - __shfl_up(F[q], 8);
+            dI[q] = I[q] - __shfl_up(I[q], 8);
         }
-        const double nu = a.nu, mu = a.mu;
-        const double mom_x = vc[0] * vc[1] - nu * (Fr[1] - Fl[1]) - mu * (Gy[1] - Gl[1]);
-        const double mom_y = vc[0] * vc[2] - nu * (Fr[2] - Fl[2]) - mu * (Gy[2] - Gl[2]);
-        const double ene = vc[0] * e_c - nu * (Fr[3] - Fl[3]) - mu * (Gy[3] - Gl[3]);
-        const double rho = vc[0] + (-nu * (Fr[0] - Fl[0]) - mu * (Gy[0] - Gl[0]));
-        double uu, vv, e_new, dx[4], dy[4], sn[4], tn[4];
-        quot3(mom_x, mom_y, ene, rho, uu, vv, e_new);
-        const double p = (ene - 0.5 * mom_x * uu - 0.5 * mom_y * vv) * a.gas.gm1();
-        double *fo = a.st_o + o;
-        const size_t P = a.plane;
-        fo[0] = rho; fo[P] = uu; fo[2 * P] = vv; fo[4 * P] = e_new; fo[3 * P] = p;
-        if (p < a.eps || rho < a.eps) atomicOr(&a.status[0].flags, 1u);
+        if (own) {
+            const double e_c = a.st[o + 4 * P];
+            double vc[4], sn[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) { dx[q] = Ixr[q] - Ixl[q]; dy[q] = Iy[q] - Iyl[q]; }
-        quot4(dx, a.div_hx, sn);
-        quot4(dy, a.div_hy, tn);
+            for (int q = 0; q < 4; ++q) vc[q] = sd[q][id0];
+            const double nu = a.nu, mu = a.mu;
+            const double mom_x = vc[0] * vc[1] - nu * dF[1] - mu * dG[1];
+            const double mom_y = vc[0] * vc[2] - nu * dF[2] - mu * dG[2];
+            const double ene = vc[0] * e_c - nu * dF[3] - mu * dG[3];
+            const double rho = vc[0] + (-nu * dF[0] - mu * dG[0]);
+            double uu, vv, e_new;
+            quot3(mom_x, mom_y, ene, rho, uu, vv, e_new);
+            const double p = (ene - 0.5 * mom_x * uu - 0.5 * mom_y * vv) * a.gas.gm1();
+            double *fo = a.st_o + o;
+            fo[0] = rho; fo[P] = uu; fo[2 * P] = vv; fo[4 * P] = e_new; fo[3 * P] = p;
+            if (p < a.eps || rho < a.eps) atomicOr(&a.status[0].flags, 1u);
+            quot4(dI, a.div_hx, sn);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) { a.s_o[o + q * P] = sn[q]; a.t_o[o + q * P] = tn[q]; }
+            for (int q = 0; q < 4; ++q) a.s_o[o + q * P] = sn[q];
+        }
     }
 }
 
-template <int W, int MINW, int NM>
-__global__ void __launch_bounds__(64 * W, MINW) unsplit_step_kernel(UnsplitArgs a)
+// CU_WAVES: the waves that the register budget lets a CU hold; TILE_WAVES: the
+// waves that share a tile.
+template <int CU_WAVES, int TILE_WAVES, int NM>
+__global__ void __launch_bounds__(256, CU_WAVES / 4) unsplit_step_kernel(UnsplitArgs a, int per_row)
 {
-    unsplit_step_body<W, NM, false>(a);
+    static_assert(TILE_WAVES == 1, "a tile belongs to one wave");
+    unsplit_step_body<NM, false>(a, per_row);
 }
 
 // the same step with GRP_2D_flux's alternative interface solver, G2D
-template <int W, int MINW, int NM>
-__global__ void __launch_bounds__(64 * W, MINW) unsplit_step_g2d_kernel(UnsplitArgs a)
+template <int CU_WAVES, int TILE_WAVES, int NM>
+__global__ void __launch_bounds__(256, CU_WAVES / 4) unsplit_step_g2d_kernel(UnsplitArgs a, int per_row)
 {
-    unsplit_step_body<W, NM, true>(a);
+    static_assert(TILE_WAVES == 1, "a tile belongs to one wave");
+    unsplit_step_body<NM, true>(a, per_row);
 }
 
 // Strip form: one wave per block walks down R cell rows of a 62-cell strip
@@ -505,16 +516,9 @@ __global__ void __launch_bounds__(64, 2) unsplit_strip_g2d_kernel(UnsplitArgs a,
 // Two forms: the tile (TILE_W waves, TILE_W - 2 updated rows per block) and the
 // strip (one wave per block walking down its rows).  The context picks one
 // (hgrp2d_set_unsplit_form, hgrp2d_tune) or takes the default (form 0: the tile).
-// The tile is 12 waves tall: 160 KiB of LDS (with the pow tables; the network
-// inputs lie in the x results' slots), one block per CU, 168 VGPRs
-// (15-18 spilled; 39-77 in the G2D and learned forms) for 3 waves per SIMD.
-// Against 8 waves (6 rows, 100 KiB, 192 VGPRs, 2 waves per SIMD) its halo rows
-// are 1 in 6 instead of 1 in 4: at 1024^2 the whole run takes 602 instead of
-// 696 ms (the reference's Newton setting), 667 instead of 706 ms (learned),
-// 679 instead of 726 ms (G2D); 10 waves gave 626, 696 and 710 ms, 6 waves
-// (3 waves per SIMD, 4 rows) 854 ms.
-constexpr int TILE_W = 12;
-
+// The tile's register budget is three waves per SIMD (168 VGPRs, 4-83 spilled;
+// 38 KiB of LDS for the 4 waves of a block): with two waves and no spills a step
+// of 1024^2 takes .333 instead of .283 ms, with four .360.
 // rows per strip of the strip form: enough strips to give every CU several waves
 static int strip_rows(int m, int n)
 {
@@ -524,10 +528,7 @@ static int strip_rows(int m, int n)
     return R;
 }
 
-// Form 0 and 1: the tile; 2: the strip.  On MI355X the 12-wave tile is the
-// faster at every size measured (four-quadrant, the reference's Newton
-// setting, per step from t = 0: 1024^2 0.207 against 0.313 ms, 2048^2 0.698
-// against 0.837 ms, 4096^2 2.467 against 2.88 ms).
+// Form 0 and 1: the tile, which is the faster at every size measured; 2: the strip.
 static bool use_strip(int, int, int form) { return form == 2; }
 
 int unsplit_max_rows() { return 65535 * 4; }   // grid.y of the strip form at R = 4
@@ -541,9 +542,11 @@ static hipError_t launch_unsplit(const UnsplitArgs &a, hipStream_t st)
         if (G2) hipLaunchKernelGGL(unsplit_strip_g2d_kernel<NM>, grid, dim3(64), 0, st, a, R);
         else hipLaunchKernelGGL(unsplit_strip_kernel<NM>, grid, dim3(64), 0, st, a, R);
     } else {
-        const dim3 grid((unsigned)((a.n + 61) / 62), (unsigned)((a.m + TILE_W - 3) / (TILE_W - 2)));
-        if (G2) hipLaunchKernelGGL((unsplit_step_g2d_kernel<TILE_W, 1, NM>), grid, dim3(64 * TILE_W), 0, st, a);
-        else hipLaunchKernelGGL((unsplit_step_kernel<TILE_W, 1, NM>), grid, dim3(64 * TILE_W), 0, st, a);
+        const int per_row = (a.n + TILE_C - 1) / TILE_C;
+        const long tiles = (long)((a.m + TILE_R - 1) / TILE_R) * per_row;
+        const dim3 grid((unsigned)((tiles + 3) / 4));
+        if (G2) hipLaunchKernelGGL((unsplit_step_g2d_kernel<12, 1, NM>), grid, dim3(256), 0, st, a, per_row);
+        else hipLaunchKernelGGL((unsplit_step_kernel<12, 1, NM>), grid, dim3(256), 0, st, a, per_row);
     }
     return hipGetLastError();
 }

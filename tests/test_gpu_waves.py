@@ -61,3 +61,19 @@ def test_two_fluid_layout_edges(hg, oracle, m, n):
         finally:
             c.close()
     assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("g2d", [False, True], ids=["Q1D", "G2D"])
+@pytest.mark.parametrize("m,n", [(1, 1), (6, 7), (7, 8), (8, 9), (14, 31), (15, 33), (2, 40)])
+def test_unsplit_tile_edges(hg, oracle, m, n, g2d):
+    init = cases.smooth_random(m, n, m + 100 * n)
+    for bx, by in ((-4, -4), (-2, -7), (-24, -1)):
+        cfg = make_config(t_all=0.03, h_x=1 / m, h_y=1 / n, bc_x=bx, bc_y=by, split=0)
+        tp = np.array([0.0, cfg[1]])
+        fo, npo, tpo, co, st = oracle.unsplit2d(m, n, init, cfg, time_plot=tp, g2d=g2d)
+        tile, strip = (hg.run_unsplit2d(m, n, init, cfg, time_plot=tp, g2d=g2d, form=f)
+                       for f in (hg.UNSPLIT_TILE, hg.UNSPLIT_STRIP))
+        for fg, npg, tpg, cg, res in (tile, strip):
+            assert (co[5], npo, tpo[npo - 1], st) == (cg[5], npg, tpg[npg - 1], res.status), (bx, by)
+            assert parity(fg[:, npg - 1], fo[:, npo - 1]).max() <= 1e-10, (bx, by)      # glibc's pow against the device's
+        assert np.array_equal(tile[0][:, npo - 1], strip[0][:, npo - 1])
