@@ -108,8 +108,8 @@ __global__ void mlp_data_kernel(uint64_t seed, int count, double tol, float *fea
 }
 
 // ---- forward / backward ------------------------------------------------------------
-constexpr int TB = 64;                    // samples per block (one wave)
-constexpr int PSTRIDE = MLP_NP + 1;       // partial gradients + loss per block
+constexpr int TB = 64;                    // samples per wave, one per lane
+constexpr int PSTRIDE = MLP_NP + 1;       // partial gradients + loss per wave
 
 __device__ __forceinline__ float gelu_grad(float x)
 {
@@ -119,109 +119,200 @@ __device__ __forceinline__ float gelu_grad(float x)
     return s + x * s * (1.0f - s) * 2.0f * k * (1.0f + 3.0f * c * x * x);
 }
 
-// Block b handles samples start + b*TB .. +TB-1 (those < count with ok set);
-// writes the gradient of sum_s (y_s - t_s)^2 * inv_b and the sum of squared
-// errors to partial[b].
-__global__ void __launch_bounds__(TB) mlp_fwdbwd_kernel(const float *__restrict__ P, const float *__restrict__ feat,
-                                                        const float *__restrict__ target, const int *__restrict__ ok,
-                                                        int count, int start, float inv_b, float *partial)
+// One wave's LDS: per-sample rows of 36 words, so that a lane writes and reads
+// four neighbouring entries at once.
+constexpr int ROW = MLP_H + 4;
+struct WaveRows {
+    float h1[TB][ROW], g1[TB][ROW], h2[TB][ROW], g2[TB][ROW], x[TB][MLP_IN + 1], dy[TB], loss[TB];
+};
+__device__ __forceinline__ float4 ld4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
+__device__ __forceinline__ void st4(float *p, const float v[4])
 {
-    __shared__ float w[MLP_NP];
-    // per-sample rows, padded by one word so that a column walk is conflict-free
-    __shared__ float sx[TB][MLP_IN + 1], sh1[TB][MLP_H + 1], sg1[TB][MLP_H + 1], sh2[TB][MLP_H + 1],
-        sg2[TB][MLP_H + 1];
-    __shared__ float sdy[TB], sloss[TB];
-    const int t = threadIdx.x;
-    for (int p = t; p < MLP_NP; p += TB) {
+    *reinterpret_cast<float4 *>(p) = make_float4(v[0], v[1], v[2], v[3]);
+}
+
+// Wave b handles samples start + b*TB .. +TB-1 (those < count with ok set);
+// writes the gradient of sum_s (y_s - t_s)^2 * inv_b and the sum of squared
+// errors to partial[b], b < nb.  Every sum is taken in index order.
+// The layers' products run four outputs at a time: one 16-byte LDS read serves
+// four of them (weights, the same for all lanes) or the four rows' (a lane's
+// 4 x 4 block of W2's gradient, summed over the samples), and the four sums
+// hide each other's latency.  Four waves to a block share the weights: 158 KiB of
+// LDS, one block to a CU and so 1024 waves at once, where blocks of one wave (44
+// KiB) fit only three times.  65536 samples: 35 us (62 by single waves; 122 with
+// one LDS word per product), 8192: 31 (32).
+constexpr int WAVES = 4;
+__global__ void __launch_bounds__(TB * WAVES) mlp_fwdbwd_kernel(const float *__restrict__ P, const float *__restrict__ feat,
+                                                                const float *__restrict__ target,
+                                                                const int *__restrict__ ok, int count, int start,
+                                                                float inv_b, float *partial, int nb)
+{
+    __shared__ __attribute__((aligned(16))) float w[(MLP_NP + 3) / 4 * 4];
+    __shared__ __attribute__((aligned(16))) WaveRows rows[WAVES];
+    for (int p = threadIdx.x; p < MLP_NP; p += TB * WAVES) {
         const float v = P[p];
         const bool bias = (p >= MLP_OFF_B1 && p < MLP_OFF_W2) || (p >= MLP_OFF_B2 && p < MLP_OFF_W3) || p == MLP_OFF_B3;
         w[p] = bias ? v : bf16_value(v);
     }
     __syncthreads();
 
-    const long s = (long)start + (long)blockIdx.x * TB + t;
-    const bool valid = s < count && (ok == nullptr || ok[s] != 0);
+    const int t = threadIdx.x & (TB - 1);
+    const long wave = (long)blockIdx.x * WAVES + threadIdx.x / TB;
+    WaveRows &W = rows[threadIdx.x / TB];
+    const long s = (long)start + wave * TB + t;
+    const bool valid = wave < nb && s < count && (ok == nullptr || ok[s] != 0);
     float x[MLP_IN], y = 0.f;
 #pragma unroll
     for (int k = 0; k < MLP_IN; ++k) {
         const float v = valid ? feat[s * MLP_IN + k] : 0.f;
         const float hi = bf16_value(v);
         x[k] = hi + bf16_value(v - hi);
-        sx[t][k] = x[k];
+        W.x[t][k] = x[k];
     }
     if (valid) y = target[s];
-    // forward; sg1 / sg2 first hold GELU'(a1) / GELU'(a2)
-    for (int o = 0; o < MLP_H; ++o) {
-        float acc = w[MLP_OFF_B1 + o];
+    // forward; g1 / g2 first hold GELU'(a1) / GELU'(a2)
+#pragma unroll 1
+    for (int o = 0; o < MLP_H; o += 4) {
+        float h[4], g[4];
 #pragma unroll
-        for (int k = 0; k < MLP_IN; ++k) acc += w[MLP_OFF_W1 + o * MLP_IN + k] * x[k];
-        sh1[t][o] = bf16_value(gelu_f(acc));
-        sg1[t][o] = gelu_grad(acc);
+        for (int j = 0; j < 4; ++j) {
+            float acc = w[MLP_OFF_B1 + o + j];
+#pragma unroll
+            for (int k = 0; k < MLP_IN; ++k) acc += w[MLP_OFF_W1 + (o + j) * MLP_IN + k] * x[k];
+            h[j] = bf16_value(gelu_f(acc));
+            g[j] = gelu_grad(acc);
+        }
+        st4(&W.h1[t][o], h);
+        st4(&W.g1[t][o], g);
+    }
+    float v[MLP_H];                           // the lane's row: h1, then g2
+#pragma unroll
+    for (int i = 0; i < MLP_H; i += 4) {
+        const float4 q = ld4(&W.h1[t][i]);
+        v[i] = q.x; v[i + 1] = q.y; v[i + 2] = q.z; v[i + 3] = q.w;
     }
     float yhat = w[MLP_OFF_B3];
-    for (int o = 0; o < MLP_H; ++o) {
-        float acc = w[MLP_OFF_B2 + o];
-#pragma unroll 8
-        for (int i = 0; i < MLP_H; ++i) acc += w[MLP_OFF_W2 + o * MLP_H + i] * sh1[t][i];
-        const float h2 = gelu_f(acc);
-        sh2[t][o] = h2;
-        sg2[t][o] = gelu_grad(acc);
-        yhat += w[MLP_OFF_W3 + o] * h2;
+#pragma unroll 1
+    for (int o = 0; o < MLP_H; o += 4) {
+        float acc[4], h[4], g[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[j] = w[MLP_OFF_B2 + o + j];
+#pragma unroll
+        for (int i = 0; i < MLP_H; i += 4) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float4 q = ld4(&w[MLP_OFF_W2 + (o + j) * MLP_H + i]);
+                acc[j] += q.x * v[i];
+                acc[j] += q.y * v[i + 1];
+                acc[j] += q.z * v[i + 2];
+                acc[j] += q.w * v[i + 3];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            h[j] = gelu_f(acc[j]);
+            g[j] = gelu_grad(acc[j]);
+            yhat += w[MLP_OFF_W3 + o + j] * h[j];
+        }
+        st4(&W.h2[t][o], h);
+        st4(&W.g2[t][o], g);
     }
     // backward (the bf16 roundings pass gradients straight through)
     const float r = valid ? yhat - y : 0.f;
     const float dy = 2.0f * r * inv_b;
-    for (int o = 0; o < MLP_H; ++o) sg2[t][o] = dy * w[MLP_OFF_W3 + o] * sg2[t][o];
-    for (int i = 0; i < MLP_H; ++i) {
-        float acc = 0.f;
-#pragma unroll 8
-        for (int o = 0; o < MLP_H; ++o) acc += w[MLP_OFF_W2 + o * MLP_H + i] * sg2[t][o];
-        sg1[t][i] = acc * sg1[t][i];
+#pragma unroll
+    for (int o = 0; o < MLP_H; o += 4) {
+        const float4 q = ld4(&W.g2[t][o]);
+        v[o] = dy * w[MLP_OFF_W3 + o] * q.x;
+        v[o + 1] = dy * w[MLP_OFF_W3 + o + 1] * q.y;
+        v[o + 2] = dy * w[MLP_OFF_W3 + o + 2] * q.z;
+        v[o + 3] = dy * w[MLP_OFF_W3 + o + 3] * q.w;
+        st4(&W.g2[t][o], &v[o]);
     }
-    sdy[t] = dy;
-    sloss[t] = r * r;
-    __syncthreads();
-
-    float *out = partial + (size_t)blockIdx.x * PSTRIDE;
-    for (int p = t; p < MLP_NP; p += TB) {
-        float acc = 0.f;
-        if (p < MLP_OFF_B1) {
-            const int o = p / MLP_IN, k = p % MLP_IN;
-            for (int q = 0; q < TB; ++q) acc += sg1[q][o] * sx[q][k];
-        } else if (p < MLP_OFF_W2) {
-            const int o = p - MLP_OFF_B1;
-            for (int q = 0; q < TB; ++q) acc += sg1[q][o];
-        } else if (p < MLP_OFF_B2) {
-            const int o = (p - MLP_OFF_W2) / MLP_H, i = (p - MLP_OFF_W2) % MLP_H;
-            for (int q = 0; q < TB; ++q) acc += sg2[q][o] * sh1[q][i];
-        } else if (p < MLP_OFF_W3) {
-            const int o = p - MLP_OFF_B2;
-            for (int q = 0; q < TB; ++q) acc += sg2[q][o];
-        } else if (p < MLP_OFF_B3) {
-            const int o = p - MLP_OFF_W3;
-            for (int q = 0; q < TB; ++q) acc += sdy[q] * sh2[q][o];
-        } else {
-            for (int q = 0; q < TB; ++q) acc += sdy[q];
+#pragma unroll 1
+    for (int i = 0; i < MLP_H; i += 4) {
+        float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int o = 0; o < MLP_H; ++o) {
+            const float4 q = ld4(&w[MLP_OFF_W2 + o * MLP_H + i]);
+            acc[0] += q.x * v[o];
+            acc[1] += q.y * v[o];
+            acc[2] += q.z * v[o];
+            acc[3] += q.w * v[o];
         }
-        out[p] = acc;
+        const float4 g = ld4(&W.g1[t][i]);
+        acc[0] *= g.x; acc[1] *= g.y; acc[2] *= g.z; acc[3] *= g.w;
+        st4(&W.g1[t][i], acc);
     }
-    if (t == 0) {
-        float l = 0.f;
-        for (int q = 0; q < TB; ++q) l += sloss[q];
-        out[MLP_NP] = l;
+    W.dy[t] = dy;
+    W.loss[t] = r * r;
+    __syncthreads();
+    if (wave >= nb) return;
+
+    // Sums over the wave's samples.  Lane t: W2[o0 .. o0+3][i0 .. i0+3]; W1's entries t, t + 64,
+    // t + 128; b1 (lanes 0-31) or b2 (32-63); w3 (0-31); b3 (even lanes) or the loss (odd).
+    const int o0 = (t >> 3) * 4, i0 = (t & 7) * 4, o = t & 31;
+    float a2[4][4] = {}, a1[3] = {0.f, 0.f, 0.f}, ab = 0.f, a3 = 0.f, as = 0.f;
+    int w1o[3], w1k[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) { w1o[j] = (t + 64 * j) / MLP_IN; w1k[j] = (t + 64 * j) % MLP_IN; }
+    const float *bias = t < 32 ? &W.g1[0][o] : &W.g2[0][o], *sum = t & 1 ? W.loss : W.dy;
+#pragma unroll 4
+    for (int q = 0; q < TB; ++q) {
+        const float4 g4 = ld4(&W.g2[q][o0]), h4 = ld4(&W.h1[q][i0]);
+        const float g[4] = {g4.x, g4.y, g4.z, g4.w}, h[4] = {h4.x, h4.y, h4.z, h4.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) a2[j][i] += g[j] * h[i];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) a1[j] += W.g1[q][w1o[j]] * W.x[q][w1k[j]];
+        ab += bias[q * ROW];
+        a3 += W.dy[q] * W.h2[q][o];
+        as += sum[q];
     }
+    float *out = partial + (size_t)wave * PSTRIDE;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) out[MLP_OFF_W2 + (o0 + j) * MLP_H + i0 + i] = a2[j][i];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) out[MLP_OFF_W1 + t + 64 * j] = a1[j];
+    out[(t < 32 ? MLP_OFF_B1 : MLP_OFF_B2) + o] = ab;
+    if (t < 32) out[MLP_OFF_W3 + o] = a3;
+    if (t < 2) out[t ? MLP_NP : MLP_OFF_B3] = as;
 }
 
-// Sums the per-block partials in block order (deterministic).  mode 0: Adam
-// step on P; mode 1: write the gradient to grad.  The loss sum is added to
-// *loss_acc.
-__global__ void mlp_adam_kernel(const float *__restrict__ partial, int nblocks, float *P, float *m1, float *m2,
-                                float lr, float bc1, float bc2, int mode, float *grad, float *loss_acc)
+static void launch_fwdbwd(hipStream_t st, const float *P, const float *feat, const float *target, const int *ok, int count,
+                          int start, float inv_b, float *partial, int nb)
+{
+    hipLaunchKernelGGL(mlp_fwdbwd_kernel, dim3((nb + WAVES - 1) / WAVES), dim3(TB * WAVES), 0, st, P, feat, target, ok,
+                       count, start, inv_b, partial, nb);
+}
+
+// Sums the per-wave partials in order (deterministic).  mode 0: Adam step on P;
+// mode 1: write the gradient to grad.  The loss sum is added to *loss_acc.  One
+// dependent sum per parameter, so what bounds it is the latency of its loads:
+// 64 of them go out before their sums (1024 partials: 232 -> 22 us, one at a time
+// before), and a wave to a block spreads them over as many CUs.
+constexpr int ADAM_BLOCK = 64;
+__global__ void __launch_bounds__(ADAM_BLOCK) mlp_adam_kernel(const float *__restrict__ partial, int nblocks, float *P,
+                                                              float *m1, float *m2, float lr, float bc1, float bc2,
+                                                              int mode, float *grad, float *loss_acc)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p > MLP_NP) return;
+    constexpr int DEEP = 64;
     float g = 0.f;
-    for (int b = 0; b < nblocks; ++b) g += partial[(size_t)b * PSTRIDE + p];
+    int b = 0;
+    for (; b + DEEP <= nblocks; b += DEEP) {
+        float v[DEEP];
+#pragma unroll
+        for (int k = 0; k < DEEP; ++k) v[k] = partial[(size_t)(b + k) * PSTRIDE + p];
+#pragma unroll
+        for (int k = 0; k < DEEP; ++k) g += v[k];
+    }
+    for (; b < nblocks; ++b) g += partial[(size_t)b * PSTRIDE + p];
     if (p == MLP_NP) { *loss_acc += g; return; }
     if (mode == 1) { grad[p] = g; return; }
     const float a = 0.9f * m1[p] + 0.1f * g;
@@ -314,11 +405,10 @@ extern "C" int hgrp_mlp_loss_grad(const float *params, const float *feat, const 
     MCHECK(hipMemcpy(df.p, feat, (size_t)count * MLP_IN * 4, hipMemcpyHostToDevice));
     MCHECK(hipMemcpy(dt.p, target, (size_t)count * 4, hipMemcpyHostToDevice));
     MCHECK(hipMemset(dl.p, 0, 4));
-    hipLaunchKernelGGL(mlp_fwdbwd_kernel, dim3(nb), dim3(TB), 0, 0, dp.p, df.p, dt.p, (const int *)nullptr, count, 0,
-                       1.0f / (float)count, part.p);
+    launch_fwdbwd(0, dp.p, df.p, dt.p, nullptr, count, 0, 1.0f / (float)count, part.p, nb);
     MCHECK(hipGetLastError());
-    hipLaunchKernelGGL(mlp_adam_kernel, dim3((MLP_NP + 1 + 255) / 256), dim3(256), 0, 0, part.p, nb, dp.p,
-                       (float *)nullptr, (float *)nullptr, 0.f, 1.f, 1.f, 1, dg.p, dl.p);
+    hipLaunchKernelGGL(mlp_adam_kernel, dim3((MLP_NP + ADAM_BLOCK) / ADAM_BLOCK), dim3(ADAM_BLOCK), 0, 0, part.p, nb,
+                       dp.p, (float *)nullptr, (float *)nullptr, 0.f, 1.f, 1.f, 1, dg.p, dl.p);
     MCHECK(hipGetLastError());
     MCHECK(hipDeviceSynchronize());
     MCHECK(hipMemcpy(grad, dg.p, MLP_NP * 4, hipMemcpyDeviceToHost));
@@ -416,10 +506,9 @@ extern "C" int hgrp_mlp_train(unsigned long long seed, int n_samples, int epochs
             const double lr_t = lr_min + 0.5 * (lr - lr_min) * (1.0 + cos(M_PI * (double)t / (double)total));
             const float bc1 = (float)(1.0 - pow(0.9, (double)(t + 1)));
             const float bc2 = (float)(1.0 - pow(0.999, (double)(t + 1)));
-            hipLaunchKernelGGL(mlp_fwdbwd_kernel, dim3(nb), dim3(TB), 0, st, dp.p, df.p, dt.p, dk.p, n_samples,
-                               s * batch, 1.0f / (float)batch, part.p);
-            hipLaunchKernelGGL(mlp_adam_kernel, dim3((MLP_NP + 1 + 255) / 256), dim3(256), 0, st, part.p, nb, dp.p,
-                               m1.p, m2.p, (float)lr_t, bc1, bc2, 0, (float *)nullptr, dl.p + e);
+            launch_fwdbwd(st, dp.p, df.p, dt.p, dk.p, n_samples, s * batch, 1.0f / (float)batch, part.p, nb);
+            hipLaunchKernelGGL(mlp_adam_kernel, dim3((MLP_NP + ADAM_BLOCK) / ADAM_BLOCK), dim3(ADAM_BLOCK), 0, st,
+                               part.p, nb, dp.p, m1.p, m2.p, (float)lr_t, bc1, bc2, 0, (float *)nullptr, dl.p + e);
         }
         MCHECK(hipGetLastError());
     }
