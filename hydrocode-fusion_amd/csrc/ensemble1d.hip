@@ -204,7 +204,7 @@ __device__ __forceinline__ int wave_index()
     return __builtin_amdgcn_readfirstlane((int)((blockIdx.x * BS + threadIdx.x) >> 6));
 }
 
-// four waves per SIMD: 128 VGPRs and a 4-register spill (unbounded it takes 130, three waves);
+// four waves per SIMD: 128 VGPRs and a few spilled (unbounded it takes 130, three waves);
 // measured 5 % faster on the 512-instance ensemble
 template <int BS>
 __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) iface_kernel(Tables T, int n_w, Inst *inst, Params P, const double *rho,

@@ -513,12 +513,13 @@ __global__ void __launch_bounds__(64, 2) unsplit_strip_g2d_kernel(UnsplitArgs a,
 }
 
 // ---- launchers -----------------------------------------------------------------
-// Two forms: the tile (TILE_W waves, TILE_W - 2 updated rows per block) and the
+// Two forms: the tile (TILE_R x TILE_C cells to a wave) and the
 // strip (one wave per block walking down its rows).  The context picks one
 // (hgrp2d_set_unsplit_form, hgrp2d_tune) or takes the default (form 0: the tile).
 // The tile's register budget is three waves per SIMD (168 VGPRs, 4-83 spilled;
 // 38 KiB of LDS for the 4 waves of a block): with two waves and no spills a step
 // of 1024^2 takes .333 instead of .283 ms, with four .360.
+
 // rows per strip of the strip form: enough strips to give every CU several waves
 static int strip_rows(int m, int n)
 {

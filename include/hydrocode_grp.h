@@ -148,7 +148,7 @@ int hgrp2d_set_newton(hgrp2d *ctx, double tol, int rule, const float *params);
  * hgrp_g2d_batch).  A split context (config[33] != 0) takes Q1D only: -1002
  * and a message for G2D.  Works with every Newton setting of hgrp2d_set_newton. */
 /* Launch form of the unsplit step (no counterpart in the reference): TILE
- * blocks of 12 waves over 10 x 62 updated cells, STRIP one wave per 62-cell
+ * one wave per 7 x 8 updated cells, STRIP one wave per 62-cell
  * strip walking down its rows; AUTO takes the tile, the faster at every size
  * measured on MI355X.  hgrp2d_tune on an unsplit context times both and keeps
  * the faster.  Results do not depend on the form. */
@@ -213,7 +213,7 @@ int hgrp2db_upload(hgrp2db *ctx, const double *rho, const double *u, const doubl
 /* As hgrp2d_set_newton, for every grid. */
 int hgrp2db_set_newton(hgrp2db *ctx, double tol, int rule, const float *params);
 
-/* Launch variants as hgrp2d_set_sweeps (the same numbering). */
+/* Launch variants as hgrp2d_set_sweeps (the same numbering, X 0..4, Y 0..4). */
 int hgrp2db_set_sweeps(hgrp2db *ctx, int x_variant, int y_variant);
 
 /* Times every X variant, then every Y variant, over the first `steps` steps
