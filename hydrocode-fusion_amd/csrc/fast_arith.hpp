@@ -10,7 +10,10 @@
 // rounds the exact remainder's correction (Markstein).  A quotient is then 3
 // operations once the divisor's reciprocal is known, and several quotients by
 // one divisor share it (Rcp); a fresh reciprocal is the seed and 4 operations,
-// a square root the seed and 9, its reciprocal 3 more.
+// a square root the seed and 9.  A root that is a divisor takes a reciprocal of
+// its own: what the root's steps leave of 1/sqrt(x) is not rounded right for a
+// root just below a power of two (1/(2 - j 2^-52) lies j^2 2^-107 above the
+// middle of two doubles for odd j), and some quotients by it end an ulp off.
 //
 // In range means: divisors and radicands in [2^-700, 2^700], numerators zero
 // or in [2^-900, 2^900], quotients in [2^-900, 2^900].  The quotient of a zero
@@ -73,8 +76,7 @@ HGRP_HD double recip_q(const Rcp &r) { return fma(-fma(r.y, r.b, -1.0), r.y, r.y
 HGRP_HD double recip_1(double b) { return recip_q(rcp_of(b)); }
 HGRP_HD double div_1(double a, double b) { return div_q(a, rcp_of(b)); }
 
-// sqrt(x); *half_inv receives 1/(2 sqrt(x)) to about 2^-47
-HGRP_HD double sqrt_h(double x, double *half_inv)
+HGRP_HD double sqrt_q(double x)
 {
     const double y = rsq_seed(x);
     double s = x * y, h = 0.5 * y;
@@ -82,24 +84,7 @@ HGRP_HD double sqrt_h(double x, double *half_inv)
     h = fma(h, r, h);
     s = fma(s, r, s);
     s = fma(fma(-s, s, x), h, s);
-    s = fma(fma(-s, s, x), h, s);
-    *half_inv = h;
-    return s;
-}
-HGRP_HD double sqrt_q(double x)
-{
-    double h;
-    return sqrt_h(x, &h);
-}
-// sqrt(x) as a divisor, x >= 1: its reciprocal, rounded, comes from the root's
-// own seed (2^-94 before the rounding; no root from 1 up has a reciprocal so
-// close to the middle of two doubles)
-HGRP_HD Rcp sqrt_rcp(double x)
-{
-    double h;
-    const double s = sqrt_h(x, &h);
-    const double y = h + h;
-    return {s, fma(y, fma(-s, y, 1.0), y)};
+    return fma(fma(-s, s, x), h, s);
 }
 
 // log_dd and exp_dd (fastpow.hpp) with every operation that changes nothing

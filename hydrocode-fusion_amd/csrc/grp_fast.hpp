@@ -78,8 +78,8 @@ HGRP_HD bool gas_in_range(const Gas &G) { return G.gm1() >= 0x1p-20 && G.g <= 0x
 // ---- the exact Riemann solve ---------------------------------------------------------
 // What the wave curve leaves for the Newton slope at the same pressure and, from
 // the last one, for the state behind the wave: on the rarefaction branch
-// l = log(p/p_s) and m = (p/p_s)^mu; on the shock branch m = 0 and
-// l.hi = 1/sqrt(1 + nu (p - p_s)/p_s).
+// l = log(p/p_s) and m = (p/p_s)^mu; on the shock branch m = 0 and l is
+// sqrt(1 + nu (p - p_s)/p_s) with its reciprocal (an Rcp).
 struct Keep {
     DD l;
     double m;
@@ -90,8 +90,8 @@ HGRP_HD double curve_q(double p, double u_s, const Rcp &p_s, double c_s, const G
     double w;
     if (p > p_s.b) {
         const double dp = p - p_s.b;
-        const Rcp s = sqrt_rcp(1.0 + div_q(G.nu * dp, p_s));
-        keep->l.hi = s.y;
+        const Rcp s = rcp_of(sqrt_q(1.0 + div_q(G.nu * dp, p_s)));
+        keep->l = {s.b, s.y};
         keep->m = 0.0;
         w = div_q(div_q(div_q(dp * c_s, {G.g, G.inv_g}), p_s), s);
     } else {
@@ -108,7 +108,7 @@ HGRP_HD double slope_q(double p, const Rcp &p_s, double c_s, const Gas &G, const
 {
     const double t2 = div_q(div_q(c_s, {G.g, G.inv_g}), p_s);
     if (p > p_s.b) {
-        const double t1 = keep.l.hi;
+        const double t1 = recip_q({keep.l.hi, keep.l.lo});
         const double t3 = div_q(0.5 * t2 * G.nu, p_s);
         return t2 * t1 - t3 * (p - p_s.b) * cube(t1);
     }

@@ -1,0 +1,52 @@
+"""The steps' interface solver (csrc/grp_fast.hpp) against the IEEE solver, both
+built for the host, bit for bit (a zero's sign aside), where random interfaces
+do not lead: wave curves whose root lies just below a power of two."""
+import ctypes as C
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from _libs import ROOT
+
+INC = [os.path.join(ROOT, "tests", "native", "shim"), os.path.join(ROOT, "hydrocode-fusion_amd", "csrc")]
+
+
+def _build(tmp_path_factory, name):
+    so = str(tmp_path_factory.mktemp(name) / f"{name}.so")
+    subprocess.run(["g++", "-std=c++17", "-O2", "-ffp-contract=off", "-fPIC", "-shared", *[f"-I{d}" for d in INC],
+                    os.path.join(ROOT, "tests", "native", f"{name}.cpp"), "-o", so], check=True)
+    return C.CDLL(so)
+
+
+@pytest.fixture(scope="module")
+def fast(tmp_path_factory):
+    return _build(tmp_path_factory, "fast_host")
+
+
+def _dp(a):
+    return a.ctypes.data_as(C.POINTER(C.c_double))
+
+
+def _split(lib, L, R, direction, conv, guess, tau=1e-3, eps=1e-9):
+    L, R, guess = (np.ascontiguousarray(a) for a in (L, R, guess))
+    f, i = np.full((len(L), 9), np.nan), np.zeros((len(L), 9))
+    took = lib.fh_split_many(_dp(L), _dp(R), len(L), C.c_double(tau), C.c_double(eps), direction, conv, _dp(guess),
+                             _dp(f), _dp(i))
+    return took, f, i
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 4])
+def test_shock_curve_roots_below_powers_of_two(fast, k):
+    """gamma = 2 and p_R = 1: 1 + nu (p - p_R)/p_R is 4^k at p = 1 + (4^k - 1)/0.75.
+    Newton starts at the doubles just below that pressure."""
+    n, rng = 40000, np.random.default_rng(k)
+    p0 = 1.0 + (4.0 ** k - 1.0) / 0.75
+    L, R = np.zeros((n, 15)), np.zeros((n, 15))
+    for A in (L, R):
+        A[:, 0], A[:, 3], A[:, 4] = 2.0, rng.uniform(0.5, 2, n), rng.uniform(-1, 1, n)
+        A[:, 7:11] = rng.uniform(-1, 1, (n, 4))
+    R[:, 6], L[:, 6] = 1.0, rng.uniform(p0, 2.4 * p0, n)
+    took, f, i = _split(fast, L, R, 0, 1, p0 - rng.integers(1, 36, n) * np.spacing(np.nextafter(p0, 0.0)))
+    assert took == n and np.array_equal(f, i)
