@@ -171,7 +171,9 @@ HGRP_HD bool newton_q(const Gas &GL, const Gas &GR, double u_L, double u_R, cons
             break;
         }
     }
-    u = div_1(k1 * (v_R - v_L), k1 - k3) + v_L;
+    // a tolerance below the velocities themselves lets the iteration end on a tiny gap
+    const double share = k1 * (v_R - v_L);
+    u = (__builtin_expect(tiny(v_R - v_L), 0) ? share / (k1 - k3) : div_1(share, k1 - k3)) + v_L;
     return true;
 }
 

@@ -1,6 +1,7 @@
 """The steps' interface solver (csrc/grp_fast.hpp) against the IEEE solver, both
 built for the host, bit for bit (a zero's sign aside), where random interfaces
-do not lead: wave curves whose root lies just below a power of two."""
+do not lead: wave curves whose root lies just below a power of two, Newton
+iterations that end on a tiny gap."""
 import ctypes as C
 import os
 import subprocess
@@ -49,4 +50,21 @@ def test_shock_curve_roots_below_powers_of_two(fast, k):
         A[:, 7:11] = rng.uniform(-1, 1, (n, 4))
     R[:, 6], L[:, 6] = 1.0, rng.uniform(p0, 2.4 * p0, n)
     took, f, i = _split(fast, L, R, 0, 1, p0 - rng.integers(1, 36, n) * np.spacing(np.nextafter(p0, 0.0)))
+    assert took == n and np.array_equal(f, i)
+
+
+@pytest.mark.parametrize("eps", [0.0, 1e-300])
+@pytest.mark.parametrize("direction", [0, 1])
+def test_gap_of_a_few_denormals(fast, direction, eps):
+    """A tolerance below the velocities themselves: the iteration ends with the
+    curves' velocities a tiny number apart, and u* is that number's share."""
+    n, rng = 8000, np.random.default_rng(direction)
+    L, R = np.zeros((n, 15)), np.zeros((n, 15))
+    for A in (L, R):
+        A[:, 0], A[:, 3] = 1.4, rng.choice([1.0, 0.5, 1.3], n)
+        A[:, 6] = rng.choice([1.0, 0.7, 1.0 - 2.0 ** -53], n)
+        A[:, 7:11] = rng.uniform(-1, 1, (n, 4))
+        for q in (4, 5):
+            A[:, q] = np.ldexp(rng.uniform(-1, 1, n), rng.integers(-1074, 0, n)) * rng.choice([0, 0, 0, 1], n)
+    took, f, i = _split(fast, L, R, direction, 0, np.full(n, -1.0), 1.0, eps)
     assert took == n and np.array_equal(f, i)
