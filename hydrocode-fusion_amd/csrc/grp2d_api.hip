@@ -30,7 +30,7 @@ const char *sweep_kernel_name(int dir, int variant, int nm);
 int sweep_variants(int dir);
 int default_sweep(int dir, int m, int n);
 hipError_t launch_sweep_x_tf(const SweepArgs &a, hipStream_t st);
-const char *sweep_tf_kernel_name(int dir, int nm);
+const char *sweep_tf_kernel_name(int dir, int nm, int m, int n);
 hipError_t launch_sweep_y_tf(const SweepArgs &a, hipStream_t st);
 hipError_t launch_cfl_tf(const double *rho, const double *u, const double *v, const double *p, const double *fa,
                          int m, int n, int ld, const TwoGas &two, double hmin, unsigned long long *out, hipStream_t st);
@@ -206,7 +206,7 @@ extern "C" const char *hgrp2d_sweep_kernel(hgrp2d *c, int dir)
     if (!c || dir < 0 || dir > 2) return "";
     const int nm = c->use_mlp ? NM_LEARNED : c->newton_rule == HGRP_NEWTON_CONVERGE ? NM_CONV : NM_REF;
     if (dir == 2) return unsplit_kernel_name(c->m, c->n, nm, c->g2d, c->uform);
-    if (c->two_fluid) return sweep_tf_kernel_name(dir, nm);
+    if (c->two_fluid) return sweep_tf_kernel_name(dir, nm, c->m, c->n);
     return sweep_kernel_name(dir, dir == 0 ? c->xv : c->yv, nm);
 }
 

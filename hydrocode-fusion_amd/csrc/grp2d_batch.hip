@@ -149,7 +149,7 @@ static void launch_bx(const BatchSweep &b, int v, int blocks, hipStream_t st)
     case 1: hipLaunchKernelGGL((batch_x_kernel<4, NM, 32>), dim3(blocks), dim3(256), 0, st, b); break;
     case 2: hipLaunchKernelGGL((batch_x_kernel<4, NM, 8>), dim3(blocks), dim3(256), 0, st, b); break;
     case 3: hipLaunchKernelGGL((batch_x_kernel<3, NM, 16>), dim3(blocks), dim3(256), 0, st, b); break;
-    case 4: hipLaunchKernelGGL((batch_x_kernel<3, NM, 8>), dim3(blocks), dim3(256), 0, st, b); break;
+    case 4: hipLaunchKernelGGL((batch_x_kernel<4, NM, 4>), dim3(blocks), dim3(256), 0, st, b); break;
     default: hipLaunchKernelGGL((batch_x_kernel<4, NM, 16>), dim3(blocks), dim3(256), 0, st, b); break;
     }
 }
@@ -338,6 +338,11 @@ extern "C" int hgrp2db_create(hgrp2db **out, int count, const int *m, const int 
         total += (size_t)26 * m[i] * c->ld[i] + (size_t)8 * (m[i] + n[i]);
     }
     c->block_doubles = total;
+    long blocks[3] = {0, 0, 0};                         // of all grids' X sweeps, as variants 0, 2 and 4
+    for (int i = 0; i < count; ++i)
+        for (int v = 0; v < 3; ++v) blocks[v] += wave_grid(0, m[i], n[i], sweep_shape(0, 2 * v).G).blocks;
+    const int G = x_lanes(blocks[0], blocks[1], blocks[2]);
+    c->xv = G == 16 ? 0 : G == 8 ? 2 : 4;
     hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipMalloc((void **)&c->block, total * sizeof(double));
     if (e == hipSuccess) e = hipMalloc((void **)&c->grids_d, (size_t)count * sizeof(BatchGrid));

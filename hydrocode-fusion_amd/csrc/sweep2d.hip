@@ -59,6 +59,7 @@ static hipError_t launch_x(const SweepArgs &a, int v, hipStream_t st)
     switch (v) {
     case 1: hipLaunchKernelGGL((sweep_x_kernel<4, NM, 32>), grid, block, 0, st, a, w.per_row); break;
     case 2: hipLaunchKernelGGL((sweep_x_kernel<4, NM, 8>), grid, block, 0, st, a, w.per_row); break;
+    case 4: hipLaunchKernelGGL((sweep_x_kernel<4, NM, 4>), grid, block, 0, st, a, w.per_row); break;
     default: hipLaunchKernelGGL((sweep_x_kernel<4, NM, 16>), grid, block, 0, st, a, w.per_row); break;
     }
     return hipGetLastError();
@@ -104,7 +105,7 @@ const char *sweep_kernel_name(int dir, int variant, int nm)
 #define HGRP_NAMES(k, w, g) {k "<" #w ", 0, " #g ">", k "<" #w ", 1, " #g ">", k "<" #w ", 2, " #g ">"}
     static const char *xn[6][3] = {HGRP_NAMES("sweep_x_kernel", 4, 16), HGRP_NAMES("sweep_x_kernel", 4, 32),
                                    HGRP_NAMES("sweep_x_kernel", 4, 8),  HGRP_NAMES("sweep_x_kernel", 3, 16),
-                                   HGRP_NAMES("sweep_x_kernel", 3, 8),  HGRP_NAMES("sweep_x_kernel", 3, 32)};
+                                   HGRP_NAMES("sweep_x_kernel", 4, 4),  HGRP_NAMES("sweep_x_kernel", 3, 32)};
     static const char *yn[5][3] = {HGRP_NAMES("sweep_y_kernel", 4, 16), HGRP_NAMES("sweep_y_kernel", 4, 32),
                                    HGRP_NAMES("sweep_y_kernel", 4, 64), HGRP_NAMES("sweep_y_kernel", 4, 8),
                                    HGRP_NAMES("sweep_y_kernel", 3, 16)};

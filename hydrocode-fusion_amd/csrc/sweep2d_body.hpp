@@ -245,20 +245,23 @@ __device__ __forceinline__ double interface_guess(const SweepArgs &a, bool activ
 // is 2-4 % faster (384^2 .1056 against .1073, 127 x 329 .072 against .075), so that
 // is a smaller grid's default.
 // G = 16: the repeated face is 1 in 16 and a front along the lines still meets
-// few waves; G = 8 repeats 1 in 8 (1024^2: X .120 ms), G = 32 reads X lines in
-// 16-byte pieces (4096^2 learned: X 1.64 ms against 1.36).
+// few waves; G = 32 reads X lines in 16-byte pieces (4096^2 learned: X 1.64 ms
+// against 1.36).
 struct SweepShape {
     int G, minw;
 };
 inline SweepShape sweep_shape(int dir, int variant)
 {
-    static const SweepShape x[6] = {{16, 4}, {32, 4}, {8, 4}, {16, 3}, {8, 3}, {32, 3}};
+    static const SweepShape x[6] = {{16, 4}, {32, 4}, {8, 4}, {16, 3}, {4, 4}, {32, 3}};
     static const SweepShape y[5] = {{16, 4}, {32, 4}, {64, 4}, {8, 4}, {16, 3}};
     return dir == 0 ? x[variant] : y[variant];
 }
 inline int default_variant(int dir, int m, int n)
 {
-    return wave_grid(dir, m, n, 16).blocks <= 3 * 256 ? (dir == 0 ? 3 : 4) : 0;
+    if (wave_grid(dir, m, n, 16).blocks <= FEW_BLOCKS) return dir == 0 ? 3 : 4;
+    if (dir == 1) return 0;
+    const int G = x_lanes(wave_grid(0, m, n, 16).blocks, wave_grid(0, m, n, 8).blocks, wave_grid(0, m, n, 4).blocks);
+    return G == 16 ? 0 : G == 8 ? 2 : 4;
 }
 
 // Wave-parallel sweep along DIR: a wave holds 64/G grid lines of G lanes each;
@@ -280,7 +283,7 @@ template <int DIR, int MINW, int NM, int G, class Src>
 __device__ __forceinline__ void wave_sweep(const SweepArgs &a, const Src &src, long wave, int per_row,
                                            double (*st)[64], uint32_t *mlp, double *tab)
 {
-    static_assert(G == 64 || G == 32 || G == 16 || G == 8, "lanes per line");
+    static_assert(G == 64 || G == 32 || G == 16 || G == 8 || G == 4, "lanes per line");
     constexpr int LINES = 64 / G, STEP = DIR == 0 ? LINES : 1;   // STEP: lanes between neighbours along the sweep
     constexpr bool LEARNED = NM == NM_LEARNED;
     const int lane = threadIdx.x & 63, k = DIR == 0 ? lane / LINES : lane % G;

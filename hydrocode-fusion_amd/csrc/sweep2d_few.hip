@@ -15,7 +15,6 @@ static hipError_t launch_few(int dir, const SweepArgs &a, int v, hipStream_t st)
     const dim3 grid((unsigned)w.blocks), block(256);
     if (dir == 1) hipLaunchKernelGGL((sweep_y_kernel<3, NM, 16>), grid, block, 0, st, a, w.per_row);
     else if (v == 3) hipLaunchKernelGGL((sweep_x_kernel<3, NM, 16>), grid, block, 0, st, a, w.per_row);
-    else if (v == 4) hipLaunchKernelGGL((sweep_x_kernel<3, NM, 8>), grid, block, 0, st, a, w.per_row);
     else hipLaunchKernelGGL((sweep_x_kernel<3, NM, 32>), grid, block, 0, st, a, w.per_row);
     return hipGetLastError();
 }

@@ -419,25 +419,44 @@ hipError_t launch_energy_tf(const double *rho, const double *u, const double *v,
     return hipGetLastError();
 }
 
-// the two-fluid sweep kernel's name as profilers print it
-const char *sweep_tf_kernel_name(int dir, int nm)
+static int x_tf_lanes(int m, int n)
 {
-    static const char *xn[3] = {"sweep_x_tf_kernel<0, 16>", "sweep_x_tf_kernel<1, 16>", "sweep_x_tf_kernel<2, 16>"};
+    return x_lanes(wave_grid(0, m, n, 16).blocks, wave_grid(0, m, n, 8).blocks, wave_grid(0, m, n, 4).blocks);
+}
+
+// the two-fluid sweep kernel's name as profilers print it
+const char *sweep_tf_kernel_name(int dir, int nm, int m, int n)
+{
+    static const char *xn[3][3] = {
+        {"sweep_x_tf_kernel<0, 16>", "sweep_x_tf_kernel<1, 16>", "sweep_x_tf_kernel<2, 16>"},
+        {"sweep_x_tf_kernel<0, 8>", "sweep_x_tf_kernel<1, 8>", "sweep_x_tf_kernel<2, 8>"},
+        {"sweep_x_tf_kernel<0, 4>", "sweep_x_tf_kernel<1, 4>", "sweep_x_tf_kernel<2, 4>"}};
     static const char *yn[3] = {"sweep_y_tf_kernel<0, 16>", "sweep_y_tf_kernel<1, 16>", "sweep_y_tf_kernel<2, 16>"};
     if (nm < 0 || nm > 2 || dir < 0 || dir > 1) return "";
-    return dir == 0 ? xn[nm] : yn[nm];
+    const int G = x_tf_lanes(m, n);
+    return dir == 0 ? xn[G == 16 ? 0 : G == 8 ? 1 : 2][nm] : yn[nm];
+}
+
+template <int G>
+static hipError_t launch_x_tf(const SweepArgs &a, hipStream_t st)
+{
+    const WaveGrid w = wave_grid(0, a.m, a.n, G);
+    const dim3 grid((unsigned)w.blocks), block(256);
+    switch (newton_mode(a)) {
+    case NM_LEARNED: hipLaunchKernelGGL((sweep_x_tf_kernel<NM_LEARNED, G>), grid, block, 0, st, a, w.per_row); break;
+    case NM_CONV: hipLaunchKernelGGL((sweep_x_tf_kernel<NM_CONV, G>), grid, block, 0, st, a, w.per_row); break;
+    default: hipLaunchKernelGGL((sweep_x_tf_kernel<NM_REF, G>), grid, block, 0, st, a, w.per_row); break;
+    }
+    return hipGetLastError();
 }
 
 hipError_t launch_sweep_x_tf(const SweepArgs &a, hipStream_t st)
 {
-    const WaveGrid w = wave_grid(0, a.m, a.n, 16);
-    const dim3 grid((unsigned)w.blocks), block(256);
-    switch (newton_mode(a)) {
-    case NM_LEARNED: hipLaunchKernelGGL((sweep_x_tf_kernel<NM_LEARNED, 16>), grid, block, 0, st, a, w.per_row); break;
-    case NM_CONV: hipLaunchKernelGGL((sweep_x_tf_kernel<NM_CONV, 16>), grid, block, 0, st, a, w.per_row); break;
-    default: hipLaunchKernelGGL((sweep_x_tf_kernel<NM_REF, 16>), grid, block, 0, st, a, w.per_row); break;
+    switch (x_tf_lanes(a.m, a.n)) {
+    case 4: return launch_x_tf<4>(a, st);
+    case 8: return launch_x_tf<8>(a, st);
+    default: return launch_x_tf<16>(a, st);
     }
-    return hipGetLastError();
 }
 
 hipError_t launch_sweep_y_tf(const SweepArgs &a, hipStream_t st)
