@@ -258,10 +258,10 @@ inline SweepShape sweep_shape(int dir, int variant)
 }
 inline int default_variant(int dir, int m, int n)
 {
-    if (wave_grid(dir, m, n, 16).blocks <= FEW_BLOCKS) return dir == 0 ? 3 : 4;
-    if (dir == 1) return 0;
-    const int G = x_lanes(wave_grid(0, m, n, 16).blocks, wave_grid(0, m, n, 8).blocks, wave_grid(0, m, n, 4).blocks);
-    return G == 16 ? 0 : G == 8 ? 2 : 4;
+    const long b16 = wave_grid(dir, m, n, 16).blocks;
+    const int G = dir == 0 ? x_lanes(b16, wave_grid(0, m, n, 8).blocks, wave_grid(0, m, n, 4).blocks) : 16;
+    if (G < 16) return G == 8 ? 2 : 4;
+    return b16 > FEW_BLOCKS ? 0 : dir == 0 ? 3 : 4;
 }
 
 // Wave-parallel sweep along DIR: a wave holds 64/G grid lines of G lanes each;

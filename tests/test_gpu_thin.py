@@ -36,10 +36,11 @@ def test_layout_edges(hg, oracle, m, n):
     assert parity(first, fo[:, npo - 1]).max() <= 1e-10      # glibc's pow against the device's
 
 
-# 769 blocks of 16 lanes and more: the lanes that give the fewest blocks
-@pytest.mark.parametrize("m,n,lanes", [(1, 12305, 4), (3, 12305, 4), (4, 12305, 8), (7, 12305, 8), (9, 12305, 4),
-                                       (15, 12305, 16), (16, 8192, 8), (22, 8192, 16)])
-def test_size_rule(hg, m, n, lanes):
+# 769 blocks of 16 lanes and more: the lanes that give the fewest blocks; below, 4 lanes on up to 3 cells
+@pytest.mark.parametrize("m,n,w,lanes", [(1, 12305, 4, 4), (3, 12305, 4, 4), (4, 12305, 4, 8), (7, 12305, 4, 8),
+                                         (9, 12305, 4, 4), (15, 12305, 4, 16), (16, 8192, 4, 8), (22, 8192, 4, 16),
+                                         (1, 49, 4, 4), (3, 64, 4, 4), (3, 32, 3, 16), (3, 304, 4, 4), (4, 304, 3, 16)])
+def test_size_rule(hg, m, n, w, lanes):
     s0 = cases.smooth_random(m, n, m)
     cfg = _config(m, n, t_all=1.0)
     out = []
@@ -47,7 +48,7 @@ def test_size_rule(hg, m, n, lanes):
         c = hg.Solver2D(m, n, cfg)
         try:
             if xv is None and not two:
-                assert c.sweep_kernel(0) == f"sweep_x_kernel<4, 0, {lanes}>"
+                assert c.sweep_kernel(0) == f"sweep_x_kernel<{w}, 0, {lanes}>"
             if xv is not None:
                 c.set_sweeps(xv, 0)
             c.upload(s0["rho"], s0["u"], s0["v"], s0["p"])
