@@ -224,23 +224,33 @@ __device__ __forceinline__ double unsplit_guess(const UnsplitArgs &a, bool activ
 // at the barriers.  A step with it and with this: 300^2 .062 and .054 ms, 512^2
 // .108 and .092, 1024^2 .281 and .283, 4096^2 3.84 and 3.22; G2D 257 x 190 .089
 // and .049, 1024^2 .337 and .347.)
-constexpr int TILE_R = 7, TILE_C = 8, SIDE_C = TILE_C + 2, SIDES = (TILE_R + 2) * SIDE_C - 1;   // not the last corner
+// Of 8 or 9 cells in x the second row of such tiles holds one or two; a tile of 9
+// x 6 (10 x 6 and 9 x 7 interfaces) takes them all (tile_shape).
+template <int SHAPE>
+struct Tile {
+    static constexpr int R = SHAPE == 1 ? 7 : 9, C = SHAPE == 1 ? 8 : 6;
+    static constexpr int SIDE_C = C + 2, SIDES = (R + 2) * SIDE_C - 1;   // not the last corner
+    static constexpr int XF = (R + 1) * C, YF = R * (C + 1);             // interfaces, a lane each
+    static_assert(XF <= 64 && YF <= 64, "a lane to an interface");
+};
 
-template <int NM, bool G2>
+template <int SHAPE, int NM, bool G2>
 __device__ __forceinline__ void unsplit_step_body(const UnsplitArgs &a, int per_row)
 {
     constexpr bool LEARNED = NM == NM_LEARNED;
+    constexpr int R = Tile<SHAPE>::R, C = Tile<SHAPE>::C, SIDE_C = Tile<SHAPE>::SIDE_C, SIDES = Tile<SHAPE>::SIDES;
+    constexpr int XF = Tile<SHAPE>::XF, YF = Tile<SHAPE>::YF;
     __shared__ double sides_lds[4][12][SIDES];   // value, x-slope, y-slope of the tile's cells and the ones around
     __shared__ double tab[POW_TAB];
     __shared__ uint32_t mlp_lds[LEARNED ? 4 : 1][LEARNED ? 64 * 8 : 1];
     const int lane = threadIdx.x & 63, wv = (threadIdx.x >> 6) & 3;
     const long wave = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int j0 = (int)(wave / per_row) * TILE_R, i0 = (int)(wave % per_row) * TILE_C;
+    const int j0 = (int)(wave / per_row) * R, i0 = (int)(wave % per_row) * C;
     double(*sd)[SIDES] = sides_lds[wv];
     // the lane's cell (row r, column k of the tile with its halo; updated for r >= 1) and x-interface,
     // between rows r and r + 1
-    const int r = lane >> 3, k = (lane & 7) + 1, c = j0 - 1 + r, ci = i0 - 1 + k;
-    const bool own = r >= 1 && c < a.m && ci < a.n;
+    const int r = lane / C, k = lane % C + 1, c = j0 - 1 + r, ci = i0 - 1 + k;
+    const bool own = r >= 1 && lane < XF && c < a.m && ci < a.n;
     {
         const Grid G(a);
         TabLoad<256> tl;
@@ -273,11 +283,11 @@ __device__ __forceinline__ void unsplit_step_body(const UnsplitArgs &a, int per_
     //        y-slope, transversal = -(x-slope);
     // dir 0: x-interface f = c + 1 between rows c and c + 1 (flux_generator_x.c:42-121).
     // One solve site for both, so the GRP code and its registers are laid out once.
-    const int yr = lane / (TILE_C + 1) + 1, yk = lane % (TILE_C + 1), yc = j0 - 1 + yr, ycell = i0 - 1 + yk;
+    const int yr = lane / (C + 1) + 1, yk = lane % (C + 1), yc = j0 - 1 + yr, ycell = i0 - 1 + yk;
     double dG[4];
 #pragma unroll 1
     for (int dir = 1; dir >= 0; --dir) {
-        const bool active = dir ? lane < TILE_R * (TILE_C + 1) && yc < a.m && ycell < a.n : c < a.m && ci < a.n;
+        const bool active = dir ? lane < YF && yc < a.m && ycell < a.n : lane < XF && c < a.m && ci < a.n;
         const int id0 = dir ? yr * SIDE_C + yk : r * SIDE_C + k, id1 = dir ? id0 + 1 : id0 + SIDE_C;
         Side SL, SR;
         double TL[4], TR[4];
@@ -310,7 +320,7 @@ __device__ __forceinline__ void unsplit_step_body(const UnsplitArgs &a, int per_
         const UnsplitArgs a = reload_args<UnsplitArgs>();
         const size_t o = (size_t)c * (size_t)a.ld + (size_t)ci, P = a.plane;
         if (dir) {   // the y-faces on both sides of the lane's cell
-            const int hi = r >= 1 ? (r - 1) * (TILE_C + 1) + k : 1;
+            const int hi = r >= 1 && lane < XF ? (r - 1) * (C + 1) + k : 1;
             double dI[4], tn[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
@@ -328,8 +338,8 @@ __device__ __forceinline__ void unsplit_step_body(const UnsplitArgs &a, int per_
         double dF[4], dI[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            dF[q] = F[q] - __shfl_up(F[q], 8);
-            dI[q] = I[q] - __shfl_up(I[q], 8);
+            dF[q] = F[q] - __shfl_up(F[q], C);
+            dI[q] = I[q] - __shfl_up(I[q], C);
         }
         if (own) {
             const double e_c = a.st[o + 4 * P];
@@ -354,21 +364,19 @@ __device__ __forceinline__ void unsplit_step_body(const UnsplitArgs &a, int per_
     }
 }
 
-// CU_WAVES: the waves that the register budget lets a CU hold; TILE_WAVES: the
-// waves that share a tile.
-template <int CU_WAVES, int TILE_WAVES, int NM>
+// CU_WAVES: the waves that the register budget lets a CU hold; SHAPE: the tile's
+// (1: 7 x 8, 2: 9 x 6).
+template <int CU_WAVES, int SHAPE, int NM>
 __global__ void __launch_bounds__(256, CU_WAVES / 4) unsplit_step_kernel(UnsplitArgs a, int per_row)
 {
-    static_assert(TILE_WAVES == 1, "a tile belongs to one wave");
-    unsplit_step_body<NM, false>(a, per_row);
+    unsplit_step_body<SHAPE, NM, false>(a, per_row);
 }
 
 // the same step with GRP_2D_flux's alternative interface solver, G2D
-template <int CU_WAVES, int TILE_WAVES, int NM>
+template <int CU_WAVES, int SHAPE, int NM>
 __global__ void __launch_bounds__(256, CU_WAVES / 4) unsplit_step_g2d_kernel(UnsplitArgs a, int per_row)
 {
-    static_assert(TILE_WAVES == 1, "a tile belongs to one wave");
-    unsplit_step_body<NM, true>(a, per_row);
+    unsplit_step_body<SHAPE, NM, true>(a, per_row);
 }
 
 // Strip form: one wave per block walks down R cell rows of a 62-cell strip
@@ -513,8 +521,8 @@ __global__ void __launch_bounds__(64, 2) unsplit_strip_g2d_kernel(UnsplitArgs a,
 }
 
 // ---- launchers -----------------------------------------------------------------
-// Two forms: the tile (TILE_R x TILE_C cells to a wave) and the
-// strip (one wave per block walking down its rows).  The context picks one
+// Two forms: the tile (a wave to a tile of cells) and the strip (one wave per
+// block walking down its rows).  The context picks one
 // (hgrp2d_set_unsplit_form, hgrp2d_tune) or takes the default (form 0: the tile).
 // The tile's register budget is three waves per SIMD (168 VGPRs, 4-83 spilled;
 // 38 KiB of LDS for the 4 waves of a block): with two waves and no spills a step
@@ -530,24 +538,47 @@ static int strip_rows(int m, int n)
 }
 
 // Form 0 and 1: the tile, which is the faster at every size measured; 2: the strip.
-static bool use_strip(int, int, int form) { return form == 2; }
+static bool use_strip(int form) { return form == 2; }
 
 int unsplit_max_rows() { return 65535 * 4; }   // grid.y of the strip form at R = 4
+
+template <int SHAPE>
+static long tiles_of(int m, int n)
+{
+    return (long)((m + Tile<SHAPE>::R - 1) / Tile<SHAPE>::R) * ((n + Tile<SHAPE>::C - 1) / Tile<SHAPE>::C);
+}
+
+// The tile's shape: 9 x 6 where the grid has more tiles of 7 x 8 than the chip
+// holds waves at once (12 to a CU) and a quarter fewer of 9 x 6, which is so on 8
+// and 9 cells in x.  A step of 8 x 31000 with 7 x 8 and with 9 x 6: .144 and .123
+// ms, 9 x 16384 .084 and .070; G2D 8 x 31000 .183 and .156.
+static int tile_shape(int m, int n)
+{
+    const long t = tiles_of<1>(m, n);
+    return t > 12 * 256 && 4 * tiles_of<2>(m, n) <= 3 * t ? 2 : 1;
+}
+
+template <int SHAPE, int NM, bool G2>
+static void launch_tile(const UnsplitArgs &a, hipStream_t st)
+{
+    const int per_row = (a.n + Tile<SHAPE>::C - 1) / Tile<SHAPE>::C;
+    const dim3 grid((unsigned)((tiles_of<SHAPE>(a.m, a.n) + 3) / 4));
+    if (G2) hipLaunchKernelGGL((unsplit_step_g2d_kernel<12, SHAPE, NM>), grid, dim3(256), 0, st, a, per_row);
+    else hipLaunchKernelGGL((unsplit_step_kernel<12, SHAPE, NM>), grid, dim3(256), 0, st, a, per_row);
+}
 
 template <int NM, bool G2>
 static hipError_t launch_unsplit(const UnsplitArgs &a, hipStream_t st)
 {
-    if (use_strip(a.m, a.n, a.form)) {
+    if (use_strip(a.form)) {
         const int R = strip_rows(a.m, a.n);
         const dim3 grid((unsigned)((a.n + 61) / 62), (unsigned)((a.m + R - 1) / R));
         if (G2) hipLaunchKernelGGL(unsplit_strip_g2d_kernel<NM>, grid, dim3(64), 0, st, a, R);
         else hipLaunchKernelGGL(unsplit_strip_kernel<NM>, grid, dim3(64), 0, st, a, R);
+    } else if (tile_shape(a.m, a.n) == 2) {
+        launch_tile<2, NM, G2>(a, st);
     } else {
-        const int per_row = (a.n + TILE_C - 1) / TILE_C;
-        const long tiles = (long)((a.m + TILE_R - 1) / TILE_R) * per_row;
-        const dim3 grid((unsigned)((tiles + 3) / 4));
-        if (G2) hipLaunchKernelGGL((unsplit_step_g2d_kernel<12, 1, NM>), grid, dim3(256), 0, st, a, per_row);
-        else hipLaunchKernelGGL((unsplit_step_kernel<12, 1, NM>), grid, dim3(256), 0, st, a, per_row);
+        launch_tile<1, NM, G2>(a, st);
     }
     return hipGetLastError();
 }
@@ -566,15 +597,15 @@ hipError_t launch_unsplit_step(const UnsplitArgs &a, hipStream_t st)
 
 const char *unsplit_kernel_name(int m, int n, int nm, int g2d, int form)
 {
-    static const char *names[2][3][2] = {
-        {{"unsplit_step_kernel<12, 1, 0>", "unsplit_strip_kernel<0>"},
-         {"unsplit_step_kernel<12, 1, 1>", "unsplit_strip_kernel<1>"},
-         {"unsplit_step_kernel<12, 1, 2>", "unsplit_strip_kernel<2>"}},
-        {{"unsplit_step_g2d_kernel<12, 1, 0>", "unsplit_strip_g2d_kernel<0>"},
-         {"unsplit_step_g2d_kernel<12, 1, 1>", "unsplit_strip_g2d_kernel<1>"},
-         {"unsplit_step_g2d_kernel<12, 1, 2>", "unsplit_strip_g2d_kernel<2>"}}};
+    static const char *names[2][3][3] = {
+        {{"unsplit_step_kernel<12, 1, 0>", "unsplit_step_kernel<12, 2, 0>", "unsplit_strip_kernel<0>"},
+         {"unsplit_step_kernel<12, 1, 1>", "unsplit_step_kernel<12, 2, 1>", "unsplit_strip_kernel<1>"},
+         {"unsplit_step_kernel<12, 1, 2>", "unsplit_step_kernel<12, 2, 2>", "unsplit_strip_kernel<2>"}},
+        {{"unsplit_step_g2d_kernel<12, 1, 0>", "unsplit_step_g2d_kernel<12, 2, 0>", "unsplit_strip_g2d_kernel<0>"},
+         {"unsplit_step_g2d_kernel<12, 1, 1>", "unsplit_step_g2d_kernel<12, 2, 1>", "unsplit_strip_g2d_kernel<1>"},
+         {"unsplit_step_g2d_kernel<12, 1, 2>", "unsplit_step_g2d_kernel<12, 2, 2>", "unsplit_strip_g2d_kernel<2>"}}};
     if (nm < 0 || nm > 2) return "";
-    return names[g2d ? 1 : 0][nm][use_strip(m, n, form) ? 1 : 0];
+    return names[g2d ? 1 : 0][nm][use_strip(form) ? 2 : tile_shape(m, n) - 1];
 }
 
 }  // namespace hgrp

@@ -1,6 +1,7 @@
 """Grids of few cells in x: the X sweep's lines of 4 and 8 lanes
 (csrc/sweep2d.hpp x_lanes) at the edges of their layout, and the size rule that
-takes them, for one grid, a batch and two fluids."""
+takes them, for one grid, a batch and two fluids; the unsplit step's tile of 9 x 6
+cells (csrc/unsplit2d.hip tile_shape)."""
 import numpy as np
 import pytest
 
@@ -79,3 +80,27 @@ def test_batch_of_thin_grids(hg):
             b.close()
     for got in out[1:]:
         assert all(np.array_equal(a, g) for a, g in zip(out[0], got))
+
+
+# 3073 tiles of 7 x 8 and more, and a quarter fewer of 9 x 6: the unsplit step's second tile shape
+@pytest.mark.parametrize("g2d", [False, True], ids=["Q1D", "G2D"])
+@pytest.mark.parametrize("m,n,shape", [(8, 12289, 2), (9, 12293, 2), (8, 12288, 1), (10, 12289, 1), (7, 24577, 1)])
+def test_unsplit_tile_shape(hg, m, n, shape, g2d):
+    s0 = cases.smooth_random(m, n, m)
+    for bx, by in ((-2, -7), (-24, -1)):
+        cfg = make_config(t_all=1.0, h_x=1 / m, h_y=1 / n, bc_x=bx, bc_y=by, split=0)
+        out = []
+        for form in (hg.UNSPLIT_TILE, hg.UNSPLIT_STRIP):
+            c = hg.Solver2D(m, n, cfg)
+            try:
+                if g2d:
+                    c.set_interface_solver(True)
+                c.set_unsplit_form(form)
+                if form == hg.UNSPLIT_TILE:
+                    assert c.sweep_kernel(2) == f"unsplit_step_{'g2d_' if g2d else ''}kernel<12, {shape}, 0>"
+                c.upload(s0["rho"], s0["u"], s0["v"], s0["p"])
+                c.bench_unsplit(3)
+                out.append(np.asarray(c.download()))
+            finally:
+                c.close()
+        assert np.array_equal(out[0], out[1]), (bx, by)
