@@ -104,3 +104,23 @@ def test_unsplit_tile_shape(hg, m, n, shape, g2d):
             finally:
                 c.close()
         assert np.array_equal(out[0], out[1]), (bx, by)
+
+
+@pytest.mark.parametrize("m,n", [(1, 33), (1, 64), (2, 33), (2, 64), (3, 33)])
+def test_round_trip_of_few_rows(hg, m, n):
+    """Grids of one or two rows come down row by row (csrc/layout2d.hip): any of the fields alone, too."""
+    s = cases.smooth_random(m, n, m + n)
+    c = hg.Solver2D(m, n, _config(m, n, t_all=0.1))
+    try:
+        c.upload(s["rho"], s["u"], s["v"], s["p"])
+        got = np.asarray(c.download()).reshape(5, m, n)
+        for f, k in enumerate(("rho", "u", "v", "p")):
+            assert np.array_equal(got[f], s[k].reshape(m, n)), k
+        a = np.random.default_rng(n).random((m, n))
+        c.set_fluids(1.67, a)
+        assert np.array_equal(np.asarray(c.download_fraction()).reshape(m, n), a)
+        p = np.empty((m, n))
+        assert hg.lib().hgrp2d_download(c._h, None, None, None, hg._p(p), None) == 0
+        assert np.array_equal(p, s["p"].reshape(m, n))
+    finally:
+        c.close()
