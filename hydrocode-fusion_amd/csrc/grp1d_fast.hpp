@@ -1,6 +1,7 @@
 // grp1d_fast.hpp -- the 1D ensemble's interface solver in the arithmetic of
 // fast_arith.hpp: grp_edir (grp1d_device.hpp) at atc = eps, bit for bit (a
-// zero's sign aside), for sides far from the ends of the exponent range.  The
+// zero's sign aside), for sides far from the ends of the exponent range (slopes
+// of density and pressure zero or differences of such values over h).  The
 // star state, the reciprocals and the treatment of tiny velocities are those of
 // grp_fast.hpp; a shock's speed is formed once.
 #pragma once
@@ -13,7 +14,7 @@ HGRP_HD bool sides1_in_range(const Side1 &L, const Side1 &R)
 {
     const double m = ((fabs(L.u) + fabs(R.u)) + (fabs(L.s_rho) + fabs(R.s_rho))) +
                      ((fabs(L.s_u) + fabs(R.s_u)) + (fabs(L.s_p) + fabs(R.s_p)));      // NaN for a NaN
-    return L.rho >= 0x1p-100 && L.p >= 0x1p-100 && R.rho >= 0x1p-100 && R.p >= 0x1p-100 &&
+    return L.rho >= LEAST && L.p >= LEAST && R.rho >= LEAST && R.p >= LEAST &&
            fmax(fmax(L.rho, L.p), fmax(R.rho, R.p)) <= 0x1p100 && m <= 0x1p100;
 }
 

@@ -26,8 +26,13 @@ namespace hgrp {
 // ---- which interfaces -------------------------------------------------------------
 HGRP_HD bool tiny(double x) { return fabs(x) < 0x1p-300 && x != 0.0; }
 
-// Densities and pressures in [2^-100, 2^100], velocities and derivatives below
-// 2^100.  Ahead of a front velocities decay cell by cell through every
+// Densities and pressures in [LEAST, 2^100], velocities and derivatives below
+// 2^100; derivatives of density and pressure zero or differences of such values
+// over h.  LEAST is 7e-40, thinner than gas in the usual units: an interface that
+// is left to the IEEE solver costs more than it did before there were two (512^2
+// with the learned guess at densities of 2^-120: .397 ms a step, .156 taken here,
+// .260 by the IEEE solver alone).
+// Ahead of a front velocities decay cell by cell through every
 // magnitude down to the denormals, over regions tens of cells wide, while
 // differences of pressure and density stop at their rounding: so what may be a
 // velocity (or a fraction) by itself is divided by IEEE division in the
@@ -37,9 +42,10 @@ HGRP_HD double magnitude(const Side &S)           // of the velocities and deriv
 {
     return ((fabs(S.u) + fabs(S.v)) + (fabs(S.d_rho) + fabs(S.d_u))) + (fabs(S.d_v) + fabs(S.d_p));
 }
+static constexpr double LEAST = 0x1p-130;
 HGRP_HD bool sides_in_range(const Side &L, const Side &R)
 {
-    return L.rho >= 0x1p-100 && L.p >= 0x1p-100 && R.rho >= 0x1p-100 && R.p >= 0x1p-100 &&
+    return L.rho >= LEAST && L.p >= LEAST && R.rho >= LEAST && R.p >= LEAST &&
            fmax(fmax(L.rho, L.p), fmax(R.rho, R.p)) <= 0x1p100 && magnitude(L) + magnitude(R) <= 0x1p100;
 }
 // a / rho, b / rho, c / rho of a cell's update
@@ -49,7 +55,7 @@ __device__ __forceinline__ void quot3(double a, double b, double c, double rho, 
     qa = div_q(a, r);
     qb = div_q(b, r);
     qc = div_q(c, r);
-    const bool in = rho >= 0x1p-100 && rho <= 0x1p100 && fmax(fmax(fabs(a), fabs(b)), fabs(c)) <= 0x1p300 &&
+    const bool in = rho >= LEAST && rho <= 0x1p100 && fmax(fmax(fabs(a), fabs(b)), fabs(c)) <= 0x1p300 &&
                     !tiny(c);
     if (tiny(a) || tiny(b)) {                    // a momentum ahead of a front
         qa = a / rho;
