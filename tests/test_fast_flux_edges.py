@@ -1,7 +1,8 @@
 """The steps' interface solver (csrc/grp_fast.hpp) against the IEEE solver, both
 built for the host, bit for bit (a zero's sign aside), where random interfaces
 do not lead: wave curves whose root lies just below a power of two, Newton
-iterations that end on a tiny gap."""
+iterations that end on a tiny gap, gas of another unit; and in the forms that
+the unsplit step and the two-fluid sweeps run."""
 import ctypes as C
 import os
 import subprocess
@@ -87,3 +88,61 @@ def test_thin_and_dense_gas(fast, direction, scale):
     inside = np.all((values >= 2.0 ** -130) & (values <= 2.0 ** 100), axis=1)
     assert took == on.sum() and inside.mean() > 0.5 and np.mean(on | vacuum | ~inside) > 0.99
     assert np.array_equal(f[on], i[on])
+
+
+@pytest.fixture(scope="module")
+def forms(tmp_path_factory):
+    return _build(tmp_path_factory, "fast_forms_host")
+
+
+def _pairs(n, seed, unit=1.0):
+    """Interfaces, a third of them of gas out of the solver's range, and starting pressures for two of three."""
+    L, R = cases.interface_pairs(n, seed)
+    out = np.arange(n) % 3 == 0
+    for A in (L, R):
+        A[out, 3] *= unit
+        A[out, 6] *= unit
+    guess = np.sqrt(L[:, 6]) * np.sqrt(R[:, 6]) * np.random.default_rng(seed).uniform(0.5, 2.0, n)
+    return L, R, np.where(np.arange(n) % 3 == 1, -1.0, guess)
+
+
+@pytest.mark.parametrize("conv", [0, 1])
+@pytest.mark.parametrize("guessed", [False, True])
+@pytest.mark.parametrize("direction", [0, 1])
+def test_stopping_rules_and_starting_pressures(forms, direction, guessed, conv):
+    """The unsplit step's flux and the two-fluid one as the steps call them."""
+    n, tol, tau, eps = 8000, 1e-12 if conv else 1e-9, 1e-3, 1e-9
+    L, R, guess = _pairs(n, 61 + conv)
+    guess = guess if guessed else np.full(n, -1.0)
+    f, i = np.full((n, 9), np.nan), np.zeros((n, 9))
+    took = forms.ff_transversal(_dp(L), _dp(R), n, C.c_double(tau), C.c_double(eps), C.c_double(tol), direction, conv,
+                                _dp(guess), _dp(f), _dp(i))
+    on = ~np.isnan(f[:, 0])
+    assert took == on.sum() > 0.95 * n and np.array_equal(f[on], i[on])
+    rng = np.random.default_rng(conv)
+    FA = np.zeros((n, 4))
+    for q in (0, 2):
+        FA[:, q] = np.choose(rng.integers(0, 4, n), [np.zeros(n), np.ones(n), rng.random(n), 10.0 ** rng.uniform(-320, 0, n)])
+        FA[:, q + 1] = rng.choice([0.0, 1.0, 1e-200], n) * rng.uniform(-1, 1, n)
+    f, i = np.full((n, 12), np.nan), np.zeros((n, 12))
+    took = forms.ff_two_fluid(_dp(L), _dp(R), _dp(FA), n, C.c_double(tau), C.c_double(eps), C.c_double(tol), direction, conv,
+                              C.c_double(1.4), C.c_double(1.67), _dp(guess), _dp(f), _dp(i))
+    on = ~np.isnan(f[:, 0])
+    # (the pairs are drawn for one gas: with two, a few more open a vacuum)
+    assert took == on.sum() > 0.9 * n and np.array_equal(f[on], i[on])
+
+
+@pytest.mark.parametrize("conv", [0, 1])
+@pytest.mark.parametrize("guessed", [False, True])
+@pytest.mark.parametrize("gamma", [1.4, 3.0])
+def test_g2d_star_state(forms, gamma, guessed, conv):
+    """G2D with its star state from the steps' Riemann solve, and from the IEEE one where that is out of range."""
+    n, tol = 8000, 1e-12 if conv else 1e-9
+    L, R, guess = _pairs(n, 71 + conv, 2.0 ** -140)
+    guess = guess if guessed else np.full(n, -1.0)
+    rng = np.random.default_rng(conv)
+    L, R = (np.ascontiguousarray(np.hstack([A, rng.uniform(0, 1, (n, 6))])) for A in (L, R))
+    L[:, 0] = R[:, 0] = gamma
+    f, i = np.zeros((n, 20)), np.zeros((n, 20))
+    took = forms.ff_g2d(_dp(L), _dp(R), n, C.c_double(1e-9), C.c_double(tol), conv, _dp(guess), _dp(f), _dp(i))
+    assert 0.6 * n < took < 0.7 * n and np.array_equal(f, i, equal_nan=True)
