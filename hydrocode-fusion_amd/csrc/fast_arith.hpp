@@ -102,8 +102,9 @@ HGRP_HD DD fast_sum(double a, double b)      // |a| >= |b| or a == 0
 // The pow functions below take the tables (powtab::TAB or a copy of it) as P.
 // A power looks up two entries, each in the middle of its dependent chain and
 // each lane its own: LDS answers in half the time of the vector cache.  The
-// steps' kernels therefore copy the tables to LDS (5 KiB a block) while their
-// first global loads are in flight.  A step before and after: split 64^2 .0751
+// steps' kernels therefore copy the tables to LDS (5 KiB a block), the sweeps and
+// the unsplit tile while their first global loads are in flight, the 1D ensemble
+// and the unsplit strip before them.  A step before and after: split 64^2 .0751
 // -> .0724 ms, 1024^2 .391 -> .377, 4096^2 learned 4.86 -> 4.55; unsplit 1024^2
 // .337 -> .327, learned .412 -> .381; two fluids 2048 x 512 .539 -> .512.
 static constexpr int POW_TAB = powtab::EXP_BASE + 128 * powtab::EXP_ROW;

@@ -85,7 +85,7 @@ struct hgrp2d {
     int newton_rule;            // HGRP_NEWTON_REFERENCE or HGRP_NEWTON_CONVERGE
     int xv, yv;                 // launch variants of the X and Y sweeps (hgrp2d_tune)
     int g2d;                    // the unsplit step's interface solver: 0 Q1D, 1 G2D
-    int uform;                  // the unsplit step's launch form: 0 by grid size, 1 tile, 2 strip
+    int uform;                  // the unsplit step's launch form: 0 the default (tile), 1 tile, 2 strip
     MlpPacked *mlp;             // device copy of the learned-guess weights
     bool use_mlp;
     bool two_fluid;             // volume fraction of fluid a carried (hgrp2d_set_fluids)

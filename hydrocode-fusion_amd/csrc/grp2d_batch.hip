@@ -35,7 +35,6 @@
 
 namespace hgrp {
 
-int sweep_variants(int dir);
 hipError_t launch_cfl(const double *rho, const double *u, const double *v, const double *p, int m, int n,
                       int ld, double gamma, double hmin, unsigned long long *out, hipStream_t st);
 

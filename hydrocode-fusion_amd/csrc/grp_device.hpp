@@ -93,8 +93,8 @@ __host__ __device__ inline RecipDiv recip_div(double b)
     d.ok = ab >= 0x1p-100 && ab <= 0x1p100;
     return d;
 }
-// the division itself, out of line: div_by is inlined at dozens of sites and
-// this path (zeros, infinities, NaN, extreme quotients) is rarely taken
+// One quotient; the kernels' come in fours (quot4).  The division itself, for
+// zeros, infinities, NaN and extreme quotients, is out of line.
 __device__ __attribute__((noinline)) static double div_slow(double a, double b) { return a / b; }
 
 __device__ __forceinline__ double div_by(double a, const RecipDiv &d)
@@ -108,9 +108,9 @@ __device__ __forceinline__ double div_by(double a, const RecipDiv &d)
     return div_slow(a, d.b);
 }
 
-// Four quotients by one divisor with a single check for the whole wave: div_by
-// for each where every lane's quotients are in range, else all of them by IEEE
-// division, out of line.  One branch instead of eight keeps the limiter short.
+// N quotients by one divisor with a single check for all of a lane's: as div_by
+// where all are in range, else all by IEEE division, out of line.  One branch
+// instead of N keeps the limiter short.
 struct Quot4 {
     double q[4];
 };

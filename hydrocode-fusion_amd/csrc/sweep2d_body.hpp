@@ -144,15 +144,9 @@ struct Line {
 #pragma unroll
         for (int q = 0; q < 4; ++q) s[q] = keep && q == NV ? near[q] : 0.0;
     }
-    // conservative update of cell k and slope refresh (grp_solver_2D_split_EUL_source.c:236-254)
-    __device__ void update(int k, const double w[4], const double Fl[4], const double Fr[4],
+    // conservative update of cell k (e: its E) and slope refresh (grp_solver_2D_split_EUL_source.c:236-254)
+    __device__ void update(int k, const double w[4], const double e, const double Fl[4], const double Fr[4],
                            const double Il[4], const double Ir[4]) const
-    {
-        update_e(k, w, a.st[at(k) + 4 * a.plane], Fl, Fr, Il, Ir);
-    }
-    // the same with E of the cell already loaded
-    __device__ void update_e(int k, const double w[4], const double e, const double Fl[4], const double Fr[4],
-                             const double Il[4], const double Ir[4]) const
     {
         const size_t o = at(k);
         const double nu = a.nu;
@@ -239,14 +233,18 @@ __device__ __forceinline__ double interface_guess(const SweepArgs &a, bool activ
 }
 
 // Launch variants: lanes along a line and the register budget (waves per SIMD).
-// Four waves cost some 30 spilled registers and are 5-8 % faster than three (none
-// spilled) once a grid gives every SIMD more than three waves (a step of 512^2
-// .143 against .150 ms, 1024^2 .313 against .338); below that the budget of three
-// is 2-4 % faster (384^2 .1056 against .1073, 127 x 329 .072 against .075), so that
-// is a smaller grid's default.
-// G = 16: the repeated face is 1 in 16 and a front along the lines still meets
-// few waves; G = 32 reads X lines in 16-byte pieces (4096^2 learned: X 1.64 ms
-// against 1.36).
+// Four waves are faster than three once a grid gives every SIMD more than three
+// (an X sweep of 1024^2 .123 ms against .131, of 4096^2 with the learned guess 1.29
+// against 1.42); below that the budget of three is (a step of 127 x 329 .073 ms
+// with both sweeps' against .075), so that is a smaller grid's default.
+// G = 16: the repeated face is 1 in 16 and a front along the lines still meets few
+// waves.  An X sweep with 32, 16 and 8 lanes to a line: 1024^2 .122, .123 and .135
+// ms, 4096^2 learned 1.53 (it reads the lines in 16-byte pieces), 1.29 and 1.30; a
+// Y sweep with 64, 32, 16 and 8: 1024^2 .129, .122, .120 and .122 ms, 4096^2 1.26,
+// 1.24, 1.21 and 1.30.  The others are the tuner's: which is fastest depends on how
+// a state's fronts lie (Y of 384^2, the same kind of state: .035 with 32, .039 with
+// 16).  Lines of 4 and 8 are also the default where they leave fewer lanes idle
+// (x_lanes).
 struct SweepShape {
     int G, minw;
 };
@@ -269,8 +267,8 @@ inline int default_variant(int dir, int m, int n)
 // updates cell c0-1+k for k >= 1 (G-1 cells per line).  Neighbours are lanes of
 // the same wave, so no wave waits for another once the pow tables are there: a
 // row of waves that hands its faces on through LDS waits 40 % of the time at
-// its three barriers (X of 4096^2: 1.56 ms against 1.36 with the learned guess,
-// 1.83 against 1.50 without; 1024^2 .123 against .109).
+// its three barriers (X of 4096^2, both built before the solver's last steps: 1.56
+// ms against 1.36 with the learned guess, 1.83 against 1.50 without).
 // DIR 1: the lanes of a line are consecutive (and so are its cells in memory);
 // DIR 0: the lines are (lane k 64/G + l: line l, so 64/G consecutive i), and a
 // block's waves take neighbouring lines, so that together they read whole cache
@@ -382,7 +380,7 @@ __device__ __forceinline__ void wave_sweep(const SweepArgs &a, const Src &src, l
         double wc[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) wc[q] = st[q][lane];
-        Lr.update_e(c, wc, st[4][lane], Fl, F, Il, I);
+        Lr.update(c, wc, st[4][lane], Fl, F, Il, I);
     }
 }
 

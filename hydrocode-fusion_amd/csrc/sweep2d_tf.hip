@@ -246,11 +246,10 @@ __device__ __forceinline__ bool tf_halted(const SweepArgs &a)
     return false;
 }
 
-// Both sweeps in the wave form of the single-fluid ones (wave_sweep): G = 16
-// cells of 4 lines per wave, a register budget for three waves per SIMD (some
-// 50 registers spilled; a step of 2048 x 512 .414 ms, at two waves .467, at four
-// .541).  The X sweep as rows of waves that hand faces on through LDS took .170
-// ms, this form .137.
+// Both sweeps in the wave form of the single-fluid ones (wave_sweep), lines of 16
+// cells (X of few cells: x_lanes), a register budget for three waves per SIMD (33-36
+// registers spilled; a step of 2048 x 512 with the learned guess .403 ms, at two
+// waves .473, at four .614; converge rule .434, .502 and .528).
 template <int DIR, int NM, int G>
 __device__ __forceinline__ void wave_sweep_tf(const SweepArgs &a, int per_row, double (*st)[64], uint32_t *mlp, double *tab)
 {

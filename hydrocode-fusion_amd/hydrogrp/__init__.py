@@ -190,7 +190,7 @@ class Solver2D:
         _check(lib().hgrp2d_set_interface_solver(self._h, 1 if g2d else 0), "hgrp2d_set_interface_solver")
 
     def set_unsplit_form(self, form):
-        """Launch form of the unsplit step: UNSPLIT_AUTO (by grid size), UNSPLIT_TILE
+        """Launch form of the unsplit step: UNSPLIT_AUTO (the tile), UNSPLIT_TILE
         or UNSPLIT_STRIP; tune() on an unsplit context picks the faster."""
         _check(lib().hgrp2d_set_unsplit_form(self._h, form), "hgrp2d_set_unsplit_form")
 

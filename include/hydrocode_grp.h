@@ -148,8 +148,8 @@ int hgrp2d_set_newton(hgrp2d *ctx, double tol, int rule, const float *params);
  * hgrp_g2d_batch).  A split context (config[33] != 0) takes Q1D only: -1002
  * and a message for G2D.  Works with every Newton setting of hgrp2d_set_newton. */
 /* Launch form of the unsplit step (no counterpart in the reference): TILE
- * one wave per 7 x 8 updated cells, STRIP one wave per 62-cell
- * strip walking down its rows; AUTO takes the tile, the faster at every size
+ * one wave per 7 x 8 updated cells (9 x 6 on long grids of 8 or 9 cells in x),
+ * STRIP one wave per 62-cell strip walking down its rows; AUTO takes the tile, the faster at every size
  * measured on MI355X.  hgrp2d_tune on an unsplit context times both and keeps
  * the faster.  Results do not depend on the form. */
 #define HGRP_UNSPLIT_AUTO 0
@@ -164,9 +164,11 @@ int hgrp2d_set_interface_solver(hgrp2d *ctx, int solver);
 /* Launch variants of the X sweep (0..5) and the Y sweep (0..4) (no counterpart
  * in the reference): a wave holds 64/G grid lines of G lanes along the sweep, at
  * a register budget for w waves per SIMD.  X: 0 = G 16, w 4; 1 = 32, 4; 2 = 8, 4;
- * 3 = 16, 3; 4 = 8, 3; 5 = 32, 3.  Y: 0 = 16, 4; 1 = 32, 4; 2 = 64, 4; 3 = 8, 4;
+ * 3 = 16, 3; 4 = 4, 4; 5 = 32, 3.  Y: 0 = 16, 4; 1 = 32, 4; 2 = 64, 4; 3 = 8, 4;
  * 4 = 16, 3.  The defaults are G 16 with w 4, on grids too small to give every
- * SIMD more than three waves with w 3.  Results do not depend on them. */
+ * SIMD more than three waves with w 3; X takes 8 or 4 lanes (2, 4) on grids of few
+ * cells in x, where 16 would leave more lanes idle.  Results do not depend on
+ * them. */
 int hgrp2d_set_sweeps(hgrp2d *ctx, int x_variant, int y_variant);
 
 /* Sweep autotuner: times every X variant, then every Y variant, over `steps`
