@@ -221,8 +221,8 @@ __device__ __forceinline__ void grp_g2d(double D[6], double U[6], double ws[2], 
     } else {
         StarQ st;
         if constexpr (FAST) {
-            bool in = gas_in_range(L.G) && gas_in_range(R.G) && fmin(L.p, R.p) >= LEAST && L.p + R.p <= 0x1p100 &&
-                      fmin(L.c, R.c) >= LEAST && fabs(L.u) + fabs(R.u) + L.c + R.c <= 0x1p100;
+            bool in = gas_in_range(L.G) && gas_in_range(R.G) && fmin(L.p, R.p) >= LEAST && L.p + R.p <= MOST &&
+                      fmin(L.c, R.c) >= LEAST && fabs(L.u) + fabs(R.u) + L.c + R.c <= MOST;
             Keep kL, kR;
             if (in)
                 in = riemann_q<CONV>(L.G, R.G, L.u, R.u, rcp_of(L.p), rcp_of(R.p), L.c, R.c, eps, tol, p_guess, st, kL,

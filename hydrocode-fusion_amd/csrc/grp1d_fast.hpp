@@ -15,7 +15,7 @@ HGRP_HD bool sides1_in_range(const Side1 &L, const Side1 &R)
     const double m = ((fabs(L.u) + fabs(R.u)) + (fabs(L.s_rho) + fabs(R.s_rho))) +
                      ((fabs(L.s_u) + fabs(R.s_u)) + (fabs(L.s_p) + fabs(R.s_p)));      // NaN for a NaN
     return L.rho >= LEAST && L.p >= LEAST && R.rho >= LEAST && R.p >= LEAST &&
-           fmax(fmax(L.rho, L.p), fmax(R.rho, R.p)) <= 0x1p100 && m <= 0x1p100;
+           fmax(fmax(L.rho, L.p), fmax(R.rho, R.p)) <= MOST && m <= MOST;
 }
 
 // the axis inside the rarefaction next to side S (grp_edir's sonic branches)

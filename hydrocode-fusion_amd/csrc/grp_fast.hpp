@@ -26,27 +26,27 @@ namespace hgrp {
 // ---- which interfaces -------------------------------------------------------------
 HGRP_HD bool tiny(double x) { return fabs(x) < 0x1p-300 && x != 0.0; }
 
-// Densities and pressures in [LEAST, 2^100], velocities and derivatives below
-// 2^100; derivatives of density and pressure zero or differences of such values
-// over h.  LEAST is 7e-40, thinner than gas in the usual units: an interface that
-// is left to the IEEE solver costs more than it did before there were two (512^2
-// with the learned guess at densities of 2^-120: .397 ms a step, .156 taken here,
-// .260 by the IEEE solver alone).
-// Ahead of a front velocities decay cell by cell through every
-// magnitude down to the denormals, over regions tens of cells wide, while
-// differences of pressure and density stop at their rounding: so what may be a
-// velocity (or a fraction) by itself is divided by IEEE division in the
-// acoustic case and in the passive members, and after the Riemann solve where
-// a wave holds such an interface (div_r).
+// Densities and pressures in [LEAST, MOST], velocities and derivatives below
+// MOST; derivatives of density and pressure zero or differences of such values
+// over h.  7e-40 to 1e39 holds gas in the usual units: an interface that is left
+// to the IEEE solver costs more than it did before there were two (512^2 with the
+// learned guess, left there .397 ms a step, taken here .156, .260 by the IEEE
+// solver alone).
+// Ahead of a front velocities decay cell by cell through every magnitude down to
+// the denormals, over regions tens of cells wide, while differences of pressure
+// and density stop at their rounding: so what may be a velocity (or a fraction)
+// by itself is divided by IEEE division in the acoustic case and in the passive
+// members, and after the Riemann solve where a wave holds such an interface
+// (div_r).
 HGRP_HD double magnitude(const Side &S)           // of the velocities and derivatives; NaN for a NaN
 {
     return ((fabs(S.u) + fabs(S.v)) + (fabs(S.d_rho) + fabs(S.d_u))) + (fabs(S.d_v) + fabs(S.d_p));
 }
-static constexpr double LEAST = 0x1p-130;
+static constexpr double LEAST = 0x1p-130, MOST = 0x1p130;
 HGRP_HD bool sides_in_range(const Side &L, const Side &R)
 {
     return L.rho >= LEAST && L.p >= LEAST && R.rho >= LEAST && R.p >= LEAST &&
-           fmax(fmax(L.rho, L.p), fmax(R.rho, R.p)) <= 0x1p100 && magnitude(L) + magnitude(R) <= 0x1p100;
+           fmax(fmax(L.rho, L.p), fmax(R.rho, R.p)) <= MOST && magnitude(L) + magnitude(R) <= MOST;
 }
 // a / rho, b / rho, c / rho of a cell's update
 __device__ __forceinline__ void quot3(double a, double b, double c, double rho, double &qa, double &qb, double &qc)
@@ -55,7 +55,7 @@ __device__ __forceinline__ void quot3(double a, double b, double c, double rho, 
     qa = div_q(a, r);
     qb = div_q(b, r);
     qc = div_q(c, r);
-    const bool in = rho >= LEAST && rho <= 0x1p100 && fmax(fmax(fabs(a), fabs(b)), fabs(c)) <= 0x1p300 &&
+    const bool in = rho >= LEAST && rho <= MOST && fmax(fmax(fabs(a), fabs(b)), fabs(c)) <= 0x1p300 &&
                     !tiny(c);
     if (tiny(a) || tiny(b)) {                    // a momentum ahead of a front
         qa = a / rho;
@@ -556,7 +556,7 @@ __device__ __forceinline__ bool flux_transversal_q(const Side &L, const Side &R,
 {
     const double t = ((fabs(TL[0]) + fabs(TL[1])) + (fabs(TL[2]) + fabs(TL[3]))) +
                      ((fabs(TR[0]) + fabs(TR[1])) + (fabs(TR[2]) + fabs(TR[3])));
-    if (!(gas_in_range(G) && sides_in_range(L, R) && t <= 0x1p100)) return false;
+    if (!(gas_in_range(G) && sides_in_range(L, R) && t <= MOST)) return false;
     Side l = L, r = R;
     double tl[4] = {TL[0], TL[1], TL[2], TL[3]}, tr[4] = {TR[0], TR[1], TR[2], TR[3]};
     if (dir) {                                   // into the interface's frame

@@ -80,8 +80,8 @@ static int g2d(const double *L, const double *R, int n, double eps, double tol, 
     for (int k = 0; k < n; ++k) {
         const double *l = L + 21 * k, *r = R + 21 * k;
         const G2Side a = g2_side_of(l, -1.0), b = g2_side_of(r, 1.0);
-        in += fmin(a.p, b.p) >= LEAST && a.p + b.p <= 0x1p100 && fmin(a.c, b.c) >= LEAST &&
-              fabs(a.u) + fabs(b.u) + a.c + b.c <= 0x1p100 && gas_in_range(a.G) && gas_in_range(b.G);
+        in += fmin(a.p, b.p) >= LEAST && a.p + b.p <= MOST && fmin(a.c, b.c) >= LEAST &&
+              fabs(a.u) + fabs(b.u) + a.c + b.c <= MOST && gas_in_range(a.G) && gas_in_range(b.G);
         double *f = fast + 20 * k, *o = ieee + 20 * k;
         grp_g2d<CONV, true>(f + 2, f + 8, f, f + 14, a, b, l[1], r[2], eps, eps, tol, guess[k], powtab::TAB);
         grp_g2d<CONV, false>(o + 2, o + 8, o, o + 14, a, b, l[1], r[2], eps, eps, tol, guess[k]);

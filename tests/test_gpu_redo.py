@@ -4,7 +4,7 @@ Runs that continue past the steps' fallback (redo_face, redo_face_tf,
 redo_face_t, redo_iface: sides, ghosts and previous slopes built again from
 memory), over enough steps that the previous slopes count.  Densities and
 pressures in units of 2^-140 are out of the fast solver's range everywhere; so
-are slopes over cells of 2^-120, and there every operation scales by powers of
+are slopes over cells of 2^-150, and there every operation scales by powers of
 two exactly, so that the run has the bits of one over cells of 1.  eps lies
 below all that is compared with it (and the runs end by their number of steps).
 And interface batches through both solvers, values next to powers of two among
@@ -74,7 +74,7 @@ def test_two_fluids(hg, ends, converge):
     s, frac = cases.smooth_random(m, n, 8), np.random.default_rng(1).random((m, n))
     frac[:5], frac[12:] = 0.0, 1.0
     (one, fa), (small, fb) = (_run(hg, m, n, s, _config(m, n, ends, h, split=1), converge, frac)
-                              for h in (1.0, 2.0 ** -120))
+                              for h in (1.0, 2.0 ** -150))
     assert np.array_equal(one, small) and np.array_equal(fa, fb)
     # a second gas out of the fast solver's range, of which there is none: the single-fluid run
     lone, _ = _run(hg, m, n, s, _config(m, n, ends, split=1), converge)
@@ -99,7 +99,7 @@ def test_batch(hg):
     sizes = [(17, 22), (5, 9), (30, 3)]
     states = [cases.smooth_random(m, n, m) for m, n in sizes]
     out = []
-    for h in (1.0, 2.0 ** -120):
+    for h in (1.0, 2.0 ** -150):
         cfg = make_config(t_all=10.0, N=9, bc_x=-2, bc_y=-7, eps=EPS, split=1)
         b = hg.Batch2D([(m, n, h / m, h / n) for m, n in sizes], cfg)
         try:
@@ -120,7 +120,7 @@ def test_ensemble(hg, bc):
     x = np.concatenate([(np.arange(m) + 0.5) / m for m in cells])
     rho, u, p = (b + 0.2 * np.sin(2 * np.pi * (x + rng.random())) for b in (1.0, 0.05, 1.0))
     out = []
-    for h in (1.0, 2.0 ** -120):
+    for h in (1.0, 2.0 ** -150):
         e = hg.Ensemble1D(cells, h / cells, make_config(t_all=10.0, N=9, bc_x=bc, eps=EPS))
         try:
             e.upload(rho, u, p)
