@@ -267,7 +267,7 @@ inline int default_variant(int dir, int m, int n)
 // updates cell c0-1+k for k >= 1 (G-1 cells per line).  Neighbours are lanes of
 // the same wave, so no wave waits for another once the pow tables are there: a
 // row of waves that hands its faces on through LDS waits 40 % of the time at
-// its three barriers (X of 4096^2, both built before the solver's last steps: 1.56
+// its three barriers (X of 4096^2, an earlier interface solve in both: 1.56
 // ms against 1.36 with the learned guess, 1.83 against 1.50 without).
 // DIR 1: the lanes of a line are consecutive (and so are its cells in memory);
 // DIR 0: the lines are (lane k 64/G + l: line l, so 64/G consecutive i), and a
